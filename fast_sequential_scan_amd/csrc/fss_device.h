@@ -76,16 +76,25 @@ __device__ __forceinline__ Ptr uniform_ptr(Ptr ptr) {
 
 // Loads/stores of N dwords per lane.  NT marks the access non-temporal: the data
 // is touched once, so the caches should not keep it in preference to other lines.
+// The types promise no more than 2-byte alignment: gfx950 serves global accesses of 4 to 16 bytes
+// at any address (the compiler emits the same instructions for them), so rows whose length or
+// start is odd need no narrower kernels.  Three streams of 512 MiB, 16 bytes per lane: every
+// stream aligned 4.6 TB/s, every stream 2 bytes off 4.6, 4 or 8 bytes off 4.2, 2-byte accesses
+// instead 4.1-4.6; 4 bytes per lane: 5.4 aligned, 4.0-4.2 at 2 bytes off.
+typedef uint32_t io_u32x1 __attribute__((aligned(2)));
+typedef uint32_t io_u32x2 __attribute__((ext_vector_type(2), aligned(2)));
+typedef uint32_t io_u32x4 __attribute__((ext_vector_type(4), aligned(2)));
+
 template <int N, bool NT>
 struct DwordIO;
 template <bool NT>
 struct DwordIO<1, NT> {
   static __device__ __forceinline__ void load(uint32_t *dst, gcptr_t p) {
-    const FSS_GLOBAL uint32_t *q = reinterpret_cast<const FSS_GLOBAL uint32_t *>(p);
+    const FSS_GLOBAL io_u32x1 *q = reinterpret_cast<const FSS_GLOBAL io_u32x1 *>(p);
     dst[0] = NT ? __builtin_nontemporal_load(q) : *q;
   }
   static __device__ __forceinline__ void store(gptr_t p, const uint32_t *src) {
-    FSS_GLOBAL uint32_t *q = reinterpret_cast<FSS_GLOBAL uint32_t *>(p);
+    FSS_GLOBAL io_u32x1 *q = reinterpret_cast<FSS_GLOBAL io_u32x1 *>(p);
     if (NT)
       __builtin_nontemporal_store(src[0], q);
     else
@@ -95,14 +104,14 @@ struct DwordIO<1, NT> {
 template <bool NT>
 struct DwordIO<2, NT> {
   static __device__ __forceinline__ void load(uint32_t *dst, gcptr_t p) {
-    const FSS_GLOBAL u32x2 *q = reinterpret_cast<const FSS_GLOBAL u32x2 *>(p);
-    const u32x2 v = NT ? __builtin_nontemporal_load(q) : *q;
+    const FSS_GLOBAL io_u32x2 *q = reinterpret_cast<const FSS_GLOBAL io_u32x2 *>(p);
+    const io_u32x2 v = NT ? __builtin_nontemporal_load(q) : *q;
     dst[0] = v.x;
     dst[1] = v.y;
   }
   static __device__ __forceinline__ void store(gptr_t p, const uint32_t *src) {
-    const u32x2 v = {src[0], src[1]};
-    FSS_GLOBAL u32x2 *q = reinterpret_cast<FSS_GLOBAL u32x2 *>(p);
+    const io_u32x2 v = {src[0], src[1]};
+    FSS_GLOBAL io_u32x2 *q = reinterpret_cast<FSS_GLOBAL io_u32x2 *>(p);
     if (NT)
       __builtin_nontemporal_store(v, q);
     else
@@ -112,16 +121,16 @@ struct DwordIO<2, NT> {
 template <bool NT>
 struct DwordIO<4, NT> {
   static __device__ __forceinline__ void load(uint32_t *dst, gcptr_t p) {
-    const FSS_GLOBAL u32x4 *q = reinterpret_cast<const FSS_GLOBAL u32x4 *>(p);
-    const u32x4 v = NT ? __builtin_nontemporal_load(q) : *q;
+    const FSS_GLOBAL io_u32x4 *q = reinterpret_cast<const FSS_GLOBAL io_u32x4 *>(p);
+    const io_u32x4 v = NT ? __builtin_nontemporal_load(q) : *q;
     dst[0] = v.x;
     dst[1] = v.y;
     dst[2] = v.z;
     dst[3] = v.w;
   }
   static __device__ __forceinline__ void store(gptr_t p, const uint32_t *src) {
-    const u32x4 v = {src[0], src[1], src[2], src[3]};
-    FSS_GLOBAL u32x4 *q = reinterpret_cast<FSS_GLOBAL u32x4 *>(p);
+    const io_u32x4 v = {src[0], src[1], src[2], src[3]};
+    FSS_GLOBAL io_u32x4 *q = reinterpret_cast<FSS_GLOBAL io_u32x4 *>(p);
     if (NT)
       __builtin_nontemporal_store(v, q);
     else
@@ -157,6 +166,40 @@ struct Row<E, VEC, 2> {
 #pragma unroll
     for (int i = 0; i < kDwords; ++i) dw[i] = E::pack2(f[2 * i], f[2 * i + 1]);
   }
+  // Moves the elements k places down (element k becomes element 0) or up; zeros come in.
+  __device__ __forceinline__ void shift_down(int k) {
+#pragma unroll
+    for (int i = 0; i < kDwords; ++i) {
+      const uint32_t next = i + 1 < kDwords ? dw[i + 1 < kDwords ? i + 1 : i] : 0u;
+      dw[i] = (k & 1) ? (dw[i] >> 16) | (next << 16) : dw[i];
+    }
+#pragma unroll
+    for (int step = 1; step < kDwords; step <<= 1)
+#pragma unroll
+      for (int i = 0; i < kDwords; ++i)
+        dw[i] = ((k >> 1) & step) ? (i + step < kDwords ? dw[i + step < kDwords ? i + step : i] : 0u) : dw[i];
+  }
+  __device__ __forceinline__ void shift_up(int k) {
+#pragma unroll
+    for (int i = kDwords - 1; i >= 0; --i) dw[i] = (k & 1) ? (dw[i] << 16) | (i > 0 ? dw[i > 0 ? i - 1 : 0] >> 16 : 0u) : dw[i];
+#pragma unroll
+    for (int step = 1; step < kDwords; step <<= 1)
+#pragma unroll
+      for (int i = kDwords - 1; i >= 0; --i)
+        dw[i] = ((k >> 1) & step) ? (i >= step ? dw[i >= step ? i - step : 0] : 0u) : dw[i];
+  }
+  // Elements [first, end) of the segment: dwords, and a half where an end is odd.
+  __device__ __forceinline__ void store_some(gptr_t p, int first, int end) const {
+#pragma unroll
+    for (int i = 0; i < kDwords; ++i) {
+      if (2 * i >= first && 2 * i + 2 <= end) {
+        *reinterpret_cast<FSS_GLOBAL io_u32x1 *>(p + 4 * i) = dw[i];
+      } else {
+        if (2 * i >= first && 2 * i < end) *reinterpret_cast<FSS_GLOBAL uint16_t *>(p + 4 * i) = static_cast<uint16_t>(dw[i]);
+        if (2 * i + 1 >= first && 2 * i + 1 < end) *reinterpret_cast<FSS_GLOBAL uint16_t *>(p + 4 * i + 2) = static_cast<uint16_t>(dw[i] >> 16);
+      }
+    }
+  }
 };
 
 template <typename E>
@@ -180,6 +223,9 @@ struct Row<E, 1, 2> {
   __device__ __forceinline__ float get(int) const { return E::lo(dw[0]); }
   __device__ __forceinline__ void fill(float x) { dw[0] = E::bits(x); }
   __device__ __forceinline__ void pack(const float *f) { dw[0] = E::pack2(f[0], 0.0f) & 0xffffu; }
+  __device__ __forceinline__ void shift_down(int) {}
+  __device__ __forceinline__ void shift_up(int) {}
+  __device__ __forceinline__ void store_some(gptr_t p, int, int) const { store(p); }
 };
 
 template <typename E, int VEC>
@@ -204,6 +250,24 @@ struct Row<E, VEC, 4> {
   __device__ __forceinline__ void pack(const float *f) {
 #pragma unroll
     for (int i = 0; i < kDwords; ++i) dw[i] = as_u32(f[i]);
+  }
+  __device__ __forceinline__ void shift_down(int k) {
+#pragma unroll
+    for (int step = 1; step < kDwords; step <<= 1)
+#pragma unroll
+      for (int i = 0; i < kDwords; ++i)
+        dw[i] = (k & step) ? (i + step < kDwords ? dw[i + step < kDwords ? i + step : i] : 0u) : dw[i];
+  }
+  __device__ __forceinline__ void shift_up(int k) {
+#pragma unroll
+    for (int step = 1; step < kDwords; step <<= 1)
+#pragma unroll
+      for (int i = kDwords - 1; i >= 0; --i) dw[i] = (k & step) ? (i >= step ? dw[i >= step ? i - step : 0] : 0u) : dw[i];
+  }
+  __device__ __forceinline__ void store_some(gptr_t p, int first, int end) const {
+#pragma unroll
+    for (int i = 0; i < kDwords; ++i)
+      if (i >= first && i < end) *reinterpret_cast<FSS_GLOBAL uint32_t *>(p + 4 * i) = dw[i];
   }
 };
 

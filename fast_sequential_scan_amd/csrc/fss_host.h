@@ -432,20 +432,14 @@ inline int make_cm_plan(CmPlan &pl, int64_t rows, int64_t seq, int dtype, int di
   const int widest = 16 / esize;  // 16 bytes per lane and load
   int vec = user ? user->vec : 0, waves = user ? user->waves : 0;
   if (user && (user->max_groups < 0 || user->steps != 0)) return FSS_ERR_BAD_CONFIG;
-  if (vec == 0) {
-    vec = widest;
-    // rows start at multiples of seq elements: every row must keep the vectors aligned
-    while (vec > 2 || (vec == 2 && esize == 4)) {
-      if (ss % vec == 0 && align % (static_cast<size_t>(vec) * esize) == 0) break;
-      vec = 2;  // only 1, 2 and the widest are compiled (fp32: 1 and 4)
-      if (esize == 4) vec = 1;
-    }
-    if (vec == 2 && (ss % 2 != 0 || align % (2 * static_cast<size_t>(esize)) != 0)) vec = 1;
-  }
+  // 16 bytes per lane whatever the rows' length and alignment, from the length that fills one lane on
+  // (a configuration that names the vector width keeps to naturally aligned accesses)
+  const bool any_rows = vec == 0;
+  if (any_rows) vec = ss >= widest ? widest : 1;
   const bool vec_ok = vec == 1 || vec == widest || (vec == 2 && esize == 2);
   if (!vec_ok) return FSS_ERR_BAD_CONFIG;
-  if (ss % vec != 0) return FSS_ERR_BAD_CONFIG;
-  if (align % (static_cast<size_t>(vec) * esize) != 0) return FSS_ERR_MISALIGNED;
+  if (!any_rows && ss % vec != 0) return FSS_ERR_BAD_CONFIG;
+  if (!any_rows && align % (static_cast<size_t>(vec) * esize) != 0) return FSS_ERR_MISALIGNED;
   if (waves == 0) {
     const int64_t w = ceil_div(ss, static_cast<int64_t>(64) * vec);
     waves = static_cast<int>(w < 8 ? w : 8);

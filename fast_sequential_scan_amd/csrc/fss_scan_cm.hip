@@ -23,12 +23,28 @@ namespace fss {
 // holds scan positions (k*64 + l)*VEC .. +VEC-1, i.e. timesteps descending from
 // seq-1-(k*64+l)*VEC, and takes alpha[t+1] / h[t-1] of its first / last step from
 // the neighbouring lane (or, at a slice edge, from a one-element load).
+//
+// Rows need no alignment beyond an element's and no length that is a multiple of VEC: global
+// accesses work at any address (DwordIO), and the one lane per row whose vector would reach past
+// the end of the scan loads one that ends there and shifts it.  Kernels with one timestep per
+// lane for such rows (128 bytes per wave and load, chunks of 512 steps instead of 4096) took three
+// times as long: bf16 forward and backward of (8, 1024, 2047) 159 -> 55.5 us (2048: 52), of
+// (8, 1024, 4095) 323 -> 112 us (4096: 98), of (1, 256, 65521) 193 -> 65 us.  What is left between
+// odd and aligned rows is the price of 16-byte accesses at odd addresses; keeping the stores'
+// lines in L2 for the neighbouring wave (no streaming hint) costs another 3-5 %.
 
 __device__ __forceinline__ float lane_read(float v, int lane) {
   return as_f32(__builtin_amdgcn_readlane(as_u32(v), lane));
 }
 
-template <typename E, int VEC, int ROWS, bool BWD>
+template <bool B>
+struct Flag {
+  static constexpr bool value = B;
+};
+
+// RAGGED: seq is no multiple of VEC (a kernel of its own: the shifts cost the forward four spilled
+// registers, 2 % of the time of rows that need none).
+template <typename E, int VEC, int ROWS, bool BWD, bool RAGGED>
 __device__ __forceinline__ void cm_tile(const ScanArgs &p, const TileCtx &c, int64_t row0, int64_t n_rows) {
   using RowT = Row<E, VEC>;
   using OneT = Row<E, 1>;
@@ -36,7 +52,12 @@ __device__ __forceinline__ void cm_tile(const ScanArgs &p, const TileCtx &c, int
   const int lane = c.lane;
   const int64_t slice = static_cast<int64_t>(c.chunk) * c.n_waves + c.wave;
   const int64_t r_base = (slice * 64 + lane) * VEC;             // first scan position of this lane
-  const bool in_seq = r_base < seq;                             // seq % VEC == 0: all of the vector or none
+  const bool in_seq = r_base < seq;
+  // The last lane of the scan may hold fewer than VEC steps (backward: the missing ones are the low end
+  // of its vector, timesteps below 0).  It loads the VEC timesteps that end (backward: start) with the
+  // sequence and moves them to their places, so that no lane reads outside its row and no load waits.
+  const bool ragged = RAGGED && slice * 64 * VEC < seq && seq < (slice + 1) * 64 * VEC;  // in this slice
+  const int missing = ragged && in_seq && seq - r_base < VEC ? VEC - static_cast<int>(seq - r_base) : 0;
   const int64_t t_lo = BWD ? seq - r_base - VEC : r_base;       // lowest timestep of the vector
   const int64_t t_hi = t_lo + VEC - 1;
   // wave-uniform base (the lowest timestep any lane of the slice holds) + a 32-bit lane offset
@@ -46,6 +67,24 @@ __device__ __forceinline__ void cm_tile(const ScanArgs &p, const TileCtx &c, int
   RowT a[ROWS], b[ROWS], hp[BWD ? ROWS : 1];
   float edge_a[BWD ? ROWS : 1], edge_h[BWD ? ROWS : 1];
   bool ok[ROWS];
+  constexpr int kBack = BWD || !RAGGED ? 0 : VEC * E::kBytes;  // (lane offsets are unsigned: the base makes room)
+  const uint32_t load_off = lane_off + kBack + (BWD ? missing : -missing) * E::kBytes;
+  auto load_vector = [&](RowT &v, const char *tensor, int64_t off, auto nt) {
+    v.template load<decltype(nt)::value>(uniform_ptr((gcptr_t)tensor + off - kBack) + load_off);
+  };
+  auto place = [&](RowT &v) {
+    if (BWD)
+      v.shift_up(missing);
+    else
+      v.shift_down(missing);
+  };
+  auto store_vector = [&](const RowT &v, char *tensor, int64_t off, auto nt) {
+    const gptr_t base = uniform_ptr((gptr_t)tensor + off) + lane_off;
+    if (missing == 0)
+      v.template store<decltype(nt)::value>(base);
+    else
+      v.store_some(base, BWD ? missing : 0, BWD ? VEC : VEC - missing);
+  };
 
   // ---- phase 1a: loads ---------------------------------------------------------------
 #pragma unroll
@@ -56,8 +95,15 @@ __device__ __forceinline__ void cm_tile(const ScanArgs &p, const TileCtx &c, int
     b[r].fill(0.0f);
     if (ok[r]) {
       const int64_t off = (row * seq + t_base) * E::kBytes;
-      a[r].template load<(BWD ? kNtABwd : kNtAFwd)>(uniform_ptr((gcptr_t)p.in_a + off) + lane_off);
-      b[r].template load<(BWD ? kNtBBwd : kNtBFwd)>(uniform_ptr((gcptr_t)p.in_b + off) + lane_off);
+      load_vector(a[r], p.in_a, off, Flag<(BWD ? kNtABwd : kNtAFwd)>());
+      load_vector(b[r], p.in_b, off, Flag<(BWD ? kNtBBwd : kNtBFwd)>());
+    }
+  }
+  if (ragged) {
+#pragma unroll
+    for (int r = 0; r < ROWS; ++r) {
+      place(a[r]);
+      place(b[r]);
     }
   }
   if (BWD) {
@@ -83,7 +129,7 @@ __device__ __forceinline__ void cm_tile(const ScanArgs &p, const TileCtx &c, int
         hp[r].fill(0.0f);
         if (ok[r]) {
           const int64_t off = ((row0 + r) * seq + t_base) * E::kBytes;
-          hp[r].template load<kNtH>(uniform_ptr((gcptr_t)p.in_h + off) + lane_off);
+          load_vector(hp[r], p.in_h, off, Flag<kNtH>());
         }
         if (lane == 63 && ok[r] && t_lo >= 1) eh[r].load((gcptr_t)p.in_h + ((row0 + r) * seq + t_lo - 1) * E::kBytes);
       }
@@ -149,6 +195,10 @@ __device__ __forceinline__ void cm_tile(const ScanArgs &p, const TileCtx &c, int
     chain_chunks<1, BWD>(p, c, &mA, &mB, nullptr, &slice_in, load_h);
   else
     load_h();
+  if (BWD && ragged) {
+#pragma unroll
+    for (int r = 0; r < ROWS; ++r) place(hp[r]);
+  }
   if (BWD) {
     // h[t_lo-1] for the last step: from the neighbouring lane, except at the end of the slice
 #pragma unroll
@@ -180,11 +230,11 @@ __device__ __forceinline__ void cm_tile(const ScanArgs &p, const TileCtx &c, int
       const int64_t off = ((row0 + r) * seq + t_base) * E::kBytes;
       RowT o;
       o.pack(o0);
-      o.template store<(BWD ? kNtOutBwd : kNtOutFwd)>(uniform_ptr((gptr_t)p.out0 + off) + lane_off);
+      store_vector(o, p.out0, off, Flag<(BWD ? kNtOutBwd : kNtOutFwd)>());
       if (BWD) {
         RowT oa;
         oa.pack(o1);
-        oa.template store<kNtOutBwd>(uniform_ptr((gptr_t)p.out1 + off) + lane_off);
+        store_vector(oa, p.out1, off, Flag<kNtOutBwd>());
       }
     }
   }
@@ -192,7 +242,7 @@ __device__ __forceinline__ void cm_tile(const ScanArgs &p, const TileCtx &c, int
 
 // ScanArgs here: seq = the contiguous length, d = number of rows (bs * channels),
 // n_ctiles = ceil(rows / ROWS) row groups, n_chunks = ceil(seq / (waves*64*VEC)).
-template <typename E, int VEC, int ROWS, bool BWD>
+template <typename E, int VEC, int ROWS, bool BWD, bool RAGGED>
 __global__ __launch_bounds__(1024) void cm_scan_kernel(const ScanArgs p) {
   extern __shared__ float lds[];
   __shared__ uint32_t s_ready[16];  // per wave: see announce_map
@@ -231,24 +281,24 @@ __global__ __launch_bounds__(1024) void cm_scan_kernel(const ScanArgs p) {
     c.last = c.chunk == p.n_chunks - 1;
     c.anchor = __builtin_amdgcn_readfirstlane(chain_anchor(c.chunk, p.period, p.look_waves * kMaxSpan));
     c.span = __builtin_amdgcn_readfirstlane(chunk_span(c.chunk - c.anchor, p.look_waves));
-    cm_tile<E, VEC, ROWS, BWD>(p, c, static_cast<int64_t>(ctile) * ROWS, p.d);
+    cm_tile<E, VEC, ROWS, BWD, RAGGED>(p, c, static_cast<int64_t>(ctile) * ROWS, p.d);
   }
   count_out(p, c);
 }
 
 // ---- launching ---------------------------------------------------------------------
 
-template <typename E, int VEC, bool BWD>
+template <typename E, int VEC, bool BWD, bool RAGGED = false>
 int launch_cm_one(const ScanArgs &args, const CmPlan &pl, int max_groups, hipStream_t stream) {
   constexpr int kRows = BWD ? kCmRowsBwd : kCmRowsFwd;
   static int resident[17] = {0};
   const int waves = pl.waves;
   const size_t lds = lds_bytes(waves, 1);
-  const int fit = resident_workgroups(cm_scan_kernel<E, VEC, kRows, BWD>, waves, lds, resident);
+  const int fit = resident_workgroups(cm_scan_kernel<E, VEC, kRows, BWD, RAGGED>, waves, lds, resident);
   if (fit <= 0) return FSS_ERR_LAUNCH;
   int64_t n_groups = pl.n_tiles < fit ? pl.n_tiles : fit;
   if (max_groups > 0 && max_groups < n_groups) n_groups = max_groups;
-  hipLaunchKernelGGL((cm_scan_kernel<E, VEC, kRows, BWD>), dim3(static_cast<uint32_t>(n_groups)),
+  hipLaunchKernelGGL((cm_scan_kernel<E, VEC, kRows, BWD, RAGGED>), dim3(static_cast<uint32_t>(n_groups)),
                      dim3(static_cast<uint32_t>(waves) * 64), lds, stream, args);
   const hipError_t e = hipGetLastError();
   if (e != hipSuccess) {
@@ -261,7 +311,9 @@ int launch_cm_one(const ScanArgs &args, const CmPlan &pl, int max_groups, hipStr
 template <typename E, bool BWD>
 int launch_cm(const ScanArgs &args, const CmPlan &pl, int max_groups, hipStream_t stream) {
   constexpr int kWidest = 16 / E::kBytes;
-  if (pl.vec == kWidest) return launch_cm_one<E, kWidest, BWD>(args, pl, max_groups, stream);
+  if (pl.vec == kWidest)
+    return args.seq % kWidest == 0 ? launch_cm_one<E, kWidest, BWD>(args, pl, max_groups, stream)
+                                   : launch_cm_one<E, kWidest, BWD, true>(args, pl, max_groups, stream);
   if (pl.vec == 1) return launch_cm_one<E, 1, BWD>(args, pl, max_groups, stream);
   if constexpr (E::kBytes == 2) {
     if (pl.vec == 2) return launch_cm_one<E, 2, BWD>(args, pl, max_groups, stream);

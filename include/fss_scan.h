@@ -383,8 +383,9 @@ int fss_gated_scan_bwd_state(int dtype, const void *gate, const void *x, const v
  * (bs, seq, d) tensors (benchmark.py:67-72).  Same recurrences and gradients as
  * fss_scan_fwd_ex / fss_scan_bwd_ex, per run; the values in alpha[..., 0] are never used.  Note the
  * argument order bs, d, seq.  Of `cfg` only vec (timesteps per lane: 1, 2 or 8 for the
- * 16-bit types, 1 or 4 for fp32; seq % vec == 0 and tensors aligned to vec elements),
- * waves and max_groups are used; steps must be 0.  A workgroup of 8 waves covers
+ * 16-bit types, 1 or 4 for fp32; named, it asks for seq % vec == 0 and tensors aligned to vec
+ * elements; left 0, the library takes the widest for any seq and alignment), waves and
+ * max_groups are used; steps must be 0.  A workgroup of 8 waves covers
  * 4096 (16-bit) / 2048 (fp32) timesteps, and only longer sequences use the workspace:
  * size it with fss_cm_workspace_bytes (an upper bound over alignments).
  */

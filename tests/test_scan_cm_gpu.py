@@ -77,6 +77,29 @@ def test_cm_default_config(oracle, shape, dtype):
     _run(oracle, *shape, dtype, seed=sum(shape))
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32], ids=["bf16", "f32"])
+@pytest.mark.parametrize("seq", [3, 5, 8, 9, 15, 255, 511, 513, 2047, 4095, 4097, 8191])
+def test_cm_rows_of_any_length_and_start(oracle, seq, dtype):
+    """Rows whose length is no multiple of a lane's 16 bytes (one element short or long of a lane, a
+    wave, a workgroup), a row count that fills no tile, tensors that start one element into their
+    storage, and a NaN in alpha[..., 0], which nothing may read into a result."""
+    bs, d = 3, 5
+    alpha, beta, dout = _inputs(bs, d, seq, dtype, seed=seq)
+    h, ga, gb = _run(oracle, bs, d, seq, dtype, seed=seq)
+
+    def off_by_one(t):
+        flat = torch.full((t.numel() + 2,), float("nan"), dtype=dtype, device=DEV)
+        view = flat[1:-1].view(t.shape)
+        view.copy_(t)
+        return view
+
+    a, b, do = off_by_one(alpha), off_by_one(beta), off_by_one(dout)
+    a[..., 0] = float("nan")
+    assert torch.equal(ext.scan_forward_cm(a, b), h)
+    ga2, gb2 = ext.scan_backward_cm(a, off_by_one(h), do)
+    assert torch.equal(ga2, ga) and torch.equal(gb2, gb)
+
+
 @pytest.mark.parametrize("config", [(1, 0, 1), (1, 0, 3), (2, 0, 2), (2, 0, 16), (8, 0, 1), (8, 0, 2), (8, 0, 5),
                                     (8, 0, 16), (8, 0, 8, 3), (2, 0, 4, 1)], ids=str)
 def test_cm_result_does_not_depend_on_config_bf16(oracle, config):
