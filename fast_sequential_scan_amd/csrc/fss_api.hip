@@ -255,7 +255,9 @@ int run_scan(int dtype, int dir, const void *alpha, const void *in_b, const void
   // (variant 2 exists for the kernels large shapes run - the forward with 32 steps per lane, the
   // backward with 16 steps and 4 bytes per lane; elsewhere the forward runs as 0, the backward as 1)
   const bool large = streaming || tensor_bytes > kStreamDoutBytes;
-  if (gated)
+  if (shares_sectors(d * static_cast<int64_t>(esize)))
+    pl.alt_policy = 3;
+  else if (gated)
     pl.alt_policy = 0;
   else if (dir == FSS_FWD)
     pl.alt_policy = large ? 2 : (tensor_bytes <= kKeepOutBytes ? 1 : 0);

@@ -424,6 +424,20 @@ __host__ __device__ inline uint32_t tile_group(const TileOrder &o, uint32_t slot
   return (slot & 7u) * o.per + k;
 }
 
+// Which tile of a round of the grid (`count` tiles: the grid's size, fewer in the last round) workgroup
+// `block` takes.  Ordinarily its own index.  Where rows of several
+// tiles share cache lines (shares_lines) and the groups
+// could not be dealt out in eighths, the workgroups of one XCD take consecutive tiles instead, so that
+// both tiles that touch a line touch it in one L2.  (One to one over block < count, and every
+// workgroup still takes its tiles in ascending order, so a tile's wait for lower ones is as safe as
+// before.)  Not otherwise: it puts a column's consecutive chunks on different XCDs, and rows of whole
+// lines gain nothing for it (bf16 (1, 65521, 256) backward 36 -> 41 us).
+__host__ __device__ inline uint32_t tile_in_round(const TileOrder &o, uint32_t block, uint32_t count, bool lines_shared) {
+  if (o.per != 0 || !lines_shared) return block;
+  const uint32_t xcd = block & 7u, extra = count & 7u;
+  return xcd * (count >> 3) + (xcd < extra ? xcd : extra) + (block >> 3);
+}
+
 // Optional (bs, d) fp32 rows of the scans with a state entering/leaving the sequence.
 // The plain scan is compiled against the empty variant, whose members are constant
 // nulls: it carries no kernel arguments for them and every use folds away.
@@ -486,6 +500,19 @@ constexpr int64_t kKeepOutBytes = static_cast<int64_t>(48) << 20;
 // over one set of tensors it costs 2 % at 64 MiB per tensor, where part of beta is still
 // cached from the step before, and nothing measurable at 128 MiB.
 constexpr int64_t kStreamDoutBytes = static_cast<int64_t>(80) << 20;
+
+// Rows that are no whole number of 128-byte lines put two column tiles, worked on by different workgroups,
+// on the lines at their seam.  The L2 puts such a line together only if both tiles meet it there
+// (tile_in_round) and only if it is kept until both have: a line read or written with the hint is gone
+// before the neighbour comes and travels twice, the second time as a partial write.  Such rows
+// therefore run without any hint - unless they are whole 64-byte sectors, which the memory writes
+// without reading (bf16 (4, 17738, 1376): forward 126 us with the hints, 133 us without).  bf16, with the
+// tiles' order: (18, 4006, 1682) forward 238 -> 181 us, backward 442 -> 307 us; (17, 1516, 2249) 162 ->
+// 93 and 307 -> 161 us; fp32 (8, 2048, 1501) 80 -> 66 and 149 -> 115 us; gated fp16 (14, 6405, 856) 140 ->
+// 119 and 303 -> 219 us, where the order alone gives 219, 417; 134, 262; 79, 150; 130, 263 us.
+constexpr int kLineBytes = 128, kSectorBytes = 64;
+__host__ __device__ inline bool shares_lines(int64_t row_bytes) { return row_bytes % kLineBytes != 0; }
+__host__ __device__ inline bool shares_sectors(int64_t row_bytes) { return row_bytes % kSectorBytes != 0; }
 
 #ifdef FSS_TRACE
 #define FSS_STAMP(c, p, slot)                                                                   \

@@ -117,7 +117,7 @@ __device__ __forceinline__ void scan_tile(const ScanArgs &p, const StateArgs<STA
       // of the sequence, so it loads the row before instead.
       const int row = (BWD && s == 0 && at_start) ? 1 : s;
       a[s].template load<(BWD ? (kNtABwd || ALT == 2) : kNtAFwd)>(uniform_ptr(pa + row * step_bytes) + lane_off);
-      b[s].template load<(BWD ? (kNtBBwd || ALT != 0) : (kNtBFwd || ALT == 2))>(uniform_ptr(pb + s * step_bytes) + lane_off);
+      b[s].template load<(BWD ? (kNtBBwd || ALT == 1 || ALT == 2) : (kNtBFwd || ALT == 2))>(uniform_ptr(pb + s * step_bytes) + lane_off);
     } else {
       // Outside the sequence the step is the identity map (a=1, b=0).  The first step
       // of the plain scan has no predecessor (a=0), whatever alpha holds there; with a
@@ -127,7 +127,7 @@ __device__ __forceinline__ void scan_tile(const ScanArgs &p, const StateArgs<STA
       if (c.col_ok && s < valid) {
         if (s >= 1 || !at_start || (STATE && !BWD && st.state_in))
           a[s].template load<(BWD ? (kNtABwd || ALT == 2) : kNtAFwd)>(uniform_ptr(pa + s * step_bytes) + lane_off);
-        b[s].template load<(BWD ? (kNtBBwd || ALT != 0) : (kNtBFwd || ALT == 2))>(uniform_ptr(pb + s * step_bytes) + lane_off);
+        b[s].template load<(BWD ? (kNtBBwd || ALT == 1 || ALT == 2) : (kNtBFwd || ALT == 2))>(uniform_ptr(pb + s * step_bytes) + lane_off);
       }
     }
   }
@@ -149,11 +149,11 @@ __device__ __forceinline__ void scan_tile(const ScanArgs &p, const StateArgs<STA
   gcptr_t ph = BWD ? (gcptr_t)p.in_h + c.tile_base + (t_first - 1) * row_bytes : (gcptr_t) nullptr;
   auto load_h = [&](int s) {
     if (FULL) {
-      hp[s].template load<kNtH>(uniform_ptr(ph + s * step_bytes) + lane_off);
+      hp[s].template load<(kNtH && ALT != 3)>(uniform_ptr(ph + s * step_bytes) + lane_off);
     } else {
       hp[s].fill(0.0f);
       if (c.col_ok && s + 1 < valid)  // t - 1 >= 0
-        hp[s].template load<kNtH>(uniform_ptr(ph + s * step_bytes) + lane_off);
+        hp[s].template load<(kNtH && ALT != 3)>(uniform_ptr(ph + s * step_bytes) + lane_off);
     }
   };
   auto load_h_early = [&] {
@@ -219,7 +219,7 @@ __device__ __forceinline__ void scan_tile(const ScanArgs &p, const StateArgs<STA
     if (FULL || (c.col_ok && s < valid)) {
       RowT o;
       o.pack(state);
-      o.template store<(BWD ? kNtOutBwd : (kNtOutFwd && ALT != 1))>(uniform_ptr(po0 + s * step_bytes) + lane_off);
+      o.template store<(BWD ? (kNtOutBwd && ALT != 3) : (kNtOutFwd && ALT != 1))>(uniform_ptr(po0 + s * step_bytes) + lane_off);
       if (BWD) {
         if (!FULL && s + 1 == valid) {  // t = 0: grad_alpha[0] = g[0] * h[-1], 0 in the plain scan
 #pragma unroll
@@ -228,7 +228,7 @@ __device__ __forceinline__ void scan_tile(const ScanArgs &p, const StateArgs<STA
         }
         RowT oa;
         oa.pack(ga);
-        oa.template store<kNtOutBwd>(uniform_ptr(po1 + s * step_bytes) + lane_off);
+        oa.template store<(kNtOutBwd && ALT != 3)>(uniform_ptr(po1 + s * step_bytes) + lane_off);
       }
     }
     if (BWD && s + kHEarly < STEPS) load_h(s + kHEarly);
@@ -275,7 +275,7 @@ __device__ __forceinline__ float sigmoid_f32(float z) {
 // gradient with respect to h[-1] go out, exactly as in the plain scan (scan_tile).
 // The backward needs alpha[t+1] as the coefficient of step t and alpha[t] for its
 // elementwise part: a slice of STEPS steps loads STEPS+1 rows of the gate.
-template <typename E, int VEC, int STEPS, bool BWD, bool STATE, bool FULL>
+template <typename E, int VEC, int STEPS, bool BWD, bool STATE, bool FULL, int ALT>
 __device__ __forceinline__ void gated_tile(const ScanArgs &p, const StateArgs<STATE> &st, const TileCtx &c) {
   using RowT = Row<E, VEC>;
   const int64_t seq = c.seq, row_bytes = c.row_bytes, r0 = c.r0;
@@ -313,14 +313,14 @@ __device__ __forceinline__ void gated_tile(const ScanArgs &p, const StateArgs<ST
   gcptr_t px = BWD ? (gcptr_t)p.in_x + c.tile_base + t_first * row_bytes : (gcptr_t) nullptr;
   auto load_hx = [&](int s) {
     if (FULL) {
-      hp[s].template load<kNtH>(uniform_ptr(ph + s * step_bytes) + lane_off);
-      xs[s].template load<kNtH>(uniform_ptr(px + s * step_bytes) + lane_off);
+      hp[s].template load<(kNtH && ALT != 3)>(uniform_ptr(ph + s * step_bytes) + lane_off);
+      xs[s].template load<(kNtH && ALT != 3)>(uniform_ptr(px + s * step_bytes) + lane_off);
     } else {
       hp[s].fill(0.0f);
       xs[s].fill(0.0f);
       if (c.col_ok && s + 1 < valid)  // t - 1 >= 0
-        hp[s].template load<kNtH>(uniform_ptr(ph + s * step_bytes) + lane_off);
-      if (c.col_ok && s < valid) xs[s].template load<kNtH>(uniform_ptr(px + s * step_bytes) + lane_off);
+        hp[s].template load<(kNtH && ALT != 3)>(uniform_ptr(ph + s * step_bytes) + lane_off);
+      if (c.col_ok && s < valid) xs[s].template load<(kNtH && ALT != 3)>(uniform_ptr(px + s * step_bytes) + lane_off);
     }
   };
   if (BWD) {
@@ -433,11 +433,11 @@ __device__ __forceinline__ void gated_tile(const ScanArgs &p, const StateArgs<ST
     if (FULL || (c.col_ok && s < valid)) {
       RowT o;
       o.pack(o0);
-      o.template store<(BWD ? kNtOutBwd : kNtOutFwd)>(uniform_ptr(po0 + s * step_bytes) + lane_off);
+      o.template store<((BWD ? kNtOutBwd : kNtOutFwd) && ALT != 3)>(uniform_ptr(po0 + s * step_bytes) + lane_off);
       if (BWD) {
         RowT oz;
         oz.pack(o1);
-        oz.template store<kNtOutBwd>(uniform_ptr(po1 + s * step_bytes) + lane_off);
+        oz.template store<(kNtOutBwd && ALT != 3)>(uniform_ptr(po1 + s * step_bytes) + lane_off);
       }
     }
     if (BWD && s + kEarly < STEPS) load_hx(s + kEarly);
@@ -452,12 +452,13 @@ __device__ __forceinline__ void gated_tile(const ScanArgs &p, const StateArgs<ST
 
 // STATE: the variant that honours the optional incoming/outgoing state rows of ScanArgs;
 // the plain and the gated scan are compiled without them.  GATED: the gated scan.
-// ALT: the cache policy of the plain scan (hints only, never the arithmetic).  Forward: 0 stores
+// ALT: the cache policy (hints only, never the arithmetic).  Forward: 0 stores
 // h with the non-temporal hint, 1 without it (small outputs, left in the cache for their reader),
 // 2 = 0 and reads beta, which nothing reads again, with the hint (large tensors).  Backward:
 // 1 reads dout with the hint (large tensors), 2 = 1 and reads alpha with it as well (its last
 // use in a step; only when the caller says that nothing is found in the cache again, because
-// the forward of a loop over one set of tensors does find it there).
+// the forward of a loop over one set of tensors does find it there), 3 no hint anywhere (rows that share
+// sectors; that is 1 in the plain forward).  The gated scan has 0 and 3.
 // COLS: column tiles a workgroup covers side by side (compile-time, so that the common
 // one-column kernels keep their compile-time LDS addresses and scalar register count).
 // MAXW: the most waves a workgroup may have (max_waves of the planner): what the registers are allotted for.
@@ -505,8 +506,8 @@ __global__ __launch_bounds__(MAXW * 64) void scan_kernel(const ScanArgs p, const
   // every workgroup of a launch reads the same value: it only changes when all are done
   c.tag = c.chained ? __builtin_amdgcn_readfirstlane(ld_u32(p.hdr + HDR_EPOCH)) + 1u : 0u;
 
-  // The grid is sized to be resident all at once; each workgroup walks tiles
-  // blockIdx, blockIdx + gridDim, ...  Tiles are numbered chunk-major, so a tile
+  // The grid is sized to be resident all at once; each workgroup takes one tile of every
+  // gridDim of them (the blockIdx-th, or see tile_in_round).  Tiles are numbered chunk-major, so a tile
   // only ever waits for tiles with smaller numbers: those belong to a resident
   // workgroup that reaches them no later than this one reaches its own.
   // (which column group a slot of a chunk stands for: tile_order; bs 8 seq 4096 d 1024 bf16, forward +
@@ -516,7 +517,10 @@ __global__ __launch_bounds__(MAXW * 64) void scan_kernel(const ScanArgs p, const
   const uint32_t n_groups = order.n_groups;
   uint32_t parity = 0;
   uint32_t tile_no = 0;
-  for (uint32_t tile = blockIdx.x; tile < static_cast<uint32_t>(p.n_tiles); tile += gridDim.x, parity ^= 1u) {
+  const bool lines_shared = p.tiles_per_row > 1 && shares_lines(c.row_bytes);
+  for (uint32_t done = 0; done + blockIdx.x < static_cast<uint32_t>(p.n_tiles); done += gridDim.x, parity ^= 1u) {
+    const uint32_t left = static_cast<uint32_t>(p.n_tiles) - done;
+    const uint32_t tile = done + tile_in_round(order, blockIdx.x, left < gridDim.x ? left : gridDim.x, lines_shared);
     c.tile_no = ++tile_no;
     c.lds_map = lds_maps + (parity * waves_total + c.wcol * c.n_waves) * kLaneSlots;
     // unsigned, wave-uniform arithmetic: stays on the scalar unit
@@ -547,9 +551,9 @@ __global__ __launch_bounds__(MAXW * 64) void scan_kernel(const ScanArgs p, const
     // same barriers, so they meet
     if constexpr (GATED) {
       if (full)
-        gated_tile<E, VEC, STEPS, BWD, STATE, true>(p, st, c);
+        gated_tile<E, VEC, STEPS, BWD, STATE, true, ALT>(p, st, c);
       else
-        gated_tile<E, VEC, STEPS, BWD, STATE, false>(p, st, c);
+        gated_tile<E, VEC, STEPS, BWD, STATE, false, ALT>(p, st, c);
     } else {
       if (full)
         scan_tile<E, VEC, STEPS, BWD, STATE, true, ALT>(p, st, c);
@@ -604,7 +608,8 @@ int launch_two_columns(const ScanArgs &args, const StateArgs<true> &state, const
     if constexpr (!BWD) {
       if (pl.cfg.steps == 32) {
         if (pl.alt_policy == 2) return launch_one<E, V, 32, BWD, true, false, 2, 2>(args, state, pl, stream);
-        if (pl.alt_policy == 1) return launch_one<E, V, 32, BWD, true, false, 1, 2>(args, state, pl, stream);
+        if (pl.alt_policy == 1 || pl.alt_policy == 3)
+          return launch_one<E, V, 32, BWD, true, false, 1, 2>(args, state, pl, stream);
         return launch_one<E, V, 32, BWD, true, false, 0, 2>(args, state, pl, stream);
       }
     }
@@ -613,6 +618,7 @@ int launch_two_columns(const ScanArgs &args, const StateArgs<true> &state, const
   switch (pl.cfg.steps) {
 #define FSS_CASE2(S)                                                                                   \
   case S:                                                                                              \
+    if (pl.alt_policy == 3) return launch_one<E, V, S, BWD, false, false, BWD ? 3 : 1, 2>(args, state, pl, stream); \
     if constexpr (!BWD && S == 32) {                                                                   \
       if (pl.alt_policy == 2) return launch_one<E, V, S, BWD, false, false, 2, 2>(args, state, pl, stream); \
     }                                                                                                  \
@@ -643,6 +649,9 @@ int launch_typed(const ScanArgs &args, const StateArgs<true> &state, const Plan 
   switch (key) {
 #define FSS_CASE(V, S)                                                                            \
   case V * 100 + S:                                                                               \
+    if constexpr (V <= 2) {                                                                       \
+      if (pl.alt_policy == 3) return launch_one<E, V, S, BWD, STATE, false, BWD ? 3 : 1>(args, state, pl, stream); \
+    }                                                                                             \
     /* the scans with states carry the policy in the kernels large shapes run, the plain scan in all */ \
     if constexpr ((!BWD && S == 32) || (BWD && S == 16 && V * E::kBytes == 4)) {                  \
       if (pl.alt_policy == 2) return launch_one<E, V, S, BWD, STATE, false, 2>(args, state, pl, stream); \
@@ -675,6 +684,12 @@ int launch_typed(const ScanArgs &args, const StateArgs<true> &state, const Plan 
 }
 
 // The gated kernels: 4 bytes (bf16 x2, fp32 x1) or one bf16 element per lane.
+template <typename E, int V, int S, bool BWD, bool STATE>
+int gated_one(const ScanArgs &args, const StateArgs<true> &state, const Plan &pl, hipStream_t stream) {
+  return pl.alt_policy == 3 ? launch_one<E, V, S, BWD, STATE, true, 3>(args, state, pl, stream)
+                            : launch_one<E, V, S, BWD, STATE, true>(args, state, pl, stream);
+}
+
 template <typename E, bool BWD, bool STATE>
 int launch_gated(const ScanArgs &args, const StateArgs<true> &none, const Plan &pl, hipStream_t stream) {
   constexpr bool is_16bit = E::kBytes == 2;
@@ -683,14 +698,14 @@ int launch_gated(const ScanArgs &args, const StateArgs<true> &none, const Plan &
   switch (key) {
 #define FSS_CASE(V, S) \
   case V * 100 + S:    \
-    return launch_one<E, V, S, BWD, STATE, true>(args, none, pl, stream);
+    return gated_one<E, V, S, BWD, STATE>(args, none, pl, stream);
     FSS_CASE(1, 8)
     FSS_CASE(1, 16)
     default:
       break;
   }
   if constexpr (!BWD) {
-    if (key == 132) return launch_one<E, 1, 32, BWD, STATE, true>(args, none, pl, stream);
+    if (key == 132) return gated_one<E, 1, 32, BWD, STATE>(args, none, pl, stream);
   }
   if constexpr (is_16bit) {
     switch (key) {
@@ -700,7 +715,7 @@ int launch_gated(const ScanArgs &args, const StateArgs<true> &none, const Plan &
         break;
     }
     if constexpr (!BWD) {
-      if (key == 232) return launch_one<E, 2, 32, BWD, STATE, true>(args, none, pl, stream);
+      if (key == 232) return gated_one<E, 2, 32, BWD, STATE>(args, none, pl, stream);
     }
   }
 #undef FSS_CASE

@@ -263,7 +263,8 @@ int fss_scan_bwd_f32(const void *alpha, const void *h, const void *dout,
  * with or without states (with states: in the kernels that large shapes run - 32 steps per lane
  * in the forward, 16 steps and 4 bytes per lane in the backward); the gated and the channel-major
  * scans carry the same hints under both (outputs and the backward's reads of h streamed,
- * everything else cached).  Returns the previous policy, or -1 for an unknown one.
+ * everything else cached).  Rows of (bs, seq, d) tensors that are no multiple of 64 bytes run
+ * without any hint under both.  Returns the previous policy, or -1 for an unknown one.
  */
 enum fss_cache_policy { FSS_CACHE_AUTO = 0, FSS_CACHE_STREAMING = 1 };
 int fss_set_cache_policy(int policy);
