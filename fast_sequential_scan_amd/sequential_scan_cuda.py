@@ -200,9 +200,15 @@ def _workspace(device: torch.device, stream: "_RawStream", need: int) -> "_Works
     return ws
 
 
-def _slow_backward(kind: int, code: int, saved: List[torch.Tensor], grad_out: torch.Tensor):
+def _slow_backward(kind: int, code: int, saved: List[torch.Tensor], grad_out: torch.Tensor,
+                   grad_last: Optional[torch.Tensor] = None):
     """What the C++ dispatch calls back for a backward it does not cover (kind 0: the plain scan,
-    saved (alpha, h); kind 1: the gated scan, saved (gate, x, h))."""
+    saved (alpha, h); kind 1: the gated scan, saved (gate, x, h); kinds 3 and 4: the same two with
+    states, saved the same and the incoming state if there was one)."""
+    if kind == 4:
+        return list(gated_scan_backward_state(saved[0], saved[1], saved[2], grad_out, saved[3] if len(saved) > 3 else None, grad_last))
+    if kind == 3:
+        return list(scan_backward_state(saved[0], saved[1], grad_out, saved[2] if len(saved) > 2 else None, grad_last))
     if kind == 1:
         return gated_scan_backward(saved[0], saved[1], saved[2], grad_out)
     if kind == 2:  # channel-major, saved (alpha, h)

@@ -247,3 +247,53 @@ def test_channel_major_scan_same_bits_as_the_python_function(dtype, shape):
     with pytest.raises(RuntimeError):
         scan_cm(alpha, beta[:, :, :10])
     ext.workspace_status()
+
+
+@pytest.mark.parametrize("gated", [False, True], ids=["plain", "gated"])
+@pytest.mark.parametrize("with_state", [True, False])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32, torch.float16], ids=["bf16", "f32", "f16"])
+@pytest.mark.parametrize("shape", [(2, 777, 328), (1, 1, 64), (3, 2050, 130)])
+def test_scans_with_states_same_bits_as_the_python_wrappers(shape, dtype, with_state, gated):
+    """Forward, and the backward through both outputs or one of them, with contiguous and transposed
+    gradients; what the dispatch refuses stays refused (double differentiation, forward mode)."""
+    api = scan_cuda.scan_gated_with_state if gated else scan_with_state
+    function = scan_cuda.SequentialScanGatedState if gated else scan_cuda.SequentialScanState
+    alpha, beta, dout = _tensors(shape, dtype, seed=sum(shape))
+    bs, seq, d = shape
+    states = torch.randn(2, bs, d, device=DEV, generator=torch.Generator(DEV).manual_seed(5))
+    turned = dout.transpose(1, 2).contiguous().transpose(1, 2)  # the same values, another order in memory
+    turned_last = states[1].t().contiguous().t()
+
+    def inputs():
+        before = states[0].clone().requires_grad_(True) if with_state else None
+        return alpha.clone().requires_grad_(True), beta.clone().requires_grad_(True), before
+
+    def check(got, want):
+        assert len(got) == len(want)
+        for g, w in zip(got, want):
+            assert (g is None) == (w is None) and (g is None or torch.equal(g, w))
+
+    with torch.no_grad():
+        want = function.apply(alpha, beta, states[0] if with_state else None)  # (also makes sure a workspace exists)
+        check(api(alpha, beta, states[0] if with_state else None), want)
+    for do, dl in ((dout, states[1]), (turned, turned_last), (dout, None), (None, states[1])):
+        a, b, before = inputs()
+        h, last = api(a, b, before)
+        assert "StateNode" in _node_name(h) and "StateNode" in _node_name(last)
+        check((h, last), want)
+        outs, grads = zip(*((o, g) for o, g in ((h, do), (last, dl)) if g is not None))
+        got = torch.autograd.grad(outs, [t for t in (a, b, before) if t is not None], grads)
+        # an output nobody used has the gradient zero (of the last state: none at all)
+        do = torch.zeros_like(alpha) if do is None else do
+        with torch.no_grad():
+            ref = (ext.gated_scan_backward_state(a, b, h, do, before, dl) if gated
+                   else ext.scan_backward_state(a, h, do, before, dl))
+        check(got, [t for t in ref if t is not None])
+    a, b, before = inputs()
+    h, last = api(a, b, before)
+    (once,) = torch.autograd.grad(h, a, dout.clone().requires_grad_(True), create_graph=True)
+    with pytest.raises(RuntimeError, match="once_differentiable"):
+        once.sum().backward()
+    with torch.autograd.forward_ad.dual_level(), pytest.raises((RuntimeError, NotImplementedError)):
+        api(torch.autograd.forward_ad.make_dual(alpha, dout), beta, states[0] if with_state else None)
+    ext.workspace_status()
