@@ -247,9 +247,9 @@ int run_scan(int dtype, int dir, const void *alpha, const void *in_b, const void
   args.n_chunks = static_cast<int32_t>(pl.n_chunks);
   args.n_tiles = static_cast<int32_t>(pl.n_tiles);
   args.n_groups = static_cast<int32_t>(pl.n_groups);
-  args.wg_cols = pl.cfg.cols;
   args.look_waves = look_waves(pl.cfg.waves, pl.cfg.vec, pl.cfg.cols);
   args.period = chain_period(pl.n_groups, pl.cfg.waves);
+  set_divisors(args);
   args.spin_limit = __atomic_load_n(&g_spin_limit, __ATOMIC_RELAXED);
   const int64_t tensor_bytes = bs * seq * d * static_cast<int64_t>(esize);
   // (variant 2 exists for the kernels large shapes run - the forward with 32 steps per lane, the
@@ -409,7 +409,8 @@ int fss_debug_chain_plan(int64_t bs, int64_t seq, int64_t d, int dtype, int dir,
 
 int32_t fss_debug_chain_anchor(int32_t chunk, int32_t period, int32_t stride) {
   if (chunk < 0 || period < 1 || stride < 1) return -1;
-  return fss::chain_anchor(chunk, period, stride);
+  return fss::chain_anchor(chunk, period, fss::fast_div(static_cast<uint32_t>(period)), stride,
+                           fss::fast_div(static_cast<uint32_t>(stride)));
 }
 
 uint32_t fss_debug_set_spin_limit(uint32_t polls) {

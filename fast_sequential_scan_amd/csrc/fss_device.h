@@ -361,6 +361,36 @@ __device__ __forceinline__ void report_timeout(uint32_t *hdr) {
     __hip_atomic_store(reinterpret_cast<uint32_t *>(addr), 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
 }
 
+// Division of 32-bit unsigned numbers by a divisor the host knows, as a multiplication and shifts
+// (Granlund and Montgomery, "Division by Invariant Integers using Multiplication", 1994, section 4): five
+// scalar instructions, where the hardware's way - a vector-unit reciprocal, corrected - is a chain
+// of about thirty that a tile waited for seven times before its first load.  With the launch tag no
+// longer waited for there either (launch_tag) and the arguments not held throughout (fresh_args): bf16
+// (2, 1024, 768) forward 9.1 -> 8.3 us, backward 11.4 -> 10.4; gated (3, 156, 3456) forward 10.5 -> 9.5;
+// (4, 2048, 2048) 22.6 -> 21.9; launches of several rounds gain up to 2 % or nothing.
+struct FastDiv {
+  uint32_t mul;
+  uint8_t first, second;  // shifts
+};
+inline FastDiv fast_div(uint32_t n) {
+  int bits = 0;  // of n - 1: the least l with n <= 2^l
+  while (bits < 32 && (uint64_t{1} << bits) < n) ++bits;
+  FastDiv f;
+  f.mul = static_cast<uint32_t>(((uint64_t{1} << 32) * ((uint64_t{1} << bits) - n)) / n + 1);
+  f.first = static_cast<uint8_t>(bits < 1 ? bits : 1);
+  f.second = static_cast<uint8_t>(bits > 1 ? bits - 1 : 0);
+  return f;
+}
+__host__ __device__ inline uint32_t divide(uint32_t x, const FastDiv &f) {
+  const uint32_t t = static_cast<uint32_t>((static_cast<uint64_t>(x) * f.mul) >> 32);
+  return (t + ((x - t) >> f.first)) >> f.second;
+}
+
+struct TileOrder {
+  uint32_t n_groups, per, in_flight;
+  FastDiv by_per, by_in_flight;
+};
+
 struct ScanArgs {
   const char *in_a;  // alpha
   const char *in_b;  // beta (forward) / dout (backward)
@@ -374,17 +404,29 @@ struct ScanArgs {
   int32_t n_chunks;       // ceil(seq / (WAVES*STEPS))
   int32_t n_tiles;        // tiles the workgroups walk: n_groups * n_chunks
   int32_t n_groups;       // column groups per chunk: n_ctiles / wg_cols
-  int32_t wg_cols;        // adjacent column tiles a workgroup covers side by side (1 or 2)
   int32_t look_waves;     // waves per column tile that look back in parallel (1..kMaxLookWaves)
   int32_t period;         // chunks of one sequence that a full grid works on at once (chain_anchor), >= 1
   uint32_t spin_limit;    // polls before a look-back gives up (kSpinLimit unless a test lowered it)
   uint32_t *hdr;          // workspace header
   uint64_t *words;        // tagged words
   const char *in_x;       // gated backward only: the scan's input x (in_a is the gate there)
+  TileOrder order;        // (depends on the grid: set at the launch)
+  FastDiv by_groups, by_row, by_period, by_reach, by_look;  // n_groups, tiles_per_row, period, look_waves * kMaxSpan, look_waves
 #ifdef FSS_TRACE
   uint64_t *trace;        // debug build: 8 timestamps per tile, written by lane 0 of every wave 0
 #endif
 };
+
+// The kernel's first argument, read again wherever this is called.  For what a tile needs once, at its
+// start: held from the start of the kernel to its end it would spill (scalar registers into lanes of
+// vector ones, all of it before the first load).  Not for the chain phase, whose every step some other
+// workgroup waits for (with all arguments read again bs 1 seq 65521 d 256 lost 2.5 %).
+__device__ __forceinline__ const ScanArgs &fresh_args() {
+  typedef const __attribute__((address_space(4))) ScanArgs *Kernarg;
+  Kernarg args = (Kernarg)__builtin_amdgcn_kernarg_segment_ptr();
+  asm volatile("" : "+s"(args));
+  return *(const ScanArgs *)args;
+}
 
 // Which column group the workgroup that takes slot `slot` of chunk `chunk` works on (tiles are
 // numbered chunk-major: tile = chunk * n_groups + slot, and workgroup b takes tiles b,
@@ -398,27 +440,20 @@ struct ScanArgs {
 // with its slowest workgroup.  A column's chunks stay on one XCD, and so do the words that
 // chain them.  The turn depends on the chunk alone, so every chunk's slots map onto its groups
 // one to one whatever the grid.
-struct TileOrder {
-  uint32_t n_groups, per, in_flight;
-};
-__host__ __device__ inline uint32_t wave_uniform(uint32_t x) {
-#if defined(__HIP_DEVICE_COMPILE__)
-  return __builtin_amdgcn_readfirstlane(x);  // (divisions run on the vector unit: pin the result back)
-#else
-  return x;
-#endif
-}
-__host__ __device__ inline TileOrder tile_order(uint32_t n_groups, uint32_t grid) {
+inline TileOrder tile_order(uint32_t n_groups, uint32_t grid) {
   TileOrder o;
   o.n_groups = n_groups;
   o.per = (n_groups & 7u) == 0 ? n_groups >> 3 : 0u;
-  o.in_flight = wave_uniform((grid + n_groups - 1) / n_groups);
+  o.in_flight = (grid + n_groups - 1) / n_groups;
   if (o.in_flight < 1) o.in_flight = 1;
+  o.by_per = fast_div(o.per > 0 ? o.per : 1);
+  o.by_in_flight = fast_div(o.in_flight);
   return o;
 }
 __host__ __device__ inline uint32_t tile_group(const TileOrder &o, uint32_t slot, uint32_t chunk) {
   if (o.per <= 1) return slot;
-  const uint32_t turn = wave_uniform((chunk / o.in_flight) % o.per);
+  const uint32_t round = divide(chunk, o.by_in_flight);
+  const uint32_t turn = round - divide(round, o.by_per) * o.per;
   uint32_t k = (slot >> 3) + turn;
   if (k >= o.per) k -= o.per;
   return (slot & 7u) * o.per + k;
@@ -533,6 +568,7 @@ struct TileCtx {
   int wcol;              // which of the workgroup's column tiles this wave belongs to
   int chunk, ctile;      // position of the tile: chunk of the sequence, column tile
   bool chained, last;    // more than one chunk in the sequence; this is the last one
+  uint32_t epoch;        // the header's epoch word, as loaded (launch_tag waits for it)
   uint32_t tag;          // epoch of this launch
   int64_t tile_base;     // byte offset of (batch, row 0, first channel of the tile)
   int64_t chan_row;      // index of (batch, first channel of the tile) in a (bs, d) array; wave-uniform
@@ -575,18 +611,36 @@ struct TileCtx {
 // stride-th chunk is an anchor as well: a chunk then never composes more than `stride` maps, at
 // the price of a chain of states stride chunks apart (each available one look-back after the
 // one before).  bs 1 seq 65521 d 256 bf16: backward 34.0 -> 31.3 us, forward+backward 60.6 -> 57.7 us.
-__host__ __device__ inline int chain_anchor(int chunk, int period, int stride) {
-  const int round_first = chunk - chunk % period;
-  const int by_round = round_first > 0 ? round_first - 1 : 0;
-  const int by_stride = (chunk - 1) / stride * stride;
-  return by_round > by_stride ? by_round : by_stride;
+__host__ __device__ inline int chain_anchor(int chunk, int period, const FastDiv &by_period, int stride,
+                                            const FastDiv &by_stride) {
+  const int round_first = static_cast<int>(divide(static_cast<uint32_t>(chunk), by_period)) * period;
+  const int of_round = round_first > 0 ? round_first - 1 : 0;
+  const int of_stride = chunk > 0 ? static_cast<int>(divide(static_cast<uint32_t>(chunk) - 1u, by_stride)) * stride : 0;
+  return of_round > of_stride ? of_round : of_stride;
 }
 
 // Chunks one look-back wave covers, one after the other, when `items` chunks (the anchor
 // included; never more than look * kMaxSpan) are dealt out to `look` waves: as few as the waves allow.
-__host__ __device__ inline int chunk_span(int items, int look) {
-  const int span = (items + look - 1) / look;
+__host__ __device__ inline int chunk_span(int items, int look, const FastDiv &by_look) {
+  const int span = static_cast<int>(divide(static_cast<uint32_t>(items + look - 1), by_look));
   return span < 1 ? 1 : (span > kMaxSpan ? kMaxSpan : span);
+}
+
+// Where the chunk stands in the chain.
+__device__ __forceinline__ void place_in_chain(const ScanArgs &p, TileCtx &c) {
+  if (!c.chained) return;
+  c.anchor = chain_anchor(c.chunk, p.period, p.by_period, p.look_waves * kMaxSpan, p.by_reach);
+  c.span = chunk_span(c.chunk - c.anchor, p.look_waves, p.by_look);
+}
+
+// The launch's tag, from the epoch word whose load went out when the workgroup started: waited for in
+// the chain phase, behind the rows of the first tile, and not before its loads (a memory round trip at
+// the start of every kernel).  It is the same for all of a workgroup's tiles; the asm keeps the compiler
+// from taking the wait out of the tile loop again.
+__device__ __forceinline__ uint32_t launch_tag(const TileCtx &c) {
+  uint32_t epoch = c.epoch;
+  asm volatile("" : "+v"(epoch));
+  return __builtin_amdgcn_readfirstlane(epoch) + 1u;
 }
 
 // One look at chunk `j` of this column tile: at its outgoing state (`want_state`: j is the

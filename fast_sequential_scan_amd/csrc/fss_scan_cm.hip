@@ -45,7 +45,7 @@ struct Flag {
 // RAGGED: seq is no multiple of VEC (a kernel of its own: the shifts cost the forward four spilled
 // registers, 2 % of the time of rows that need none).
 template <typename E, int VEC, int ROWS, bool BWD, bool RAGGED>
-__device__ __forceinline__ void cm_tile(const ScanArgs &p, const TileCtx &c, int64_t row0, int64_t n_rows) {
+__device__ __forceinline__ void cm_tile(const ScanArgs &p, TileCtx &c, int64_t row0, int64_t n_rows) {
   using RowT = Row<E, VEC>;
   using OneT = Row<E, 1>;
   const int64_t seq = c.seq;
@@ -191,10 +191,12 @@ __device__ __forceinline__ void cm_tile(const ScanArgs &p, const TileCtx &c, int
   }
 
   float slice_in = 0.0f;
-  if (c.chained || c.n_waves > 1)
+  if (c.chained || c.n_waves > 1) {
+    c.tag = launch_tag(c);
     chain_chunks<1, BWD>(p, c, &mA, &mB, nullptr, &slice_in, load_h);
-  else
+  } else {
     load_h();
+  }
   if (BWD && ragged) {
 #pragma unroll
     for (int r = 0; r < ROWS; ++r) place(hp[r]);
@@ -267,20 +269,22 @@ __global__ __launch_bounds__(1024) void cm_scan_kernel(const ScanArgs p) {
   c.trace_wave = 0;
 #endif
   c.chained = p.n_chunks > 1;
-  c.tag = c.chained ? __builtin_amdgcn_readfirstlane(ld_u32(p.hdr + HDR_EPOCH)) + 1u : 0u;
+  c.epoch = c.chained ? ld_u32(p.hdr + HDR_EPOCH) : 0u;
+  c.tag = 0u;
+  c.anchor = c.span = 0;
 
   uint32_t parity = 0;
   uint32_t tile_no = 0;
   for (uint32_t tile = blockIdx.x; tile < static_cast<uint32_t>(p.n_tiles); tile += gridDim.x, parity ^= 1u) {
     c.tile_no = ++tile_no;
     c.lds_map = lds_maps + parity * c.n_waves * 64;
-    const uint32_t chunk = __builtin_amdgcn_readfirstlane(tile / static_cast<uint32_t>(p.n_ctiles));
+    const ScanArgs &plan = fresh_args();
+    const uint32_t chunk = divide(tile, plan.by_groups);
     const uint32_t ctile = tile - chunk * static_cast<uint32_t>(p.n_ctiles);
     c.chunk = static_cast<int>(chunk);
     c.ctile = static_cast<int>(ctile);
     c.last = c.chunk == p.n_chunks - 1;
-    c.anchor = __builtin_amdgcn_readfirstlane(chain_anchor(c.chunk, p.period, p.look_waves * kMaxSpan));
-    c.span = __builtin_amdgcn_readfirstlane(chunk_span(c.chunk - c.anchor, p.look_waves));
+    place_in_chain(plan, c);
     cm_tile<E, VEC, ROWS, BWD, RAGGED>(p, c, static_cast<int64_t>(ctile) * ROWS, p.d);
   }
   count_out(p, c);
@@ -357,9 +361,9 @@ int run_cm_scan(int dtype, int dir, const void *alpha, const void *in_b, const v
   args.n_chunks = static_cast<int32_t>(pl.n_chunks);
   args.n_tiles = static_cast<int32_t>(pl.n_tiles);
   args.n_groups = static_cast<int32_t>(pl.n_rowtiles);
-  args.wg_cols = 1;
   args.look_waves = look_waves(pl.waves, 1);
   args.period = chain_period(pl.n_rowtiles, pl.waves);
+  set_divisors(args);
   args.spin_limit = __atomic_load_n(&g_spin_limit, __ATOMIC_RELAXED);
   args.hdr = static_cast<uint32_t *>(workspace);
   args.words = workspace ? reinterpret_cast<uint64_t *>(static_cast<char *>(workspace) + kHeaderBytes) : nullptr;

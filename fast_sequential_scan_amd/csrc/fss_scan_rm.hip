@@ -85,9 +85,13 @@ namespace fss {
 // access is guarded.  The two variants share no registers, so the guarded one
 // costs the fast one nothing.
 template <typename E, int VEC, int STEPS, bool BWD, bool STATE, bool FULL, int ALT>
-__device__ __forceinline__ void scan_tile(const ScanArgs &p, const StateArgs<STATE> &st, const TileCtx &c) {
+__device__ __forceinline__ void scan_tile(const ScanArgs &p, const StateArgs<STATE> &st, TileCtx &c) {
   using RowT = Row<E, VEC>;
-  const int64_t seq = c.seq, row_bytes = c.row_bytes, r0 = c.r0;
+  const int64_t seq = c.seq, r0 = c.r0;
+  int64_t row_bytes = c.row_bytes;
+  // (kept from being multiplied by every step's number ahead of the tile loop: a hundred scalar
+  // instructions, and as many spilled registers, that a workgroup would run before its first load)
+  if (!FULL) asm volatile("" : "+s"(row_bytes));
   const uint32_t lane_off = c.lane_off;
 
   RowT a[STEPS], b[STEPS];
@@ -196,6 +200,7 @@ __device__ __forceinline__ void scan_tile(const ScanArgs &p, const StateArgs<STA
       }
     }
     FSS_STAMP(c, p, 1);
+    c.tag = launch_tag(c);
     chain_chunks<VEC, BWD>(p, c, mA, mB, STATE ? seq_in : nullptr, state, load_h_early);
   }
 
@@ -276,9 +281,13 @@ __device__ __forceinline__ float sigmoid_f32(float z) {
 // The backward needs alpha[t+1] as the coefficient of step t and alpha[t] for its
 // elementwise part: a slice of STEPS steps loads STEPS+1 rows of the gate.
 template <typename E, int VEC, int STEPS, bool BWD, bool STATE, bool FULL, int ALT>
-__device__ __forceinline__ void gated_tile(const ScanArgs &p, const StateArgs<STATE> &st, const TileCtx &c) {
+__device__ __forceinline__ void gated_tile(const ScanArgs &p, const StateArgs<STATE> &st, TileCtx &c) {
   using RowT = Row<E, VEC>;
-  const int64_t seq = c.seq, row_bytes = c.row_bytes, r0 = c.r0;
+  const int64_t seq = c.seq, r0 = c.r0;
+  int64_t row_bytes = c.row_bytes;
+  // (kept from being multiplied by every step's number ahead of the tile loop: a hundred scalar
+  // instructions, and as many spilled registers, that a workgroup would run before its first load)
+  if (!FULL) asm volatile("" : "+s"(row_bytes));
   const uint32_t lane_off = c.lane_off;
   constexpr int kARows = BWD ? STEPS + 1 : STEPS;
 
@@ -386,6 +395,7 @@ __device__ __forceinline__ void gated_tile(const ScanArgs &p, const StateArgs<ST
 #pragma unroll
     for (int v = 0; v < VEC; ++v) state[v] = seq_in[v];
   } else {
+    c.tag = launch_tag(c);
     chain_chunks<VEC, false>(p, c, mA, mB, STATE ? seq_in : nullptr, state, [] {});
   }
 
@@ -504,7 +514,9 @@ __global__ __launch_bounds__(MAXW * 64) void scan_kernel(const ScanArgs p, const
 #endif
   c.chained = p.n_chunks > 1;
   // every workgroup of a launch reads the same value: it only changes when all are done
-  c.tag = c.chained ? __builtin_amdgcn_readfirstlane(ld_u32(p.hdr + HDR_EPOCH)) + 1u : 0u;
+  c.epoch = c.chained ? ld_u32(p.hdr + HDR_EPOCH) : 0u;
+  c.tag = 0u;
+  c.anchor = c.span = 0;
 
   // The grid is sized to be resident all at once; each workgroup takes one tile of every
   // gridDim of them (the blockIdx-th, or see tile_in_round).  Tiles are numbered chunk-major, so a tile
@@ -513,28 +525,28 @@ __global__ __launch_bounds__(MAXW * 64) void scan_kernel(const ScanArgs p, const
   // (which column group a slot of a chunk stands for: tile_order; bs 8 seq 4096 d 1024 bf16, forward +
   // backward, against slot s = group s: 96.3 -> 94.3 us on one set of tensors, 117.7 -> 111.0 us
   // over eight sets in rotation)
-  const TileOrder order = tile_order(static_cast<uint32_t>(p.n_groups), gridDim.x);
-  const uint32_t n_groups = order.n_groups;
   uint32_t parity = 0;
   uint32_t tile_no = 0;
-  const bool lines_shared = p.tiles_per_row > 1 && shares_lines(c.row_bytes);
-  for (uint32_t done = 0; done + blockIdx.x < static_cast<uint32_t>(p.n_tiles); done += gridDim.x, parity ^= 1u) {
-    const uint32_t left = static_cast<uint32_t>(p.n_tiles) - done;
+  const uint32_t n_tiles = static_cast<uint32_t>(p.n_tiles);
+  for (uint32_t done = 0; done + blockIdx.x < n_tiles; done += gridDim.x, parity ^= 1u) {
+    const ScanArgs &plan = fresh_args();
+    const TileOrder &order = plan.order;
+    const uint32_t n_groups = order.n_groups;
+    const bool lines_shared = plan.tiles_per_row > 1 && shares_lines(c.row_bytes);
+    const uint32_t left = n_tiles - done;
     const uint32_t tile = done + tile_in_round(order, blockIdx.x, left < gridDim.x ? left : gridDim.x, lines_shared);
     c.tile_no = ++tile_no;
     c.lds_map = lds_maps + (parity * waves_total + c.wcol * c.n_waves) * kLaneSlots;
     // unsigned, wave-uniform arithmetic: stays on the scalar unit
-    // (the compiler divides through a vector-unit reciprocal: pin the quotients back)
-    const uint32_t chunk = __builtin_amdgcn_readfirstlane(tile / n_groups);
+    const uint32_t chunk = divide(tile, plan.by_groups);
     const uint32_t group = tile_group(order, tile - chunk * n_groups, chunk);
     const uint32_t ctile = group * COLS + static_cast<uint32_t>(c.wcol);
-    const uint32_t batch = __builtin_amdgcn_readfirstlane(ctile / static_cast<uint32_t>(p.tiles_per_row));
-    const uint32_t coltile = ctile - batch * static_cast<uint32_t>(p.tiles_per_row);
+    const uint32_t batch = divide(ctile, plan.by_row);
+    const uint32_t coltile = ctile - batch * static_cast<uint32_t>(plan.tiles_per_row);
     c.chunk = static_cast<int>(chunk);
     c.ctile = static_cast<int>(ctile);
     c.last = c.chunk == p.n_chunks - 1;
-    c.anchor = __builtin_amdgcn_readfirstlane(chain_anchor(c.chunk, p.period, p.look_waves * kMaxSpan));
-    c.span = __builtin_amdgcn_readfirstlane(chunk_span(c.chunk - c.anchor, p.look_waves));
+    place_in_chain(plan, c);
 
     const int64_t col0 = static_cast<int64_t>(coltile) * kLaneSlots;  // first channel of the tile
     c.col_ok = col0 + c.lane * VEC < p.d;
@@ -587,7 +599,9 @@ int launch_one(const ScanArgs &args, const StateArgs<true> &state, const Plan &p
   const dim3 block(static_cast<uint32_t>(waves) * 64);
   StateArgs<STATE> st;
   if constexpr (STATE) st = state;
-  hipLaunchKernelGGL((scan_kernel<E, VEC, STEPS, BWD, STATE, GATED, ALT, COLS, kMaxW>), grid, block, lds, stream, args, st);
+  ScanArgs placed = args;
+  placed.order = tile_order(static_cast<uint32_t>(args.n_groups), grid.x);
+  hipLaunchKernelGGL((scan_kernel<E, VEC, STEPS, BWD, STATE, GATED, ALT, COLS, kMaxW>), grid, block, lds, stream, placed, st);
   const hipError_t e = hipGetLastError();
   if (e != hipSuccess) {
     tls_hip_error = static_cast<int>(e);

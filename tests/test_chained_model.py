@@ -183,3 +183,17 @@ def test_model_within_fp32_rounding_of_sequential(tiling, recipe):
     # the long-memory recipes really exercise the composed carries: a chunk's coefficient is not 0
     if recipe != "sigmoid" and tiling[0] * tiling[1] <= 512:
         assert np.prod(alpha[0, 1 : 1 + tiling[0] * tiling[1], 0].astype(np.float64)) > 1e-3
+
+
+def test_anchor_divides_exactly_over_the_whole_range():
+    """The kernels divide by multiplying (fast_div): exact for every 31-bit chunk and every divisor,
+    powers of two and their neighbours, the largest values included."""
+    lib = _native.lib()
+    rng = np.random.default_rng(3)
+    top = 2**31 - 1
+    divisors = sorted({v for k in range(31) for v in (2**k - 1, 2**k, 2**k + 1) if v >= 1} | {int(v) for v in rng.integers(1, top, 200)} | {top})
+    for n in divisors:
+        for chunk in {0, 1, n - 1, n, min(n + 1, top), min(2 * n, top), top - 1, top, *(int(v) for v in rng.integers(0, top, 8))}:
+            first = chunk - chunk % n
+            assert lib.fss_debug_chain_anchor(chunk, n, top) == max(first - 1, 0), (chunk, n)
+            assert lib.fss_debug_chain_anchor(chunk, top, n) == max((chunk - 1) // n * n if chunk else 0, top - 1 if chunk == top else 0), (chunk, n)
