@@ -243,6 +243,7 @@ int run_scan(int dtype, int dir, const void *alpha, const void *in_b, const void
   args.seq = seq;
   args.d = d;
   args.tiles_per_row = static_cast<int32_t>(pl.tiles_per_row);
+  args.row_lanes_log2 = 6;
   args.n_ctiles = static_cast<int32_t>(pl.n_ctiles);
   args.n_chunks = static_cast<int32_t>(pl.n_chunks);
   args.n_tiles = static_cast<int32_t>(pl.n_tiles);

@@ -405,6 +405,7 @@ struct ScanArgs {
   int32_t n_tiles;        // tiles the workgroups walk: n_groups * n_chunks
   int32_t n_groups;       // column groups per chunk: n_ctiles / wg_cols
   int32_t look_waves;     // waves per column tile that look back in parallel (1..kMaxLookWaves)
+  int32_t row_lanes_log2; // channel-major only: lanes that cover a row of at most half a wave's (6: the row has waves to itself)
   int32_t period;         // chunks of one sequence that a full grid works on at once (chain_anchor), >= 1
   uint32_t spin_limit;    // polls before a look-back gives up (kSpinLimit unless a test lowered it)
   uint32_t *hdr;          // workspace header

@@ -428,6 +428,7 @@ constexpr int kCmRowsFwd = 8, kCmRowsBwd = 4;
 
 struct CmPlan {
   int vec, waves;
+  int row_lanes_log2;  // below 6: several rows share a wave's vectors (rows of at most 32 lanes)
   int64_t n_rowtiles, n_chunks, n_tiles;
   size_t ws_bytes;
 };
@@ -465,7 +466,14 @@ inline int make_cm_plan(CmPlan &pl, int64_t rows, int64_t seq, int dtype, int di
   if (waves < 1 || waves > 16) return FSS_ERR_BAD_CONFIG;
   pl.vec = vec;
   pl.waves = waves;
-  pl.n_rowtiles = ceil_div(rr, dir == FSS_BWD ? kCmRowsBwd : kCmRowsFwd);
+  // rows of at most half a wave share its vectors (SHORT in fss_scan_cm.hip: faster from one row to
+  // a million, 1.1 times where a row takes 32 lanes, 8 times where it takes four); shorter than one lane's
+  // 16 bytes they keep the one-step kernels
+  pl.row_lanes_log2 = 6;
+  if (any_rows && vec == widest && waves == 1)
+    for (int l = 5; l >= 0 && ss <= (static_cast<int64_t>(vec) << l); --l) pl.row_lanes_log2 = l;
+  const int vectors = dir == FSS_BWD || pl.row_lanes_log2 < 6 ? kCmRowsBwd : kCmRowsFwd;
+  pl.n_rowtiles = ceil_div(rr, static_cast<int64_t>(vectors) << (6 - pl.row_lanes_log2));
   pl.n_chunks = ceil_div(ss, static_cast<int64_t>(waves) * 64 * vec);
   pl.n_tiles = pl.n_rowtiles * pl.n_chunks;
   if (pl.n_rowtiles > INT32_MAX || pl.n_chunks > INT32_MAX || pl.n_tiles > INT32_MAX) return FSS_ERR_BAD_SHAPE;

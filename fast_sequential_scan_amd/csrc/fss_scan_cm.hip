@@ -44,25 +44,35 @@ struct Flag {
 
 // RAGGED: seq is no multiple of VEC (a kernel of its own: the shifts cost the forward four spilled
 // registers, 2 % of the time of rows that need none).
-template <typename E, int VEC, int ROWS, bool BWD, bool RAGGED>
+// SHORT: rows that half a wave's lanes cover.  They lie back to back in memory, so 64/L of them share a
+// vector - L lanes each, a power of two, with the lane scan confined to them - instead of leaving
+// most lanes idle: a wave's load then is as long as other waves' are, and the kernel is bound by memory
+// again.  bf16 (64, 4096, 23) forward 90 -> 11.7 us, backward 122 -> 19.2; (64, 4096, 64) 64 -> 17.0 and 85 ->
+// 28.3 us (5.9 TB/s); (64, 1024, 250) 28.0 -> 17.7 and 38.2 -> 30.1 us; (2, 1024, 256) 6.3 -> 4.2 and 5.6 -> 5.0.
+template <typename E, int VEC, int ROWS, bool BWD, bool RAGGED, bool SHORT>
 __device__ __forceinline__ void cm_tile(const ScanArgs &p, TileCtx &c, int64_t row0, int64_t n_rows) {
   using RowT = Row<E, VEC>;
   using OneT = Row<E, 1>;
   const int64_t seq = c.seq;
-  const int lane = c.lane;
+  // lanes of a row, this lane's place among them, and the row's place among those that share the vector
+  const int lanes = SHORT ? 1 << p.row_lanes_log2 : 64;
+  const int lane = SHORT ? c.lane & (lanes - 1) : c.lane;
+  const int row_of_lane = SHORT ? c.lane >> p.row_lanes_log2 : 0;
+  const int rows_per_vector = SHORT ? 64 >> p.row_lanes_log2 : 1;
   const int64_t slice = static_cast<int64_t>(c.chunk) * c.n_waves + c.wave;
   const int64_t r_base = (slice * 64 + lane) * VEC;             // first scan position of this lane
   const bool in_seq = r_base < seq;
   // The last lane of the scan may hold fewer than VEC steps (backward: the missing ones are the low end
   // of its vector, timesteps below 0).  It loads the VEC timesteps that end (backward: start) with the
   // sequence and moves them to their places, so that no lane reads outside its row and no load waits.
-  const bool ragged = RAGGED && slice * 64 * VEC < seq && seq < (slice + 1) * 64 * VEC;  // in this slice
+  const bool ragged = RAGGED && (SHORT || (slice * 64 * VEC < seq && seq < (slice + 1) * 64 * VEC));  // in this slice
   const int missing = ragged && in_seq && seq - r_base < VEC ? VEC - static_cast<int>(seq - r_base) : 0;
   const int64_t t_lo = BWD ? seq - r_base - VEC : r_base;       // lowest timestep of the vector
   const int64_t t_hi = t_lo + VEC - 1;
   // wave-uniform base (the lowest timestep any lane of the slice holds) + a 32-bit lane offset
-  const int64_t t_base = BWD ? seq - (slice * 64 + 64) * VEC : slice * 64 * VEC;
-  const uint32_t lane_off = static_cast<uint32_t>((BWD ? 63 - lane : lane) * RowT::kBytes);
+  const int64_t t_base = BWD ? seq - (slice * 64 + lanes) * VEC : slice * 64 * VEC;
+  const uint32_t lane_off = static_cast<uint32_t>((BWD ? lanes - 1 - lane : lane) * RowT::kBytes) +
+                            (SHORT ? static_cast<uint32_t>(row_of_lane) * static_cast<uint32_t>(seq) * E::kBytes : 0u);
 
   RowT a[ROWS], b[ROWS], hp[BWD ? ROWS : 1];
   float edge_a[BWD ? ROWS : 1], edge_h[BWD ? ROWS : 1];
@@ -89,8 +99,8 @@ __device__ __forceinline__ void cm_tile(const ScanArgs &p, TileCtx &c, int64_t r
   // ---- phase 1a: loads ---------------------------------------------------------------
 #pragma unroll
   for (int r = 0; r < ROWS; ++r) {
-    const int64_t row = row0 + r;
-    ok[r] = in_seq && row < n_rows;
+    const int64_t row = row0 + r * rows_per_vector;
+    ok[r] = in_seq && row + row_of_lane < n_rows;
     a[r].fill(1.0f);  // outside: identity steps
     b[r].fill(0.0f);
     if (ok[r]) {
@@ -113,7 +123,7 @@ __device__ __forceinline__ void cm_tile(const ScanArgs &p, TileCtx &c, int64_t r
     for (int r = 0; r < ROWS; ++r) {
       OneT ea;
       ea.fill(0.0f);
-      if (lane == 0 && ok[r] && t_hi + 1 < seq) ea.load((gcptr_t)p.in_a + ((row0 + r) * seq + t_hi + 1) * E::kBytes);
+      if (!SHORT && lane == 0 && ok[r] && t_hi + 1 < seq) ea.load((gcptr_t)p.in_a + ((row0 + r) * seq + t_hi + 1) * E::kBytes);
       const float from_prev = __shfl_up(a[r].get(0), 1);  // lane-1 holds timesteps just above ours
       edge_a[r] = lane == 0 ? ea.get(0) : from_prev;
     }
@@ -128,10 +138,10 @@ __device__ __forceinline__ void cm_tile(const ScanArgs &p, TileCtx &c, int64_t r
         eh[r].fill(0.0f);
         hp[r].fill(0.0f);
         if (ok[r]) {
-          const int64_t off = ((row0 + r) * seq + t_base) * E::kBytes;
+          const int64_t off = ((row0 + r * rows_per_vector) * seq + t_base) * E::kBytes;
           load_vector(hp[r], p.in_h, off, Flag<kNtH>());
         }
-        if (lane == 63 && ok[r] && t_lo >= 1) eh[r].load((gcptr_t)p.in_h + ((row0 + r) * seq + t_lo - 1) * E::kBytes);
+        if (!SHORT && lane == 63 && ok[r] && t_lo >= 1) eh[r].load((gcptr_t)p.in_h + ((row0 + r) * seq + t_lo - 1) * E::kBytes);
       }
     }
   };
@@ -162,7 +172,8 @@ __device__ __forceinline__ void cm_tile(const ScanArgs &p, TileCtx &c, int64_t r
     }
   }
 #pragma unroll
-  for (int off = 1; off < 64; off <<= 1) {
+  for (int off = 1; off < (SHORT ? 32 : 64); off <<= 1) {
+    if (SHORT && off >= lanes) break;
 #pragma unroll
     for (int r = 0; r < ROWS; ++r) {
       const float pa = __shfl_up(A[r], off), pb = __shfl_up(B[r], off);
@@ -191,7 +202,7 @@ __device__ __forceinline__ void cm_tile(const ScanArgs &p, TileCtx &c, int64_t r
   }
 
   float slice_in = 0.0f;
-  if (c.chained || c.n_waves > 1) {
+  if (!SHORT && (c.chained || c.n_waves > 1)) {
     c.tag = launch_tag(c);
     chain_chunks<1, BWD>(p, c, &mA, &mB, nullptr, &slice_in, load_h);
   } else {
@@ -206,7 +217,7 @@ __device__ __forceinline__ void cm_tile(const ScanArgs &p, TileCtx &c, int64_t r
 #pragma unroll
     for (int r = 0; r < ROWS; ++r) {
       const float from_next = __shfl_down(hp[r].get(VEC - 1), 1);  // lane+1 holds timesteps just below ours
-      edge_h[r] = lane == 63 ? eh[r].get(0) : from_next;
+      edge_h[r] = lane == lanes - 1 ? eh[r].get(0) : from_next;
     }
   }
 
@@ -219,7 +230,7 @@ __device__ __forceinline__ void cm_tile(const ScanArgs &p, TileCtx &c, int64_t r
   }
 #pragma unroll
   for (int r = 0; r < ROWS; ++r) {
-    float state = fma0(A[r], lane_read(slice_in, r), B[r]);
+    float state = SHORT ? B[r] : fma0(A[r], lane_read(slice_in, r), B[r]);
     float o0[VEC], o1[VEC];
 #pragma unroll
     for (int j = 0; j < VEC; ++j) {
@@ -229,7 +240,7 @@ __device__ __forceinline__ void cm_tile(const ScanArgs &p, TileCtx &c, int64_t r
       if (BWD) o1[VEC - 1 - j] = state * h_prev(r, j);
     }
     if (ok[r]) {
-      const int64_t off = ((row0 + r) * seq + t_base) * E::kBytes;
+      const int64_t off = ((row0 + r * rows_per_vector) * seq + t_base) * E::kBytes;
       RowT o;
       o.pack(o0);
       store_vector(o, p.out0, off, Flag<(BWD ? kNtOutBwd : kNtOutFwd)>());
@@ -244,7 +255,7 @@ __device__ __forceinline__ void cm_tile(const ScanArgs &p, TileCtx &c, int64_t r
 
 // ScanArgs here: seq = the contiguous length, d = number of rows (bs * channels),
 // n_ctiles = ceil(rows / ROWS) row groups, n_chunks = ceil(seq / (waves*64*VEC)).
-template <typename E, int VEC, int ROWS, bool BWD, bool RAGGED>
+template <typename E, int VEC, int ROWS, bool BWD, bool RAGGED, bool SHORT>
 __global__ __launch_bounds__(1024) void cm_scan_kernel(const ScanArgs p) {
   extern __shared__ float lds[];
   __shared__ uint32_t s_ready[16];  // per wave: see announce_map
@@ -285,24 +296,24 @@ __global__ __launch_bounds__(1024) void cm_scan_kernel(const ScanArgs p) {
     c.ctile = static_cast<int>(ctile);
     c.last = c.chunk == p.n_chunks - 1;
     place_in_chain(plan, c);
-    cm_tile<E, VEC, ROWS, BWD, RAGGED>(p, c, static_cast<int64_t>(ctile) * ROWS, p.d);
+    cm_tile<E, VEC, ROWS, BWD, RAGGED, SHORT>(p, c, static_cast<int64_t>(ctile) * (SHORT ? ROWS * (64 >> p.row_lanes_log2) : ROWS), p.d);
   }
   count_out(p, c);
 }
 
 // ---- launching ---------------------------------------------------------------------
 
-template <typename E, int VEC, bool BWD, bool RAGGED = false>
+template <typename E, int VEC, bool BWD, bool RAGGED = false, bool SHORT = false>
 int launch_cm_one(const ScanArgs &args, const CmPlan &pl, int max_groups, hipStream_t stream) {
-  constexpr int kRows = BWD ? kCmRowsBwd : kCmRowsFwd;
+  constexpr int kRows = BWD || SHORT ? kCmRowsBwd : kCmRowsFwd;  // (eight vectors a lane would cost SHORT 23 spilled registers)
   static int resident[17] = {0};
   const int waves = pl.waves;
   const size_t lds = lds_bytes(waves, 1);
-  const int fit = resident_workgroups(cm_scan_kernel<E, VEC, kRows, BWD, RAGGED>, waves, lds, resident);
+  const int fit = resident_workgroups(cm_scan_kernel<E, VEC, kRows, BWD, RAGGED, SHORT>, waves, lds, resident);
   if (fit <= 0) return FSS_ERR_LAUNCH;
   int64_t n_groups = pl.n_tiles < fit ? pl.n_tiles : fit;
   if (max_groups > 0 && max_groups < n_groups) n_groups = max_groups;
-  hipLaunchKernelGGL((cm_scan_kernel<E, VEC, kRows, BWD, RAGGED>), dim3(static_cast<uint32_t>(n_groups)),
+  hipLaunchKernelGGL((cm_scan_kernel<E, VEC, kRows, BWD, RAGGED, SHORT>), dim3(static_cast<uint32_t>(n_groups)),
                      dim3(static_cast<uint32_t>(waves) * 64), lds, stream, args);
   const hipError_t e = hipGetLastError();
   if (e != hipSuccess) {
@@ -315,6 +326,7 @@ int launch_cm_one(const ScanArgs &args, const CmPlan &pl, int max_groups, hipStr
 template <typename E, bool BWD>
 int launch_cm(const ScanArgs &args, const CmPlan &pl, int max_groups, hipStream_t stream) {
   constexpr int kWidest = 16 / E::kBytes;
+  if (pl.row_lanes_log2 < 6) return launch_cm_one<E, kWidest, BWD, true, true>(args, pl, max_groups, stream);
   if (pl.vec == kWidest)
     return args.seq % kWidest == 0 ? launch_cm_one<E, kWidest, BWD>(args, pl, max_groups, stream)
                                    : launch_cm_one<E, kWidest, BWD, true>(args, pl, max_groups, stream);
@@ -357,6 +369,7 @@ int run_cm_scan(int dtype, int dir, const void *alpha, const void *in_b, const v
   args.seq = seq;
   args.d = bs * d;  // rows
   args.tiles_per_row = 1;
+  args.row_lanes_log2 = pl.row_lanes_log2;
   args.n_ctiles = static_cast<int32_t>(pl.n_rowtiles);
   args.n_chunks = static_cast<int32_t>(pl.n_chunks);
   args.n_tiles = static_cast<int32_t>(pl.n_tiles);

@@ -208,3 +208,12 @@ def test_cm_growing_recurrence_with_zero_state_stays_zero():
         assert not torch.isnan(h).any()
         want = torch.pow(2.0, torch.arange(9000, device=DEV, dtype=torch.float64)).to(torch.float32).to(dtype).float()
         assert torch.equal(h, want.expand_as(h))
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32], ids=["bf16", "f16", "f32"])
+@pytest.mark.parametrize("seq", [4, 5, 8, 9, 15, 16, 17, 31, 32, 33, 64, 65, 127, 128, 129, 250, 256, 257])
+@pytest.mark.parametrize("bs,d", [(1, 1), (3, 43), (2, 131)])
+def test_short_rows_share_vectors(oracle, bs, d, seq, dtype):
+    """Rows of at most half a wave's lanes: 1, 2, 4 .. 32 lanes each (and the first length that takes a
+    whole wave again), last vectors full and ragged, last tiles full and not."""
+    _run(oracle, bs, d, seq, dtype, seed=seq + d)
