@@ -461,15 +461,11 @@ __host__ __device__ inline uint32_t tile_group(const TileOrder &o, uint32_t slot
 }
 
 // Which tile of a round of the grid (`count` tiles: the grid's size, fewer in the last round) workgroup
-// `block` takes.  Ordinarily its own index.  Where rows of several
-// tiles share cache lines (shares_lines) and the groups
-// could not be dealt out in eighths, the workgroups of one XCD take consecutive tiles instead, so that
-// both tiles that touch a line touch it in one L2.  (One to one over block < count, and every
-// workgroup still takes its tiles in ascending order, so a tile's wait for lower ones is as safe as
-// before.)  Not otherwise: it puts a column's consecutive chunks on different XCDs, and rows of whole
-// lines gain nothing for it (bf16 (1, 65521, 256) backward 36 -> 41 us).
-__host__ __device__ inline uint32_t tile_in_round(const TileOrder &o, uint32_t block, uint32_t count, bool lines_shared) {
-  if (o.per != 0 || !lines_shared) return block;
+// `block` takes: its own index, or - where takes_consecutive_tiles says so - the workgroups of one XCD
+// take consecutive ones.  (One to one over block < count, and every workgroup still takes its tiles in
+// ascending order, so a tile's wait for lower ones is as safe either way.)
+__host__ __device__ inline uint32_t tile_in_round(uint32_t block, uint32_t count, bool consecutive) {
+  if (!consecutive) return block;
   const uint32_t xcd = block & 7u, extra = count & 7u;
   return xcd * (count >> 3) + (xcd < extra ? xcd : extra) + (block >> 3);
 }
@@ -539,7 +535,7 @@ constexpr int64_t kStreamDoutBytes = static_cast<int64_t>(80) << 20;
 
 // Rows that are no whole number of 128-byte lines put two column tiles, worked on by different workgroups,
 // on the lines at their seam.  The L2 puts such a line together only if both tiles meet it there
-// (tile_in_round) and only if it is kept until both have: a line read or written with the hint is gone
+// (takes_consecutive_tiles) and only if it is kept until both have: a line read or written with the hint is gone
 // before the neighbour comes and travels twice, the second time as a partial write.  Such rows
 // therefore run without any hint - unless they are whole 64-byte sectors, which the memory writes
 // without reading (bf16 (4, 17738, 1376): forward 126 us with the hints, 133 us without).  bf16, with the
@@ -549,6 +545,18 @@ constexpr int64_t kStreamDoutBytes = static_cast<int64_t>(80) << 20;
 constexpr int kLineBytes = 128, kSectorBytes = 64;
 __host__ __device__ inline bool shares_lines(int64_t row_bytes) { return row_bytes % kLineBytes != 0; }
 __host__ __device__ inline bool shares_sectors(int64_t row_bytes) { return row_bytes % kSectorBytes != 0; }
+
+// Where rows of several tiles share lines and an XCD's share of the column groups is small (an eighth of
+// them begins and ends at a seam) or does not exist, the workgroups of one XCD take consecutive tiles of
+// a round instead, so that both tiles that touch a line touch it in one L2.  It puts a column's
+// consecutive chunks on different XCDs, so not otherwise: with whole lines bf16 (1, 65521, 256) backward
+// 36 -> 41 us; sharing lines, groups per XCD 1: (1, 65521, 1000) forward 111 -> 93, backward 185 -> 145 us;
+// 3: (2, 32768, 1500) 151 -> 140, 236 -> 211; 4: (4, 16384, 1000) 97 -> 94, 153 -> 143; 7: (14, 12174,
+// 438) 128 -> 126, 203 -> 206; 8: (8, 8192, 1000) 92 -> 94, 138 -> 143 us.
+constexpr uint32_t kConsecutiveBelow = 6;
+__host__ __device__ inline bool takes_consecutive_tiles(const TileOrder &o, int32_t tiles_per_row, int64_t row_bytes) {
+  return o.per < kConsecutiveBelow && tiles_per_row > 1 && shares_lines(row_bytes);
+}
 
 #ifdef FSS_TRACE
 #define FSS_STAMP(c, p, slot)                                                                   \

@@ -532,14 +532,15 @@ __global__ __launch_bounds__(MAXW * 64) void scan_kernel(const ScanArgs p, const
     const ScanArgs &plan = fresh_args();
     const TileOrder &order = plan.order;
     const uint32_t n_groups = order.n_groups;
-    const bool lines_shared = plan.tiles_per_row > 1 && shares_lines(c.row_bytes);
+    const bool consecutive = takes_consecutive_tiles(order, plan.tiles_per_row, c.row_bytes);
     const uint32_t left = n_tiles - done;
-    const uint32_t tile = done + tile_in_round(order, blockIdx.x, left < gridDim.x ? left : gridDim.x, lines_shared);
+    const uint32_t tile = done + tile_in_round(blockIdx.x, left < gridDim.x ? left : gridDim.x, consecutive);
     c.tile_no = ++tile_no;
     c.lds_map = lds_maps + (parity * waves_total + c.wcol * c.n_waves) * kLaneSlots;
     // unsigned, wave-uniform arithmetic: stays on the scalar unit
     const uint32_t chunk = divide(tile, plan.by_groups);
-    const uint32_t group = tile_group(order, tile - chunk * n_groups, chunk);
+    const uint32_t slot = tile - chunk * n_groups;
+    const uint32_t group = consecutive ? slot : tile_group(order, slot, chunk);
     const uint32_t ctile = group * COLS + static_cast<uint32_t>(c.wcol);
     const uint32_t batch = divide(ctile, plan.by_row);
     const uint32_t coltile = ctile - batch * static_cast<uint32_t>(plan.tiles_per_row);
