@@ -373,8 +373,8 @@ struct FastDiv {
   uint8_t first, second;  // shifts
 };
 inline FastDiv fast_div(uint32_t n) {
-  int bits = 0;  // of n - 1: the least l with n <= 2^l
-  while (bits < 32 && (uint64_t{1} << bits) < n) ++bits;
+  if (n <= 1) return FastDiv{1u, 0, 0};
+  const int bits = 32 - __builtin_clz(n - 1);  // the least l with n <= 2^l
   FastDiv f;
   f.mul = static_cast<uint32_t>(((uint64_t{1} << 32) * ((uint64_t{1} << bits) - n)) / n + 1);
   f.first = static_cast<uint8_t>(bits < 1 ? bits : 1);

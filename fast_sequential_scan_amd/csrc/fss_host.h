@@ -87,11 +87,13 @@ inline int chain_period(int64_t n_groups, int waves) {
   return static_cast<int>(period < 1 ? 1 : (period > (1 << 20) ? (1 << 20) : period));
 }
 
-// The divisors of a launch whose other numbers are set (the tile order's come with the grid).
+// The divisors of a launch whose other numbers are set (the tile order's come with the grid); a launch
+// that chains nothing, as a decode step's, needs only the first two.
 inline void set_divisors(ScanArgs &args) {
-  args.order = TileOrder{};
   args.by_groups = fast_div(static_cast<uint32_t>(args.n_groups));
   args.by_row = fast_div(static_cast<uint32_t>(args.tiles_per_row));
+  args.by_period = args.by_reach = args.by_look = FastDiv{1u, 0, 0};
+  if (args.n_chunks <= 1) return;
   args.by_period = fast_div(static_cast<uint32_t>(args.period));
   args.by_reach = fast_div(static_cast<uint32_t>(args.look_waves * kMaxSpan));
   args.by_look = fast_div(static_cast<uint32_t>(args.look_waves));

@@ -158,15 +158,11 @@ class SequentialScanState(Function):
         return grad_alpha, grad_beta, grad_h_before
 
 
-def _fast_with_state(first: torch.Tensor, second: torch.Tensor, h_before: Optional[torch.Tensor], gated: bool):
+def _resolve_fast_state() -> Any:
     global _fast_state
-    if _fast_state is _UNRESOLVED:
-        binding = _ext.fast_dispatch()
-        _fast_state = binding.state_scan if binding is not None else None
-    if (_fast_state is None or not isinstance(first, torch.Tensor) or not isinstance(second, torch.Tensor)
-            or not (h_before is None or isinstance(h_before, torch.Tensor))):
-        return None
-    return _fast_state(first, second, h_before, gated)
+    binding = _ext.fast_dispatch()
+    _fast_state = binding.state_scan if binding is not None else None
+    return _fast_state
 
 
 def scan_with_state(
@@ -175,9 +171,12 @@ def scan_with_state(
     """``h[t] = alpha[t]*h[t-1] + beta[t]`` from ``h[-1] = h_before`` (zeros when None; when given,
     ``alpha[:, 0]`` multiplies it).  Returns ``(h, h_last)`` with ``h_last`` the fp32 state after the
     last step, to be passed as ``h_before`` of the next segment."""
-    pair = _fast_with_state(alpha, beta, h_before, False)
-    if pair is not None:
-        return pair
+    fast = _fast_state if _fast_state is not _UNRESOLVED else _resolve_fast_state()
+    if (fast is not None and isinstance(alpha, torch.Tensor) and isinstance(beta, torch.Tensor)
+            and (h_before is None or isinstance(h_before, torch.Tensor))):
+        pair = fast(alpha, beta, h_before, False)
+        if pair is not None:
+            return pair
     return SequentialScanState.apply(alpha, beta, h_before)
 
 
@@ -245,9 +244,12 @@ def scan_gated_with_state(
     """:func:`scan_gated` from ``h[-1] = h_before`` (fp32 ``(bs, d_model)``, zeros when None).  Returns
     ``(h, h_last)`` with ``h_last`` the fp32 state after the last step, to be passed as ``h_before`` of
     the next segment (chunked prefill, decoding, a sequence sharded over devices)."""
-    pair = _fast_with_state(gate, x, h_before, True)
-    if pair is not None:
-        return pair
+    fast = _fast_state if _fast_state is not _UNRESOLVED else _resolve_fast_state()
+    if (fast is not None and isinstance(gate, torch.Tensor) and isinstance(x, torch.Tensor)
+            and (h_before is None or isinstance(h_before, torch.Tensor))):
+        pair = fast(gate, x, h_before, True)
+        if pair is not None:
+            return pair
     return SequentialScanGatedState.apply(gate, x, h_before)
 
 
