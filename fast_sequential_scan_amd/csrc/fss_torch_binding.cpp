@@ -10,8 +10,8 @@
 // the headline shape take and several times those of short sequences.
 //
 // This path only takes the common case: contiguous GPU tensors of the expected type and one
-// shape, on the current device, outside autocast, with a workspace of sufficient size already
-// registered for the current stream.  Everything else (and every error message) stays with the
+// shape, on the current device, outside autocast and torch.jit.trace, with a workspace of sufficient size
+// already registered for the current stream.  Everything else (and every error message) stays with the
 // Python wrappers: `scan` returns None and the caller goes through them, and a backward that
 // meets anything unusual calls them back.
 #include <torch/extension.h>
@@ -21,6 +21,7 @@
 #include <c10/hip/HIPFunctions.h>
 #include <c10/hip/HIPStream.h>
 #include <torch/csrc/autograd/functions/basic_ops.h>
+#include <torch/csrc/jit/frontend/tracer.h>
 
 #include <cstdint>
 #include <map>
@@ -127,6 +128,11 @@ bool plain_state(const at::Tensor &s, const at::Tensor &like) {
 
 // A dual tensor of forward-mode differentiation: left to the Python Functions, which refuse it.
 bool has_tangent(const at::Tensor &t) { return t._fw_grad(/*level=*/0).defined(); }
+
+// A call that torch.jit.trace records: left to the Python Functions, which it records as one operator.  Of
+// this path it would see the allocation of the outputs and not the launch that fills them, and the
+// traced program would return memory that nothing wrote.
+bool is_traced() { return torch::jit::tracer::isTracing(); }
 
 int64_t code_of(at::ScalarType t) { return t == at::kBFloat16 ? 0 : t == at::kFloat ? 1 : t == at::kHalf ? 2 : -1; }
 
@@ -366,7 +372,7 @@ void forget_workspaces() {
 // cover the call.  `code`: 0 bf16, 1 fp32, 2 fp16 (FSS_BF16, FSS_F32, FSS_F16); `kind`: 0 the plain
 // scan of (alpha, beta), 1 the gated scan of (gate, x).
 std::optional<at::Tensor> dispatch(const at::Tensor &alpha, const at::Tensor &beta, int64_t code, int kind) {
-  if (!g_fwd || code < 0 || code > 2) return std::nullopt;
+  if (!g_fwd || code < 0 || code > 2 || is_traced()) return std::nullopt;
   const at::ScalarType dtype = dtype_of(code);
   if (!plain_tensor(alpha, dtype) || !plain_tensor(beta, dtype)) return std::nullopt;
   if (alpha.sizes() != beta.sizes() || alpha.device() != beta.device() || alpha.numel() == 0) return std::nullopt;
@@ -417,7 +423,7 @@ bool wants_gradient(const at::Tensor &alpha, const at::Tensor &beta, const std::
 // the host 17 us, here 5; a segment's forward and backward 130 us, here 55.)
 std::optional<std::tuple<at::Tensor, at::Tensor>> state_scan(const at::Tensor &alpha, const at::Tensor &beta,
                                                              const std::optional<at::Tensor> &h_before, bool gated) {
-  if (!g_state_fwd || !alpha.defined()) return std::nullopt;
+  if (!g_state_fwd || !alpha.defined() || is_traced()) return std::nullopt;
   const at::ScalarType t = alpha.scalar_type();
   const int64_t code = code_of(t);
   if (code < 0 || !plain_tensor(alpha, t) || !plain_tensor(beta, t)) return std::nullopt;

@@ -49,6 +49,34 @@ def test_same_bits_as_the_python_functions(api, function, dtype, shape):
     assert api(alpha, beta).grad_fn is None
 
 
+@pytest.mark.parametrize("grads", [False, True], ids=["no_grad", "grads"])
+@pytest.mark.parametrize("name", ["scan_cu", "scan_cu_single", "scan_cu_fp16", "scan_cm", "scan_gated", "scan_with_state",
+                                  "scan_with_state_from_zero", "scan_gated_with_state"])
+def test_traced_calls_run_the_scan_again(name, grads):
+    """torch.jit.trace of every public entry point, run on other inputs than it was traced with: the
+    results and the gradients of the call itself.  The dispatch must decline a call that is being traced
+    (its launches are invisible to the tracer: the trace would return tensors that nothing writes)."""
+    import fast_sequential_scan_amd as lib
+
+    api = {"scan_with_state_from_zero": lambda a, b: lib.scan_with_state(a, b)}.get(name) or getattr(lib, name)
+    dtype = {"scan_cu_single": torch.float32, "scan_cu_fp16": torch.float16}.get(name, torch.bfloat16)
+
+    def inputs(seed):
+        alpha, beta, _ = _tensors((2, 300, 96), dtype, seed)
+        state = torch.randn(2, 96, device=DEV, generator=torch.Generator(DEV).manual_seed(seed))
+        return [t.requires_grad_(grads) for t in ((alpha, beta, state) if name.endswith("with_state") else (alpha, beta))]
+
+    first, second = inputs(1), inputs(2)
+    api(*first)  # a workspace exists from here on
+    traced = torch.jit.trace(api, tuple(first), check_trace=False)
+    got, want = (out if isinstance(out, tuple) else (out,) for out in (traced(*second), api(*second)))
+    assert len(got) == len(want) and all(torch.equal(g, w) for g, w in zip(got, want))
+    if grads:
+        got, want = (torch.autograd.grad([o.float().sum() for o in outs], second) for outs in (got, want))
+        assert all(torch.equal(g, w) for g, w in zip(got, want))
+    ext.workspace_status()
+
+
 def test_what_it_does_not_cover_goes_through_python():
     alpha, beta, dout = _tensors((2, 300, 256), torch.bfloat16, seed=3)
     scan_cu(alpha, beta)  # a workspace exists from here on
