@@ -158,11 +158,21 @@ class SequentialScanState(Function):
         return grad_alpha, grad_beta, grad_h_before
 
 
-def _resolve_fast_state() -> Any:
+# (the dispatch returns plain tensors; of a subclass's tensors the Functions return the subclass's)
+_PLAIN_TYPES = (torch.Tensor, torch.nn.Parameter)
+
+
+def _fast_state_scan(
+    first: torch.Tensor, second: torch.Tensor, h_before: Optional[torch.Tensor], gated: bool
+) -> Optional[Tuple[torch.Tensor, torch.Tensor]]:
     global _fast_state
-    binding = _ext.fast_dispatch()
-    _fast_state = binding.state_scan if binding is not None else None
-    return _fast_state
+    if _fast_state is _UNRESOLVED:
+        binding = _ext.fast_dispatch()
+        _fast_state = binding.state_scan if binding is not None else None
+    if (_fast_state is None or type(first) not in _PLAIN_TYPES or type(second) not in _PLAIN_TYPES
+            or (h_before is not None and type(h_before) not in _PLAIN_TYPES)):
+        return None
+    return _fast_state(first, second, h_before, gated)
 
 
 def scan_with_state(
@@ -171,13 +181,8 @@ def scan_with_state(
     """``h[t] = alpha[t]*h[t-1] + beta[t]`` from ``h[-1] = h_before`` (zeros when None; when given,
     ``alpha[:, 0]`` multiplies it).  Returns ``(h, h_last)`` with ``h_last`` the fp32 state after the
     last step, to be passed as ``h_before`` of the next segment."""
-    fast = _fast_state if _fast_state is not _UNRESOLVED else _resolve_fast_state()
-    if (fast is not None and isinstance(alpha, torch.Tensor) and isinstance(beta, torch.Tensor)
-            and (h_before is None or isinstance(h_before, torch.Tensor))):
-        pair = fast(alpha, beta, h_before, False)
-        if pair is not None:
-            return pair
-    return SequentialScanState.apply(alpha, beta, h_before)
+    pair = _fast_state_scan(alpha, beta, h_before, False)
+    return pair if pair is not None else SequentialScanState.apply(alpha, beta, h_before)
 
 
 class SequentialScanGated(Function):
@@ -244,13 +249,8 @@ def scan_gated_with_state(
     """:func:`scan_gated` from ``h[-1] = h_before`` (fp32 ``(bs, d_model)``, zeros when None).  Returns
     ``(h, h_last)`` with ``h_last`` the fp32 state after the last step, to be passed as ``h_before`` of
     the next segment (chunked prefill, decoding, a sequence sharded over devices)."""
-    fast = _fast_state if _fast_state is not _UNRESOLVED else _resolve_fast_state()
-    if (fast is not None and isinstance(gate, torch.Tensor) and isinstance(x, torch.Tensor)
-            and (h_before is None or isinstance(h_before, torch.Tensor))):
-        pair = fast(gate, x, h_before, True)
-        if pair is not None:
-            return pair
-    return SequentialScanGatedState.apply(gate, x, h_before)
+    pair = _fast_state_scan(gate, x, h_before, True)
+    return pair if pair is not None else SequentialScanGatedState.apply(gate, x, h_before)
 
 
 class SequentialScanChannelMajor(Function):

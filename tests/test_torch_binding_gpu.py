@@ -325,3 +325,26 @@ def test_scans_with_states_same_bits_as_the_python_wrappers(shape, dtype, with_s
     with torch.autograd.forward_ad.dual_level(), pytest.raises((RuntimeError, NotImplementedError)):
         api(torch.autograd.forward_ad.make_dual(alpha, dout), beta, states[0] if with_state else None)
     ext.workspace_status()
+
+
+@pytest.mark.parametrize("gated", [False, True], ids=["plain", "gated"])
+@pytest.mark.parametrize("grads", [False, True], ids=["no_grad", "grads"])
+def test_tensor_subclasses_in_scans_with_states(gated, grads):
+    """Tensors of a subclass, any one of the three: types and bits of the Function's results.  A Parameter
+    as the incoming state (a learned one) is taken by the dispatch."""
+    class Tagged(torch.Tensor):
+        pass
+
+    api = scan_cuda.scan_gated_with_state if gated else scan_with_state
+    function = scan_cuda.SequentialScanGatedState if gated else scan_cuda.SequentialScanState
+    alpha, beta, _ = _tensors((2, 50, 96), torch.bfloat16, seed=8)
+    plain = [alpha, beta, torch.randn(2, 96, device=DEV, generator=torch.Generator(DEV).manual_seed(3))]
+    api(*plain)  # a workspace exists from here on
+    for tagged in ((0,), (1,), (2,), (0, 1, 2)):
+        args = [(t.as_subclass(Tagged) if i in tagged else t.clone()).requires_grad_(grads) for i, t in enumerate(plain)]
+        got, want = api(*args), function.apply(*args)
+        assert [type(t) for t in got] == [type(t) for t in want]
+        assert all(torch.equal(g.as_subclass(torch.Tensor), w.as_subclass(torch.Tensor)) for g, w in zip(got, want))
+    h, _ = api(alpha, beta, torch.nn.Parameter(plain[2]))
+    assert type(h) is torch.Tensor and "StateNode" in _node_name(h)
+    ext.workspace_status()
