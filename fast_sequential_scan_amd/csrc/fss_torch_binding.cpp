@@ -376,6 +376,7 @@ std::optional<at::Tensor> dispatch(const at::Tensor &alpha, const at::Tensor &be
   const at::ScalarType dtype = dtype_of(code);
   if (!plain_tensor(alpha, dtype) || !plain_tensor(beta, dtype)) return std::nullopt;
   if (alpha.sizes() != beta.sizes() || alpha.device() != beta.device() || alpha.numel() == 0) return std::nullopt;
+  if (has_tangent(alpha) || has_tangent(beta)) return std::nullopt;
   if (at::autocast::is_autocast_enabled(at::kCUDA)) return std::nullopt;
   const int device = alpha.device().index();
   if (device != c10::hip::current_device()) return std::nullopt;

@@ -77,6 +77,22 @@ def test_traced_calls_run_the_scan_again(name, grads):
     ext.workspace_status()
 
 
+@pytest.mark.parametrize("grads", [False, True], ids=["no_grad", "grads"])
+@pytest.mark.parametrize("api", [scan_cu, scan_cu_single, scan_fp16, scan_cm, scan_gated])
+def test_forward_mode_is_refused(api, grads):
+    """A dual tensor of forward-mode differentiation, as either input: an error, and no result without a tangent."""
+    dtype = {scan_cu_single: torch.float32, scan_fp16: torch.float16}.get(api, torch.bfloat16)
+    inputs = _tensors((2, 50, 96), dtype, seed=6)[:2]
+    api(*inputs)  # a workspace exists from here on
+    for i in range(2):
+        with torch.autograd.forward_ad.dual_level():
+            args = [t.clone().requires_grad_(grads) for t in inputs]
+            args[i] = torch.autograd.forward_ad.make_dual(args[i], torch.ones_like(args[i]))
+            with pytest.raises((RuntimeError, NotImplementedError)):
+                api(*args)
+    ext.workspace_status()
+
+
 def test_what_it_does_not_cover_goes_through_python():
     alpha, beta, dout = _tensors((2, 300, 256), torch.bfloat16, seed=3)
     scan_cu(alpha, beta)  # a workspace exists from here on
