@@ -388,6 +388,7 @@ __host__ __device__ inline uint32_t divide(uint32_t x, const FastDiv &f) {
 
 struct TileOrder {
   uint32_t n_groups, per, in_flight;
+  uint32_t consecutive;  // 1: the workgroups of an XCD take consecutive tiles of a round (launch_order)
   FastDiv by_per, by_in_flight;
 };
 
@@ -430,8 +431,8 @@ __device__ __forceinline__ const ScanArgs &fresh_args() {
 }
 
 // Which column group the workgroup that takes slot `slot` of chunk `chunk` works on (tiles are
-// numbered chunk-major: tile = chunk * n_groups + slot, and workgroup b takes tiles b,
-// b + grid, ...).  Workgroup b runs on XCD b % 8, so with the groups dealt out in eighths the
+// numbered chunk-major: tile = chunk * n_groups + slot; workgroup b takes tiles b, b + grid, ... -
+// unless launch_order has the XCDs take consecutive ones: tile_in_round).  Workgroup b runs on XCD b % 8, so with the groups dealt out in eighths the
 // workgroups of one XCD share consecutive groups: whole rows of a few batch items instead of
 // one 256-byte stripe of every row (`per` groups each; 0: the number of groups does not
 // divide by 8, slot s takes group s).  Within its eighth the deal moves on by one group from one
@@ -447,6 +448,7 @@ inline TileOrder tile_order(uint32_t n_groups, uint32_t grid) {
   o.per = (n_groups & 7u) == 0 ? n_groups >> 3 : 0u;
   o.in_flight = (grid + n_groups - 1) / n_groups;
   if (o.in_flight < 1) o.in_flight = 1;
+  o.consecutive = 0;
   o.by_per = fast_div(o.per > 0 ? o.per : 1);
   o.by_in_flight = fast_div(o.in_flight);
   return o;
@@ -461,13 +463,30 @@ __host__ __device__ inline uint32_t tile_group(const TileOrder &o, uint32_t slot
 }
 
 // Which tile of a round of the grid (`count` tiles: the grid's size, fewer in the last round) workgroup
-// `block` takes: its own index, or - where takes_consecutive_tiles says so - the workgroups of one XCD
+// `block` takes: its own index, or - where launch_order says so - the workgroups of one XCD
 // take consecutive ones.  (One to one over block < count, and every workgroup still takes its tiles in
 // ascending order, so a tile's wait for lower ones is as safe either way.)
 __host__ __device__ inline uint32_t tile_in_round(uint32_t block, uint32_t count, bool consecutive) {
   if (!consecutive) return block;
   const uint32_t xcd = block & 7u, extra = count & 7u;
   return xcd * (count >> 3) + (xcd < extra ? xcd : extra) + (block >> 3);
+}
+
+// The tile that workgroup `block` works on in the round of the grid that begins with tile `done`
+// (done + block < n_tiles).  The kernels' own arithmetic, and fss_debug_tile_order's.
+struct TilePlace {
+  uint32_t chunk, group;
+};
+__host__ __device__ inline TilePlace tile_place(const TileOrder &o, const FastDiv &by_groups, uint32_t n_tiles, uint32_t grid,
+                                                uint32_t done, uint32_t block) {
+  const bool consecutive = o.consecutive != 0;
+  const uint32_t left = n_tiles - done;
+  const uint32_t tile = done + tile_in_round(block, left < grid ? left : grid, consecutive);
+  TilePlace t;
+  t.chunk = divide(tile, by_groups);
+  const uint32_t slot = tile - t.chunk * o.n_groups;
+  t.group = consecutive ? slot : tile_group(o, slot, t.chunk);
+  return t;
 }
 
 // Optional (bs, d) fp32 rows of the scans with a state entering/leaving the sequence.
@@ -535,7 +554,7 @@ constexpr int64_t kStreamDoutBytes = static_cast<int64_t>(80) << 20;
 
 // Rows that are no whole number of 128-byte lines put two column tiles, worked on by different workgroups,
 // on the lines at their seam.  The L2 puts such a line together only if both tiles meet it there
-// (takes_consecutive_tiles) and only if it is kept until both have: a line read or written with the hint is gone
+// (launch_order) and only if it is kept until both have: a line read or written with the hint is gone
 // before the neighbour comes and travels twice, the second time as a partial write.  Such rows
 // therefore run without any hint - unless they are whole 64-byte sectors, which the memory writes
 // without reading (bf16 (4, 17738, 1376): forward 126 us with the hints, 133 us without).  bf16, with the
@@ -543,8 +562,8 @@ constexpr int64_t kStreamDoutBytes = static_cast<int64_t>(80) << 20;
 // 93 and 307 -> 161 us; fp32 (8, 2048, 1501) 80 -> 66 and 149 -> 115 us; gated fp16 (14, 6405, 856) 140 ->
 // 119 and 303 -> 219 us, where the order alone gives 219, 417; 134, 262; 79, 150; 130, 263 us.
 constexpr int kLineBytes = 128, kSectorBytes = 64;
-__host__ __device__ inline bool shares_lines(int64_t row_bytes) { return row_bytes % kLineBytes != 0; }
-__host__ __device__ inline bool shares_sectors(int64_t row_bytes) { return row_bytes % kSectorBytes != 0; }
+inline bool shares_lines(int64_t row_bytes) { return row_bytes % kLineBytes != 0; }
+inline bool shares_sectors(int64_t row_bytes) { return row_bytes % kSectorBytes != 0; }
 
 // Where rows of several tiles share lines and an XCD's share of the column groups is small (an eighth of
 // them begins and ends at a seam) or does not exist, the workgroups of one XCD take consecutive tiles of
@@ -554,8 +573,10 @@ __host__ __device__ inline bool shares_sectors(int64_t row_bytes) { return row_b
 // 3: (2, 32768, 1500) 151 -> 140, 236 -> 211; 4: (4, 16384, 1000) 97 -> 94, 153 -> 143; 7: (14, 12174,
 // 438) 128 -> 126, 203 -> 206; 8: (8, 8192, 1000) 92 -> 94, 138 -> 143 us.
 constexpr uint32_t kConsecutiveBelow = 6;
-__host__ __device__ inline bool takes_consecutive_tiles(const TileOrder &o, int32_t tiles_per_row, int64_t row_bytes) {
-  return o.per < kConsecutiveBelow && tiles_per_row > 1 && shares_lines(row_bytes);
+inline TileOrder launch_order(uint32_t n_groups, int32_t tiles_per_row, int64_t row_bytes, uint32_t grid) {
+  TileOrder o = tile_order(n_groups, grid);
+  o.consecutive = o.per < kConsecutiveBelow && tiles_per_row > 1 && shares_lines(row_bytes) ? 1u : 0u;
+  return o;
 }
 
 #ifdef FSS_TRACE

@@ -530,18 +530,12 @@ __global__ __launch_bounds__(MAXW * 64) void scan_kernel(const ScanArgs p, const
   const uint32_t n_tiles = static_cast<uint32_t>(p.n_tiles);
   for (uint32_t done = 0; done + blockIdx.x < n_tiles; done += gridDim.x, parity ^= 1u) {
     const ScanArgs &plan = fresh_args();
-    const TileOrder &order = plan.order;
-    const uint32_t n_groups = order.n_groups;
-    const bool consecutive = takes_consecutive_tiles(order, plan.tiles_per_row, c.row_bytes);
-    const uint32_t left = n_tiles - done;
-    const uint32_t tile = done + tile_in_round(blockIdx.x, left < gridDim.x ? left : gridDim.x, consecutive);
+    const TilePlace place = tile_place(plan.order, plan.by_groups, n_tiles, gridDim.x, done, blockIdx.x);
     c.tile_no = ++tile_no;
     c.lds_map = lds_maps + (parity * waves_total + c.wcol * c.n_waves) * kLaneSlots;
     // unsigned, wave-uniform arithmetic: stays on the scalar unit
-    const uint32_t chunk = divide(tile, plan.by_groups);
-    const uint32_t slot = tile - chunk * n_groups;
-    const uint32_t group = consecutive ? slot : tile_group(order, slot, chunk);
-    const uint32_t ctile = group * COLS + static_cast<uint32_t>(c.wcol);
+    const uint32_t chunk = place.chunk;
+    const uint32_t ctile = place.group * COLS + static_cast<uint32_t>(c.wcol);
     const uint32_t batch = divide(ctile, plan.by_row);
     const uint32_t coltile = ctile - batch * static_cast<uint32_t>(plan.tiles_per_row);
     c.chunk = static_cast<int>(chunk);
@@ -601,7 +595,7 @@ int launch_one(const ScanArgs &args, const StateArgs<true> &state, const Plan &p
   StateArgs<STATE> st;
   if constexpr (STATE) st = state;
   ScanArgs placed = args;
-  placed.order = tile_order(static_cast<uint32_t>(args.n_groups), grid.x);
+  placed.order = launch_order(static_cast<uint32_t>(args.n_groups), args.tiles_per_row, args.d * E::kBytes, grid.x);
   hipLaunchKernelGGL((scan_kernel<E, VEC, STEPS, BWD, STATE, GATED, ALT, COLS, kMaxW>), grid, block, lds, stream, placed, st);
   const hipError_t e = hipGetLastError();
   if (e != hipSuccess) {
