@@ -389,20 +389,20 @@ int fss_debug_tile_groups(int32_t n_groups, int32_t grid, int32_t n_tiles, int32
   return FSS_OK;
 }
 
-int fss_debug_tile_order(int32_t n_groups, int32_t n_chunks, int32_t tiles_per_row, int64_t row_bytes, int32_t grid,
+int fss_debug_tile_order(int32_t n_groups, int32_t n_chunks, int32_t row_groups, int64_t row_bytes, int32_t grid,
                          int32_t *chunks, int32_t *groups) {
   if (!chunks || !groups) return FSS_ERR_NULL_POINTER;
-  if (n_groups <= 0 || n_chunks <= 0 || tiles_per_row <= 0 || row_bytes <= 0 || grid <= 0 ||
+  if (n_groups <= 0 || n_chunks <= 0 || row_groups <= 0 || n_groups % row_groups != 0 || row_bytes <= 0 || grid <= 0 ||
       static_cast<int64_t>(n_groups) * n_chunks > INT32_MAX)
     return FSS_ERR_BAD_SHAPE;
   const uint32_t n_tiles = static_cast<uint32_t>(n_groups) * static_cast<uint32_t>(n_chunks);
-  const uint32_t workgroups = static_cast<uint32_t>(grid);
-  const fss::TileOrder order = fss::launch_order(static_cast<uint32_t>(n_groups), tiles_per_row, row_bytes, workgroups);
+  const fss::TileOrder order = fss::launch_order(static_cast<uint32_t>(n_groups), static_cast<uint32_t>(row_groups), row_bytes,
+                                                 static_cast<uint32_t>(grid));
   const fss::FastDiv by_groups = fss::fast_div(static_cast<uint32_t>(n_groups));
-  for (uint32_t i = 0; i < n_tiles; ++i) {
-    const fss::TilePlace t = fss::tile_place(order, by_groups, n_tiles, workgroups, i - i % workgroups, i % workgroups);
-    chunks[i] = static_cast<int32_t>(t.chunk);
-    groups[i] = static_cast<int32_t>(t.group);
+  for (uint32_t nth = 0; nth < n_tiles; ++nth) {
+    const fss::TilePlace t = fss::tile_place(order, by_groups, n_tiles, nth);
+    chunks[nth] = static_cast<int32_t>(t.chunk);
+    groups[nth] = static_cast<int32_t>(t.group);
   }
   return FSS_OK;
 }

@@ -388,8 +388,8 @@ __host__ __device__ inline uint32_t divide(uint32_t x, const FastDiv &f) {
 
 struct TileOrder {
   uint32_t n_groups, per, in_flight;
-  uint32_t consecutive;  // 1: the workgroups of an XCD take consecutive tiles of a round (launch_order)
-  FastDiv by_per, by_in_flight;
+  uint32_t row_groups;  // column groups of a row where the tiles go by whole rows (launch_order), otherwise 0
+  FastDiv by_per, by_in_flight, by_row_groups, by_eight_rows;
 };
 
 struct ScanArgs {
@@ -432,7 +432,7 @@ __device__ __forceinline__ const ScanArgs &fresh_args() {
 
 // Which column group the workgroup that takes slot `slot` of chunk `chunk` works on (tiles are
 // numbered chunk-major: tile = chunk * n_groups + slot; workgroup b takes tiles b, b + grid, ... -
-// unless launch_order has the XCDs take consecutive ones: tile_in_round).  Workgroup b runs on XCD b % 8, so with the groups dealt out in eighths the
+// unless they go by whole rows: whole_rows_tile).  Workgroup b runs on XCD b % 8, so with the groups dealt out in eighths the
 // workgroups of one XCD share consecutive groups: whole rows of a few batch items instead of
 // one 256-byte stripe of every row (`per` groups each; 0: the number of groups does not
 // divide by 8, slot s takes group s).  Within its eighth the deal moves on by one group from one
@@ -448,7 +448,8 @@ inline TileOrder tile_order(uint32_t n_groups, uint32_t grid) {
   o.per = (n_groups & 7u) == 0 ? n_groups >> 3 : 0u;
   o.in_flight = (grid + n_groups - 1) / n_groups;
   if (o.in_flight < 1) o.in_flight = 1;
-  o.consecutive = 0;
+  o.row_groups = 0;
+  o.by_row_groups = o.by_eight_rows = FastDiv{1u, 0, 0};
   o.by_per = fast_div(o.per > 0 ? o.per : 1);
   o.by_in_flight = fast_div(o.in_flight);
   return o;
@@ -462,30 +463,31 @@ __host__ __device__ inline uint32_t tile_group(const TileOrder &o, uint32_t slot
   return (slot & 7u) * o.per + k;
 }
 
-// Which tile of a round of the grid (`count` tiles: the grid's size, fewer in the last round) workgroup
-// `block` takes: its own index, or - where launch_order says so - the workgroups of one XCD
-// take consecutive ones.  (One to one over block < count, and every workgroup still takes its tiles in
-// ascending order, so a tile's wait for lower ones is as safe either way.)
-__host__ __device__ inline uint32_t tile_in_round(uint32_t block, uint32_t count, bool consecutive) {
-  if (!consecutive) return block;
-  const uint32_t xcd = block & 7u, extra = count & 7u;
-  return xcd * (count >> 3) + (xcd < extra ? xcd : extra) + (block >> 3);
+// The order for rows that share cache lines: of every eight consecutive "rows" of tiles - the column groups of
+// one batch item in one chunk - each XCD takes one, so that the tiles that meet on a line meet in one L2.
+// The `nth` tile taken, in chunk-major numbers.  Of fewer than eight rows at the end each is
+// dealt out to the XCDs in consecutive shares.  A tile waits for the tiles of its columns in earlier chunks: a
+// whole number of rows earlier at the same place of the row, so they are taken before it here as in
+// the chunk-major order.
+__host__ __device__ inline uint32_t whole_rows_tile(const TileOrder &o, uint32_t n_tiles, uint32_t nth) {
+  const uint32_t begin = divide(nth, o.by_eight_rows) * 8u * o.row_groups, i = nth - begin;
+  if (n_tiles - begin >= 8u * o.row_groups) return begin + (i & 7u) * o.row_groups + (i >> 3);
+  const uint32_t row = divide(i, o.by_row_groups) * o.row_groups, k = i - row;
+  const uint32_t share = o.row_groups >> 3, extra = o.row_groups & 7u, xcd = k & 7u;
+  return begin + row + xcd * share + (xcd < extra ? xcd : extra) + (k >> 3);
 }
 
-// The tile that workgroup `block` works on in the round of the grid that begins with tile `done`
-// (done + block < n_tiles).  The kernels' own arithmetic, and fss_debug_tile_order's.
+// The tile that is the `nth` to be taken: workgroup b of a grid takes the b-th, the (b + grid)-th, ...
+// The kernels' own arithmetic, and fss_debug_tile_order's.
 struct TilePlace {
   uint32_t chunk, group;
 };
-__host__ __device__ inline TilePlace tile_place(const TileOrder &o, const FastDiv &by_groups, uint32_t n_tiles, uint32_t grid,
-                                                uint32_t done, uint32_t block) {
-  const bool consecutive = o.consecutive != 0;
-  const uint32_t left = n_tiles - done;
-  const uint32_t tile = done + tile_in_round(block, left < grid ? left : grid, consecutive);
+__host__ __device__ inline TilePlace tile_place(const TileOrder &o, const FastDiv &by_groups, uint32_t n_tiles, uint32_t nth) {
+  const uint32_t tile = o.row_groups ? whole_rows_tile(o, n_tiles, nth) : nth;
   TilePlace t;
   t.chunk = divide(tile, by_groups);
   const uint32_t slot = tile - t.chunk * o.n_groups;
-  t.group = consecutive ? slot : tile_group(o, slot, t.chunk);
+  t.group = o.row_groups ? slot : tile_group(o, slot, t.chunk);
   return t;
 }
 
@@ -557,25 +559,31 @@ constexpr int64_t kStreamDoutBytes = static_cast<int64_t>(80) << 20;
 // (launch_order) and only if it is kept until both have: a line read or written with the hint is gone
 // before the neighbour comes and travels twice, the second time as a partial write.  Such rows
 // therefore run without any hint - unless they are whole 64-byte sectors, which the memory writes
-// without reading (bf16 (4, 17738, 1376): forward 126 us with the hints, 133 us without).  bf16, with the
-// tiles' order: (18, 4006, 1682) forward 238 -> 181 us, backward 442 -> 307 us; (17, 1516, 2249) 162 ->
-// 93 and 307 -> 161 us; fp32 (8, 2048, 1501) 80 -> 66 and 149 -> 115 us; gated fp16 (14, 6405, 856) 140 ->
-// 119 and 303 -> 219 us, where the order alone gives 219, 417; 134, 262; 79, 150; 130, 263 us.
+// without reading.  bf16, in the order by whole rows, with the hints -> without: (18, 4006, 1682) forward 219 ->
+// 185 us, backward 415 -> 314 us; (17, 1516, 2249) 128 -> 88 and 249 -> 147 us; fp32 (8, 2048, 1501) 80 -> 66
+// and 149 -> 114 us; gated fp16 (14, 6405, 856) 128 -> 118 and 264 -> 218 us; whole sectors, (4, 17738, 1376), 126 ->
+// 133 and 198 -> 199 us, (7, 6000, 1440) 79 -> 82 and 132 -> 136 us.
 constexpr int kLineBytes = 128, kSectorBytes = 64;
 inline bool shares_lines(int64_t row_bytes) { return row_bytes % kLineBytes != 0; }
 inline bool shares_sectors(int64_t row_bytes) { return row_bytes % kSectorBytes != 0; }
 
-// Where rows of several tiles share lines and an XCD's share of the column groups is small (an eighth of
-// them begins and ends at a seam) or does not exist, the workgroups of one XCD take consecutive tiles of
-// a round instead, so that both tiles that touch a line touch it in one L2.  It puts a column's
-// consecutive chunks on different XCDs, so not otherwise: with whole lines bf16 (1, 65521, 256) backward
-// 36 -> 41 us; sharing lines, groups per XCD 1: (1, 65521, 1000) forward 111 -> 93, backward 185 -> 145 us;
-// 3: (2, 32768, 1500) 151 -> 140, 236 -> 211; 4: (4, 16384, 1000) 97 -> 94, 153 -> 143; 7: (14, 12174,
-// 438) 128 -> 126, 203 -> 206; 8: (8, 8192, 1000) 92 -> 94, 138 -> 143 us.
-constexpr uint32_t kConsecutiveBelow = 6;
-inline TileOrder launch_order(uint32_t n_groups, int32_t tiles_per_row, int64_t row_bytes, uint32_t grid) {
+// Where rows of several column groups share lines and an XCD's share of the groups is small (an eighth of
+// them begins and ends at a seam) or does not exist, the tiles go by whole rows, so that the tiles
+// that touch a line touch it in one L2.  Without hints, eighths or chunk-major -> whole rows: (18, 4006, 1682)
+// forward 206 -> 185 us, backward 356 -> 314 us; (17, 1516, 2249) 117 -> 88, 202 -> 147; gated fp16 (14, 6405, 856)
+// 133 -> 118, 261 -> 218; one group per XCD, (1, 65521, 1000), 111 -> 88, 184 -> 136; three, (2, 32768, 1500),
+// 150 -> 136, 237 -> 207; four, (4, 16384, 1000), 97 -> 91, 151 -> 135; launches of one round (6, 2048, 418) 15.9 ->
+// 12.6, 16.0 -> 15.6, (1, 4096, 1300) 15.4 -> 13.6, 18.2 -> 16.4.  From six groups on the eighths have few seams
+// and whole rows change little: six, (8, 8000, 760), 65 -> 64, 109 -> 110; seven, (14, 12174, 438), 128 -> 122,
+// 200 -> 201; eight, (8, 8192, 1000), 92 -> 91, 139 -> 140.  Rows of whole lines have nothing to gain, and
+// with the chunks of a column on different XCDs bf16 (1, 65521, 256) lost: backward 36 -> 41 us.
+constexpr uint32_t kWholeRowsBelow = 6;
+inline TileOrder launch_order(uint32_t n_groups, uint32_t row_groups, int64_t row_bytes, uint32_t grid) {
   TileOrder o = tile_order(n_groups, grid);
-  o.consecutive = o.per < kConsecutiveBelow && tiles_per_row > 1 && shares_lines(row_bytes) ? 1u : 0u;
+  if (o.per >= kWholeRowsBelow || row_groups <= 1 || row_groups >= 1u << 28 || !shares_lines(row_bytes)) return o;
+  o.row_groups = row_groups;
+  o.by_row_groups = fast_div(row_groups);
+  o.by_eight_rows = fast_div(8u * row_groups);
   return o;
 }
 

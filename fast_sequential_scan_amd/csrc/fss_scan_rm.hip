@@ -518,19 +518,19 @@ __global__ __launch_bounds__(MAXW * 64) void scan_kernel(const ScanArgs p, const
   c.tag = 0u;
   c.anchor = c.span = 0;
 
-  // The grid is sized to be resident all at once; each workgroup takes one tile of every
-  // gridDim of them (the blockIdx-th, or see tile_in_round).  Tiles are numbered chunk-major, so a tile
-  // only ever waits for tiles with smaller numbers: those belong to a resident
-  // workgroup that reaches them no later than this one reaches its own.
+  // The grid is sized to be resident all at once; each workgroup walks the tiles
+  // blockIdx, blockIdx + gridDim, ... of an order in which every tile comes after those it waits for
+  // (tile_place): they belong to a resident workgroup that reaches them no later than this one
+  // reaches its own.
   // (which column group a slot of a chunk stands for: tile_order; bs 8 seq 4096 d 1024 bf16, forward +
   // backward, against slot s = group s: 96.3 -> 94.3 us on one set of tensors, 117.7 -> 111.0 us
   // over eight sets in rotation)
   uint32_t parity = 0;
   uint32_t tile_no = 0;
   const uint32_t n_tiles = static_cast<uint32_t>(p.n_tiles);
-  for (uint32_t done = 0; done + blockIdx.x < n_tiles; done += gridDim.x, parity ^= 1u) {
+  for (uint32_t tile = blockIdx.x; tile < n_tiles; tile += gridDim.x, parity ^= 1u) {
     const ScanArgs &plan = fresh_args();
-    const TilePlace place = tile_place(plan.order, plan.by_groups, n_tiles, gridDim.x, done, blockIdx.x);
+    const TilePlace place = tile_place(plan.order, plan.by_groups, n_tiles, tile);
     c.tile_no = ++tile_no;
     c.lds_map = lds_maps + (parity * waves_total + c.wcol * c.n_waves) * kLaneSlots;
     // unsigned, wave-uniform arithmetic: stays on the scalar unit
@@ -595,7 +595,8 @@ int launch_one(const ScanArgs &args, const StateArgs<true> &state, const Plan &p
   StateArgs<STATE> st;
   if constexpr (STATE) st = state;
   ScanArgs placed = args;
-  placed.order = launch_order(static_cast<uint32_t>(args.n_groups), args.tiles_per_row, args.d * E::kBytes, grid.x);
+  placed.order = launch_order(static_cast<uint32_t>(args.n_groups), static_cast<uint32_t>(args.tiles_per_row / COLS),
+                              args.d * E::kBytes, grid.x);
   hipLaunchKernelGGL((scan_kernel<E, VEC, STEPS, BWD, STATE, GATED, ALT, COLS, kMaxW>), grid, block, lds, stream, placed, st);
   const hipError_t e = hipGetLastError();
   if (e != hipSuccess) {

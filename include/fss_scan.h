@@ -176,16 +176,17 @@ uint32_t fss_debug_set_spin_limit(uint32_t polls);
 uint64_t fss_debug_noalloc_reinit_after(uint64_t launches);
 /*
  * Test hooks (host only, no device call): the order in which the row-major kernels take their
- * tiles - a chunk of the sequence of one column group each, n_groups * n_chunks of them - over a grid
- * of `grid` workgroups (no more than there are tiles), `tiles_per_row` column tiles to a row of
- * `row_bytes` bytes.  chunks[i] and groups[i] receive the tile that workgroup i % grid takes as its
- * (i / grid)-th, for i = 0 .. n_groups * n_chunks - 1.  Every tile must be taken once.
- * fss_debug_tile_groups: the groups alone, of the launches whose workgroups take tiles b, b + grid, ...
- * of the chunk-major order (tile = chunk * n_groups + slot): rows of one column tile or of whole
- * 128-byte lines, or at least 48 column groups in a number that divides by 8.  No counterpart in the
- * reference (one block per batch row, no tiles).
+ * tiles - one chunk of the sequence of one column group each, n_groups * n_chunks of them - over a
+ * grid of `grid` workgroups, where a row of `row_bytes` bytes is `row_groups` column groups wide.
+ * chunks[i] and groups[i] receive the tile that workgroup i % grid takes as its (i / grid)-th, for
+ * i = 0 .. n_groups * n_chunks - 1.  Every tile must be taken once, and after those of its column's
+ * earlier chunks.
+ * fss_debug_tile_groups: the groups alone, tile = chunk * n_groups + slot, of the launches that take
+ * the chunks one after the other: rows of one column group or of whole 128-byte lines, or at least
+ * 48 column groups in a number that divides by 8.  (Other launches: whole rows to an XCD.)
+ * No counterpart in the reference (one block per batch row, no tiles).
  */
-int fss_debug_tile_order(int32_t n_groups, int32_t n_chunks, int32_t tiles_per_row, int64_t row_bytes,
+int fss_debug_tile_order(int32_t n_groups, int32_t n_chunks, int32_t row_groups, int64_t row_bytes,
                          int32_t grid, int32_t *chunks, int32_t *groups);
 int fss_debug_tile_groups(int32_t n_groups, int32_t grid, int32_t n_tiles, int32_t *groups);
 

@@ -474,51 +474,59 @@ def test_tile_order_covers_every_group_of_every_chunk_once():
     assert lib.fss_debug_tile_groups(8, 8, 8, None) != 0
 
 
-def _tile_order(lib, n_groups, n_chunks, tiles_per_row, row_bytes, grid):
+def _tile_order(lib, n_groups, n_chunks, row_groups, row_bytes, grid):
     n_tiles = n_groups * n_chunks
     chunks, groups = (ctypes.c_int32 * n_tiles)(), (ctypes.c_int32 * n_tiles)()
-    assert lib.fss_debug_tile_order(n_groups, n_chunks, tiles_per_row, row_bytes, grid, chunks, groups) == 0
+    assert lib.fss_debug_tile_order(n_groups, n_chunks, row_groups, row_bytes, grid, chunks, groups) == 0
     return np.frombuffer(chunks, dtype=np.int32), np.frombuffer(groups, dtype=np.int32)
 
 
-# (column groups, chunks, column tiles per row, bytes per row, workgroups): rows of whole lines and not, one
-# tile per row, shares of the groups per XCD of none, 1, 5 (the most with consecutive tiles), 6 and 8, grids
-# of one round, of whole rounds and with every remainder of the last one
+# (column groups, chunks, column groups per row, bytes per row, workgroups): rows of whole lines and not, of one
+# group; shares of the groups per XCD of none, 1, 5 (the most that go by whole rows), 6 and 8; rows in multiples of
+# eight, fewer than eight and with every remainder; rows of 2 to 40 groups
 _ORDERS = [(8, 40, 8, 2000, 256), (9, 30, 3, 700, 256), (40, 9, 5, 1000, 256), (48, 9, 6, 1400, 256), (64, 8, 8, 2000, 256),
            (64, 16, 8, 2048, 256), (12, 7, 1, 140, 44), (9, 16, 3, 700, 144), (36, 3, 36, 4498, 768), (7, 1, 7, 1700, 7),
-           *((9, 11, 3, 700, grid) for grid in range(1, 100)), *((40, 3, 5, 1000, grid) for grid in range(1, 121, 7)),
-           *((48, 3, 6, 1400, grid) for grid in range(1, 145, 7))]
+           (15, 8, 3, 700, 120), (40, 1, 40, 5000, 40),
+           *((9, n, 3, 700, grid) for n in range(1, 18) for grid in (8, 44, 256)), *((row, 11, row, 1000, 256) for row in range(2, 40)),
+           *((48, n, 6, 1400, 256) for n in range(1, 10))]
 
 
-def test_workgroups_take_every_tile_once():
-    """What the kernels compute (the same code on the host): every tile is taken, once; a workgroup's tiles
-    come in the order of the chunks, since a tile waits for tiles of earlier chunks; where rows share lines
-    the workgroups of an XCD (index modulo 8) take consecutive tiles, elsewhere the order is the one of
-    fss_debug_tile_groups."""
+def test_workgroups_take_every_tile_once_and_after_those_it_waits_for():
+    """What the kernels compute (the same code on the host): every tile is taken, once, and after the tiles
+    it waits for, those of its column's earlier chunks.  (The n-th tile is workgroup n % grid's: in a launch of
+    one round a tile thus only waits for workgroups with smaller numbers, which the device starts first, and
+    the launch gets on with part of the device while a kernel on another stream holds the rest.)  Where
+    rows share lines every row of a chunk is taken by one XCD (index modulo 8), of fewer than eight rows at
+    the end consecutive shares; elsewhere the order is the one of fss_debug_tile_groups."""
     lib = _native.lib()
-    kinds = set()
-    for n_groups, n_chunks, per_row, row_bytes, grid in _ORDERS:
-        what = (n_groups, n_chunks, per_row, row_bytes, grid)
+    by_rows = 0
+    for what in _ORDERS:
+        n_groups, n_chunks, row_groups, row_bytes, grid = what
         chunks, groups = _tile_order(lib, *what)
         n_tiles = n_groups * n_chunks
         tiles = chunks * n_groups + groups
         assert sorted(tiles.tolist()) == list(range(n_tiles)), what
-        for b in range(grid):
-            assert (np.diff(chunks[b::grid]) >= 0).all(), what
-        of_blocks = _tile_groups(lib, n_groups, grid, n_chunks)
-        consecutive = not (tiles == (np.arange(n_chunks)[:, None] * n_groups + of_blocks).ravel()).all()
-        kinds.add(consecutive)
-        if consecutive:
-            assert per_row > 1 and row_bytes % 128 != 0 and (n_groups % 8 != 0 or n_groups < 48), what
-            for done in range(0, n_tiles, grid):
-                for xcd in range(8):
-                    share = tiles[done:min(done + grid, n_tiles)][xcd::8]
-                    assert (np.diff(share) == 1).all(), what
-    assert kinds == {False, True}
+        taken = np.empty((n_groups, n_chunks), dtype=np.int64)
+        taken[groups, chunks] = np.arange(n_tiles)
+        assert (np.diff(taken, axis=1) > 0).all(), what
+        if row_groups == 1 or row_bytes % 128 == 0 or (n_groups % 8 == 0 and n_groups >= 48):
+            assert (groups.reshape(n_chunks, n_groups) == _tile_groups(lib, n_groups, grid, n_chunks)).all(), what
+            continue
+        rows, xcd = tiles // row_groups, np.arange(n_tiles) % 8
+        whole = n_tiles // row_groups // 8 * 8
+        for row in range(n_tiles // row_groups):
+            of_row = rows == row
+            if row < whole:
+                assert (xcd[of_row] == row % 8).all(), what
+            else:
+                assert all((np.diff(tiles[of_row & (xcd == x)]) == 1).all() for x in range(8)), what
+        by_rows += whole > 0
+    assert by_rows > 50
     one = (ctypes.c_int32 * 1)()
     assert lib.fss_debug_tile_order(1, 1, 1, 128, 1, None, one) != 0
     assert lib.fss_debug_tile_order(0, 1, 1, 128, 1, one, one) != 0
     assert lib.fss_debug_tile_order(1, 1, 1, 128, 0, one, one) != 0
+    assert lib.fss_debug_tile_order(3, 1, 2, 128, 1, one, one) != 0
 
 
 def test_missing_cpp_dispatch_falls_back_to_the_python_wrappers(monkeypatch, tmp_path):
