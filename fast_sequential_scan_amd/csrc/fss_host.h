@@ -446,9 +446,12 @@ inline int make_cm_plan(CmPlan &pl, int64_t rows, int64_t seq, int dtype, int di
   int vec = user ? user->vec : 0, waves = user ? user->waves : 0;
   if (user && (user->max_groups < 0 || user->steps != 0)) return FSS_ERR_BAD_CONFIG;
   // 16 bytes per lane whatever the rows' length and alignment, from the length that fills one lane on
-  // (a configuration that names the vector width keeps to naturally aligned accesses)
+  // (a configuration that names the vector width keeps to naturally aligned accesses).  Below it two
+  // 16-bit steps per lane where rows and tensors allow: bf16 forward (64, 4096, 6) 51.9 us with one, 48.9 with
+  // two, (64, 4096, 4) 50.2 and 49.3.
   const bool any_rows = vec == 0;
-  if (any_rows) vec = ss >= widest ? widest : 1;
+  const bool pairs = esize == 2 && ss % 2 == 0 && align % 4 == 0;
+  if (any_rows) vec = ss >= widest ? widest : pairs ? 2 : 1;
   const bool vec_ok = vec == 1 || vec == widest || (vec == 2 && esize == 2);
   if (!vec_ok) return FSS_ERR_BAD_CONFIG;
   if (!any_rows && ss % vec != 0) return FSS_ERR_BAD_CONFIG;

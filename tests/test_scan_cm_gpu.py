@@ -217,3 +217,25 @@ def test_short_rows_share_vectors(oracle, bs, d, seq, dtype):
     """Rows of at most half a wave's lanes: 1, 2, 4 .. 32 lanes each (and the first length that takes a
     whole wave again), last vectors full and ragged, last tiles full and not."""
     _run(oracle, bs, d, seq, dtype, seed=seq + d)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16], ids=["bf16", "f16"])
+@pytest.mark.parametrize("seq", [2, 3, 4, 6, 7])
+@pytest.mark.parametrize("start", [0, 1, 2])
+def test_rows_shorter_than_a_lane(oracle, seq, start, dtype):
+    """Two steps per lane where rows and tensors allow it (an even length, a start on 4 bytes), otherwise one."""
+    bs, d = 3, 43
+    alpha, beta, dout = _inputs(bs, d, seq, dtype, seed=seq)
+
+    def placed(t):
+        view = torch.full((t.numel() + start,), float("nan"), dtype=dtype, device=DEV)[start:].view(t.shape)
+        view.copy_(t)
+        return view
+
+    a, b, do = placed(alpha), placed(beta), placed(dout)
+    h = ext.scan_forward_cm(a, b)
+    ga, gb = ext.scan_backward_cm(a, placed(h), do)
+    _check(h, oracle.scan_fwd_f32(_t(alpha), _t(beta), fused=True), dtype, "h")
+    ga_or, gb_or = oracle.scan_bwd_f32(_t(alpha), _t(h), _t(dout), fused=True)
+    _check(gb, gb_or, dtype, "grad_beta")
+    _check(ga, ga_or, dtype, "grad_alpha")
