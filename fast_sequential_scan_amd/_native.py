@@ -33,7 +33,7 @@ EXPORTED_SYMBOLS = (
     "fss_workspace_status",
     "fss_workspace_attach_flag",
     "fss_debug_set_spin_limit",
-    "fss_debug_tile_groups", "fss_debug_tile_order",
+    "fss_debug_tile_groups", "fss_debug_tile_order", "fss_debug_cache_variant",
     "fss_debug_noalloc_reinit_after",
     "fss_debug_chain_plan",
     "fss_debug_chain_anchor",
@@ -108,6 +108,7 @@ def _declare(lib: ctypes.CDLL) -> None:
     lib.fss_debug_set_spin_limit.argtypes = [ctypes.c_uint32]
     lib.fss_debug_tile_groups.argtypes = [ctypes.c_int32, ctypes.c_int32, ctypes.c_int32, ctypes.POINTER(ctypes.c_int32)]
     lib.fss_debug_tile_order.argtypes = [ctypes.c_int32] * 3 + [_i64, ctypes.c_int32] + [ctypes.POINTER(ctypes.c_int32)] * 2
+    lib.fss_debug_cache_variant.argtypes = [_i64, _i64, _i64, _int, _int, _sz, _cfgp, _int]
     lib.fss_debug_noalloc_reinit_after.restype = ctypes.c_uint64
     lib.fss_debug_noalloc_reinit_after.argtypes = [ctypes.c_uint64]
     lib.fss_debug_chain_plan.restype = _int

@@ -252,18 +252,7 @@ int run_scan(int dtype, int dir, const void *alpha, const void *in_b, const void
   args.period = chain_period(pl.n_groups, pl.cfg.waves);
   set_divisors(args);
   args.spin_limit = __atomic_load_n(&g_spin_limit, __ATOMIC_RELAXED);
-  const int64_t tensor_bytes = bs * seq * d * static_cast<int64_t>(esize);
-  // (variant 2 exists for the kernels large shapes run - the forward with 32 steps per lane, the
-  // backward with 16 steps and 4 bytes per lane; elsewhere the forward runs as 0, the backward as 1)
-  const bool large = streaming || tensor_bytes > kStreamDoutBytes;
-  if (shares_sectors(d * static_cast<int64_t>(esize)))
-    pl.alt_policy = 3;
-  else if (gated)
-    pl.alt_policy = 0;
-  else if (dir == FSS_FWD)
-    pl.alt_policy = large ? 2 : (tensor_bytes <= kKeepOutBytes ? 1 : 0);
-  else
-    pl.alt_policy = streaming ? 2 : (large ? 1 : 0);
+  pl.alt_policy = cache_variant(pl, bs, seq, d, static_cast<int64_t>(esize), gated, dir, streaming);
   const StateArgs<true> state = {state_in, state_out, h_before};
   args.hdr = static_cast<uint32_t *>(workspace);
   args.words = workspace ? reinterpret_cast<uint64_t *>(static_cast<char *>(workspace) + kHeaderBytes) : nullptr;
@@ -430,6 +419,14 @@ int32_t fss_debug_chain_anchor(int32_t chunk, int32_t period, int32_t stride) {
   if (chunk < 0 || period < 1 || stride < 1) return -1;
   return fss::chain_anchor(chunk, period, fss::fast_div(static_cast<uint32_t>(period)), stride,
                            fss::fast_div(static_cast<uint32_t>(stride)));
+}
+
+int fss_debug_cache_variant(int64_t bs, int64_t seq, int64_t d, int dtype, int dir, size_t align_bytes,
+                            const fss_config *cfg, int policy) {
+  if (policy != FSS_CACHE_AUTO && policy != FSS_CACHE_STREAMING) return -1;
+  fss::Plan pl;
+  if (fss::make_plan(pl, bs, seq, d, dtype, dir, align_bytes ? align_bytes : 16, cfg) != FSS_OK) return -1;
+  return fss::cache_variant(pl, bs, seq, d, dtype != FSS_F32 ? 2 : 4, dir >= FSS_GATED_FWD, dir & 1, policy == FSS_CACHE_STREAMING);
 }
 
 uint32_t fss_debug_set_spin_limit(uint32_t polls) {

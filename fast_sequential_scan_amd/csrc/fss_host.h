@@ -241,7 +241,7 @@ inline void complete_config(fss_config &c, int64_t bs, int64_t seq, int64_t d, i
 
 struct Plan {
   fss_config cfg;
-  int alt_policy = 0;  // plain scan: which cache hints the kernel carries (see kKeepOutBytes, kStreamDoutBytes)
+  int alt_policy = 0;  // cache_variant
   int64_t tiles_per_row, n_ctiles, n_chunks;
   int64_t n_groups;  // column groups per chunk: n_ctiles / cfg.cols
   int64_t n_tiles;   // what the workgroups walk: n_groups * n_chunks
@@ -281,6 +281,20 @@ inline int make_plan(Plan &pl, int64_t bs, int64_t seq, int64_t d, int dtype, in
   if (pl.n_chunks > 1)
     pl.ws_bytes += static_cast<size_t>(pl.n_ctiles * pl.n_chunks) * 3 * 64 * c.vec * sizeof(uint64_t);
   return FSS_OK;
+}
+
+// Which cache hints a launch carries (ALT of scan_kernel).  The instantiations without hints exist for up to two
+// channels per lane, which is what the library chooses; wider ones are only named by a caller and keep
+// to the sizes.
+inline int cache_variant(const Plan &pl, int64_t bs, int64_t seq, int64_t d, int64_t esize, bool gated, int dir, bool streaming) {
+  if (pl.cfg.vec <= 2 && shares_sectors(d * esize)) return 3;
+  if (gated) return 0;
+  // (variant 2 exists for the kernels large shapes run - the forward with 32 steps per lane, the
+  // backward with 16 steps and 4 bytes per lane; elsewhere the forward runs as 0, the backward as 1)
+  const int64_t tensor_bytes = bs * seq * d * esize;
+  const bool large = streaming || tensor_bytes > kStreamDoutBytes;
+  if (dir == FSS_FWD) return large ? 2 : (tensor_bytes <= kKeepOutBytes ? 1 : 0);
+  return streaming ? 2 : (large ? 1 : 0);
 }
 
 inline size_t common_alignment(std::initializer_list<const void *> ptrs) {

@@ -271,10 +271,18 @@ int fss_scan_bwd_f32(const void *alpha, const void *h, const void *dout,
  * in the forward, 16 steps and 4 bytes per lane in the backward); the gated and the channel-major
  * scans carry the same hints under both (outputs and the backward's reads of h streamed,
  * everything else cached).  Rows of (bs, seq, d) tensors that are no multiple of 64 bytes run
- * without any hint under both.  Returns the previous policy, or -1 for an unknown one.
+ * without any hint under both, except in configurations that name 4 or 8 channels per lane.
+ * Returns the previous policy, or -1 for an unknown one.
  */
 enum fss_cache_policy { FSS_CACHE_AUTO = 0, FSS_CACHE_STREAMING = 1 };
 int fss_set_cache_policy(int policy);
+/*
+ * Test hook (host only, no device call): which hints a row-major launch carries under `policy`; -1 for
+ * arguments that do not launch.  Forward: 0 h streamed, 1 nothing, 2 h and beta streamed.  Backward
+ * (h and the gradients streamed): 0 nothing more, 1 dout, 2 dout and alpha.  The gated scan: 0.  3: none.
+ */
+int fss_debug_cache_variant(int64_t bs, int64_t seq, int64_t d, int dtype, int dir, size_t align_bytes,
+                            const fss_config *cfg, int policy);
 
 /*
  * fss_scan_fwd_ex with cfg = NULL for callers that cannot allocate device memory and have

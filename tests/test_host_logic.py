@@ -529,6 +529,36 @@ def test_workgroups_take_every_tile_once_and_after_those_it_waits_for():
     assert lib.fss_debug_tile_order(3, 1, 2, 128, 1, one, one) != 0
 
 
+def test_which_cache_hints_a_launch_carries():
+    """Rows that are no multiple of 64 bytes run without hints, whatever the size and the policy - unless the
+    configuration names 4 or 8 channels per lane: those keep to the sizes, like rows of whole sectors."""
+    lib = _native.lib()
+    auto, streaming = _native.FSS_CACHE_AUTO, _native.FSS_CACHE_STREAMING
+
+    def variant(shape, dtype, direction, cfg=None, policy=auto):
+        config = None if cfg is None else ctypes.byref(_native.FssConfig(*cfg, 0, 0))
+        return lib.fss_debug_cache_variant(*shape, dtype, direction, 16, config, policy)
+
+    fwd, bwd, gfwd, gbwd = (_native.FSS_FWD, _native.FSS_BWD, _native.FSS_GATED_FWD, _native.FSS_GATED_BWD)
+    bf16, f32 = _native.FSS_BF16, _native.FSS_F32
+    small, middle, large = (8, 1024), (8, 3800), (16, 8192)  # of 1000 channels in 16 bits: 16, 61 and 262 MB
+    for d, whole in ((1024, True), (1000, False), (992, True), (1001, False)):
+        for size, f, b in ((small, 1, 0), (middle, 0, 0), (large, 2, 1)):
+            assert variant((*size, d), bf16, fwd) == (f if whole else 3)
+            assert variant((*size, d), bf16, bwd) == (b if whole else 3)
+            assert variant((*size, d), bf16, fwd, None, streaming) == (2 if whole else 3)
+            assert variant((*size, d), bf16, bwd, None, streaming) == (2 if whole else 3)
+            assert variant((*size, d), bf16, gfwd) == variant((*size, d), bf16, gbwd) == (0 if whole else 3)
+            assert (variant((*size, d), f32, fwd) == 3) == (d * 4 % 64 != 0)
+            for cfg in ((4, 8, 4), (8, 8, 4), (4, 16, 4)):
+                if d % cfg[0]:
+                    assert variant((*size, d), bf16, fwd, cfg) == -1
+                    continue
+                assert variant((*size, d), bf16, fwd, cfg) == f and variant((*size, d), bf16, bwd, cfg) == b
+                assert variant((*size, d), bf16, bwd, cfg, streaming) == 2
+    assert variant((8, 1024, 1024), bf16, fwd, None, 7) == -1
+
+
 def test_missing_cpp_dispatch_falls_back_to_the_python_wrappers(monkeypatch, tmp_path):
     """The C++ dispatch only shortens the host's way to the launch: when its module is missing or
     does not load, one warning is given and every call goes through the ctypes wrappers over the
