@@ -449,13 +449,6 @@ std::optional<std::tuple<at::Tensor, at::Tensor>> state_scan(const at::Tensor &a
   return std::make_tuple(outs[0], outs[1]);
 }
 
-// The plain one of them without gradients.
-std::optional<std::tuple<at::Tensor, at::Tensor>> scan_state(const at::Tensor &alpha, const at::Tensor &beta,
-                                                             const std::optional<at::Tensor> &h_before) {
-  if (!alpha.defined() || !beta.defined() || wants_gradient(alpha, beta, h_before)) return std::nullopt;
-  return state_scan(alpha, beta, h_before, false);
-}
-
 }  // namespace
 
 PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
@@ -468,8 +461,6 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("scan", &scan, "h, or None when the call is not the common case");
   m.def("scan_gated", &scan_gated, "h of the gated scan, or None when the call is not the common case");
   m.def("scan_cm", &scan_cm, "h of the channel-major scan, or None when the call is not the common case");
-  m.def("scan_state", &scan_state, py::arg("alpha"), py::arg("beta"), py::arg("h_before") = py::none(),
-        "(h, h_last) without gradients, or None when the call is not the common case");
   m.def("state_scan", &state_scan, py::arg("alpha"), py::arg("beta"), py::arg("h_before"), py::arg("gated"),
         "(h, h_last) of the plain or the gated scan, or None when the call is not the common case");
 }

@@ -212,7 +212,7 @@ def test_decode_loop_through_the_state_dispatch(dtype):
             a, b = alpha[:, lo:hi].contiguous(), beta[:, lo:hi].contiguous()
             want_h, want_state = scan_cuda.SequentialScanState.apply(a, b, state)
             if lo > 0:
-                assert binding.scan_state(a, b, state) is not None, "the C++ dispatch declined a plain call"
+                assert binding.state_scan(a, b, state, False) is not None, "the C++ dispatch declined a plain call"
             h, new_state = scan_with_state(a, b, state)
             assert torch.equal(h, want_h) and torch.equal(new_state, want_state)
             pieces.append(h)
@@ -223,11 +223,10 @@ def test_decode_loop_through_the_state_dispatch(dtype):
     if dtype == torch.float32:
         torch.testing.assert_close(torch.cat(pieces, dim=1), whole, rtol=1e-5, atol=1e-6)
         torch.testing.assert_close(states[-1], whole_state, rtol=1e-5, atol=1e-6)
-    # with gradients the call goes through the Python Function
+    # with gradients the dispatch records its own node
     a = alpha[:, :50].contiguous().requires_grad_(True)
     h, last = scan_with_state(a, beta[:, :50].contiguous())
-    assert h.grad_fn is not None and "ScanNode" not in _node_name(h)
-    assert binding.scan_state(a, beta[:, :50].contiguous(), None) is None
+    assert "StateNode" in _node_name(h) and "StateNode" in _node_name(last)
     # what it declines: a state of the wrong type or shape (the wrappers raise)
     with pytest.raises(RuntimeError):
         scan_with_state(alpha, beta, torch.zeros(bs, d, device=DEV, dtype=torch.float64))
@@ -247,7 +246,7 @@ def test_captured_decode_step_replays_match_eager():
     with torch.cuda.stream(side), torch.no_grad():
         state = torch.zeros(bs, d, device=DEV)
         scan_with_state(alpha, beta, state)  # warm: the stream's workspace, device check, residency query
-        assert binding.scan_state(alpha, beta, state) is not None
+        assert binding.state_scan(alpha, beta, state, False) is not None
         side.synchronize()
         want = []
         s = state.clone()
@@ -363,4 +362,44 @@ def test_tensor_subclasses_in_scans_with_states(gated, grads):
         assert all(torch.equal(g.as_subclass(torch.Tensor), w.as_subclass(torch.Tensor)) for g, w in zip(got, want))
     h, _ = api(alpha, beta, torch.nn.Parameter(plain[2]))
     assert type(h) is torch.Tensor and "StateNode" in _node_name(h)
+    ext.workspace_status()
+
+
+@pytest.mark.parametrize("kind,with_state", [("plain", False), ("gated", False), ("channel_major", False), ("state", False),
+                                             ("state", True), ("gated_state", False), ("gated_state", True)])
+def test_backward_without_a_registered_workspace(kind, with_state):
+    """A backward that finds no workspace for its stream calls the Python wrappers back, which make one: the
+    gradients are those of the wrappers bit for bit, of both outputs and of each alone."""
+    api = {"plain": scan_cu, "gated": scan_gated, "channel_major": scan_cm, "state": scan_with_state,
+           "gated_state": scan_cuda.scan_gated_with_state}[kind]
+    shape = (2, 96, 700) if kind == "channel_major" else (2, 700, 96)  # (chunks that chain)
+    alpha, beta, dout = _tensors(shape, torch.bfloat16, seed=14)
+    before, last_grad = torch.randn(2, 2, 96, device=DEV, generator=torch.Generator(DEV).manual_seed(4))
+    binding = ext.fast_dispatch()
+    for do, dl in ((dout, last_grad), (dout, None), (None, last_grad)):
+        if not kind.endswith("state"):
+            dl = None
+        if do is None and dl is None:
+            continue
+        inputs = [t.clone().requires_grad_(True) for t in ((alpha, beta, before) if with_state else (alpha, beta))]
+        with torch.no_grad():
+            api(*inputs)  # a workspace exists from here on
+        outs = api(*inputs)
+        outs = outs if isinstance(outs, tuple) else (outs,)
+        assert all(("StateNode" if kind.endswith("state") else "ScanNode") in _node_name(o) for o in outs)
+        torch.cuda.synchronize()
+        binding.forget_workspaces()
+        ext._workspaces.clear()
+        used, grads = zip(*((o, g) for o, g in zip(outs, (do, dl)) if g is not None))
+        got = torch.autograd.grad(used, inputs, grads)
+        assert len(ext._workspaces) == 1, "the backward did not go through the wrappers"
+        a, b = alpha, beta
+        h0, do = before if with_state else None, torch.zeros_like(alpha) if do is None else do
+        want = {"plain": lambda: ext.scan_backward_half(a, outs[0], do),
+                "gated": lambda: ext.gated_scan_backward(a, b, outs[0], do),
+                "channel_major": lambda: ext.scan_backward_cm(a, outs[0], do),
+                "state": lambda: ext.scan_backward_state(a, outs[0], do, h0, dl),
+                "gated_state": lambda: ext.gated_scan_backward_state(a, b, outs[0], do, h0, dl)}[kind]()
+        want = [w for w in want if w is not None]
+        assert len(got) == len(want) and all(torch.equal(g, w) for g, w in zip(got, want))
     ext.workspace_status()
