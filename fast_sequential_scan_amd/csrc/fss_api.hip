@@ -556,11 +556,8 @@ int fss_scan_bwd_f32(const void *alpha, const void *h, const void *dout, void *g
 size_t fss_cm_workspace_bytes(int64_t bs, int64_t d, int64_t seq, int dtype, int dir, const fss_config *cfg) {
   fss::CmPlan pl;
   if (bs < 0 || d < 0 || (d > 0 && bs > INT64_MAX / d)) return fss::kHeaderBytes;
-  // alignment unknown here: the narrowest vector gives the most chunks, hence the upper bound
-  size_t best = fss::kHeaderBytes;
-  for (size_t align = 2; align <= 16; align <<= 1)
-    if (fss::make_cm_plan(pl, bs * d, seq, dtype, dir, align, cfg) == FSS_OK && pl.ws_bytes > best) best = pl.ws_bytes;
-  return best;
+  // (the tensors' alignment, unknown here, changes the plan of rows shorter than a lane only: one chunk either way)
+  return fss::make_cm_plan(pl, bs * d, seq, dtype, dir, 16, cfg) == FSS_OK ? pl.ws_bytes : fss::kHeaderBytes;
 }
 
 int fss_scan_fwd_cm(int dtype, const void *alpha, const void *beta, void *h, int64_t bs, int64_t d, int64_t seq,

@@ -20,7 +20,6 @@ namespace fss {
 typedef const FSS_GLOBAL char *gcptr_t;
 typedef FSS_GLOBAL char *gptr_t;
 
-typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 typedef float f32x2 __attribute__((ext_vector_type(2)));
 typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
@@ -404,7 +403,7 @@ struct ScanArgs {
   int32_t n_ctiles;       // bs * tiles_per_row
   int32_t n_chunks;       // ceil(seq / (WAVES*STEPS))
   int32_t n_tiles;        // tiles the workgroups walk: n_groups * n_chunks
-  int32_t n_groups;       // column groups per chunk: n_ctiles / wg_cols
+  int32_t n_groups;       // column groups per chunk: n_ctiles / column tiles per workgroup
   int32_t look_waves;     // waves per column tile that look back in parallel (1..kMaxLookWaves)
   int32_t row_lanes_log2; // channel-major only: lanes that cover a row of at most half a wave's (6: the row has waves to itself)
   int32_t period;         // chunks of one sequence that a full grid works on at once (chain_anchor), >= 1

@@ -479,7 +479,7 @@ __global__ __launch_bounds__(MAXW * 64) void scan_kernel(const ScanArgs p, const
   extern __shared__ float lds[];
   __shared__ uint32_t s_ready[2 * 16];  // per column tile and wave: see announce_map
 
-  // The waves of a workgroup: wg_cols column tiles side by side, each with n_waves waves
+  // The waves of a workgroup: COLS column tiles side by side, each with n_waves waves
   // that take consecutive time slices.  Everything the chain phase touches is per column tile.
   TileCtx c;
   c.lane = threadIdx.x & 63;

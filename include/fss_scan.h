@@ -403,7 +403,7 @@ int fss_gated_scan_bwd_state(int dtype, const void *gate, const void *x, const v
  * elements; left 0, the library takes the widest for any seq and alignment), waves and
  * max_groups are used; steps must be 0.  A workgroup of 8 waves covers
  * 4096 (16-bit) / 2048 (fp32) timesteps, and only longer sequences use the workspace:
- * size it with fss_cm_workspace_bytes (an upper bound over alignments).
+ * size it with fss_cm_workspace_bytes (the same for every alignment).
  */
 size_t fss_cm_workspace_bytes(int64_t bs, int64_t d, int64_t seq, int dtype, int dir,
                               const fss_config *cfg);
