@@ -77,9 +77,9 @@ __device__ __forceinline__ Ptr uniform_ptr(Ptr ptr) {
 // is touched once, so the caches should not keep it in preference to other lines.
 // The types promise no more than 2-byte alignment: gfx950 serves global accesses of 4 to 16 bytes
 // at any address (the compiler emits the same instructions for them), so rows whose length or
-// start is odd need no narrower kernels.  Three streams of 512 MiB, 16 bytes per lane: every
-// stream aligned 4.6 TB/s, every stream 2 bytes off 4.6, 4 or 8 bytes off 4.2, 2-byte accesses
-// instead 4.1-4.6; 4 bytes per lane: 5.4 aligned, 4.0-4.2 at 2 bytes off.
+// start is odd need no narrower kernels.  Two streams of 512 MiB read and one written, 16 bytes per lane: all
+// aligned 5.1 TB/s, all 2 bytes off 4.9, 4 or 8 bytes off 4.7; 4 bytes per lane: 5.8 aligned, 4.6 at 2 bytes
+// off; 2 bytes per lane: 4.4 and 4.1.
 typedef uint32_t io_u32x1 __attribute__((aligned(2)));
 typedef uint32_t io_u32x2 __attribute__((ext_vector_type(2), aligned(2)));
 typedef uint32_t io_u32x4 __attribute__((ext_vector_type(4), aligned(2)));
@@ -365,8 +365,8 @@ __device__ __forceinline__ void report_timeout(uint32_t *hdr) {
 // scalar instructions, where the hardware's way - a vector-unit reciprocal, corrected - is a chain
 // of about thirty that a tile waited for seven times before its first load.  With the launch tag no
 // longer waited for there either (launch_tag) and the arguments not held throughout (fresh_args): bf16
-// (2, 1024, 768) forward 9.1 -> 8.3 us, backward 11.4 -> 10.4; gated (3, 156, 3456) forward 10.5 -> 9.5;
-// (4, 2048, 2048) 22.6 -> 21.9; launches of several rounds gain up to 2 % or nothing.
+// (2, 1024, 768) forward 9.1 -> 8.0 us, backward 11.2 -> 10.5; gated (3, 156, 3456) forward 10.4 -> 9.4;
+// (4, 2048, 2048) 23.0 -> 22.4; launches of several rounds gain up to 2 % or nothing.
 struct FastDiv {
   uint32_t mul;
   uint8_t first, second;  // shifts

@@ -28,8 +28,8 @@ namespace fss {
 // accesses work at any address (DwordIO), and the one lane per row whose vector would reach past
 // the end of the scan loads one that ends there and shifts it.  Kernels with one timestep per
 // lane for such rows (128 bytes per wave and load, chunks of 512 steps instead of 4096) took three
-// times as long: bf16 forward and backward of (8, 1024, 2047) 159 -> 55.5 us (2048: 52), of
-// (8, 1024, 4095) 323 -> 112 us (4096: 98), of (1, 256, 65521) 193 -> 65 us.  What is left between
+// times as long: bf16 forward and backward of (8, 1024, 2047) 158 -> 53.4 us (2048: 48.5), of
+// (8, 1024, 4095) 349 -> 119 us (4096: 107), of (1, 256, 65521) 186 -> 61 us.  What is left between
 // odd and aligned rows is the price of 16-byte accesses at odd addresses; keeping the stores'
 // lines in L2 for the neighbouring wave (no streaming hint) costs another 3-5 %.
 
@@ -47,8 +47,9 @@ struct Flag {
 // SHORT: rows that half a wave's lanes cover.  They lie back to back in memory, so 64/L of them share a
 // vector - L lanes each, a power of two, with the lane scan confined to them - instead of leaving
 // most lanes idle: a wave's load then is as long as other waves' are, and the kernel is bound by memory
-// again.  bf16 (64, 4096, 23) forward 90 -> 11.7 us, backward 122 -> 19.2; (64, 4096, 64) 64 -> 17.0 and 85 ->
-// 28.3 us (5.9 TB/s); (64, 1024, 250) 28.0 -> 17.7 and 38.2 -> 30.1 us; (2, 1024, 256) 6.3 -> 4.2 and 5.6 -> 5.0.
+// again.  bf16, one row to a wave -> shared: (64, 4096, 64) forward 62 -> 16.7 us, backward 84 -> 28.8 (5.8
+// TB/s); (64, 1024, 250) 29.4 -> 17.6 and 40.2 -> 30.7 us; (2, 1024, 256) 6.4 -> 4.4 and 5.7 -> 5.0; (64, 4096,
+// 23), before with one step per lane, 52 -> 11.6 and 63 -> 19.1.
 template <typename E, int VEC, int ROWS, bool BWD, bool RAGGED, bool SHORT>
 __device__ __forceinline__ void cm_tile(const ScanArgs &p, TileCtx &c, int64_t row0, int64_t n_rows) {
   using RowT = Row<E, VEC>;
