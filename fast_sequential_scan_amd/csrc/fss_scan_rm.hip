@@ -529,19 +529,19 @@ __global__ __launch_bounds__(MAXW * 64) void scan_kernel(const ScanArgs p, const
   uint32_t tile_no = 0;
   const uint32_t n_tiles = static_cast<uint32_t>(p.n_tiles);
   for (uint32_t tile = blockIdx.x; tile < n_tiles; tile += gridDim.x, parity ^= 1u) {
-    const ScanArgs &plan = fresh_args();
-    const TilePlace place = tile_place(plan.order, plan.by_groups, n_tiles, tile);
+    const TileDeal deal = tile_deal();
+    const TilePlace place = tile_place(deal.order, deal.by_groups, n_tiles, tile);
     c.tile_no = ++tile_no;
     c.lds_map = lds_maps + (parity * waves_total + c.wcol * c.n_waves) * kLaneSlots;
     // unsigned, wave-uniform arithmetic: stays on the scalar unit
     const uint32_t chunk = place.chunk;
     const uint32_t ctile = place.group * COLS + static_cast<uint32_t>(c.wcol);
-    const uint32_t batch = divide(ctile, plan.by_row);
-    const uint32_t coltile = ctile - batch * static_cast<uint32_t>(plan.tiles_per_row);
+    const uint32_t batch = divide(ctile, deal.by_row);
+    const uint32_t coltile = ctile - batch * deal.tiles_per_row;
     c.chunk = static_cast<int>(chunk);
     c.ctile = static_cast<int>(ctile);
     c.last = c.chunk == p.n_chunks - 1;
-    place_in_chain(plan, c);
+    place_in_chain(fresh_args(), c);
 
     const int64_t col0 = static_cast<int64_t>(coltile) * kLaneSlots;  // first channel of the tile
     c.col_ok = col0 + c.lane * VEC < p.d;
