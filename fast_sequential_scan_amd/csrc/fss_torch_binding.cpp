@@ -420,10 +420,17 @@ bool wants_gradient(const at::Tensor &alpha, const at::Tensor &beta, const std::
 // (h, h_last) of the scan that starts from the fp32 state `h_before` (bs, d) - zeros when absent -,
 // plain or gated, recorded for autograd when an input asks for it: the step of a decode loop, a
 // segment of a chunked prefill or of truncated back-propagation, all of which the host's time decides.
-// None for anything else.  (Through the Python Function a call of the gated scan's decode step takes
+// None for anything else, objects that are no tensors included.  (Through the Python Function a call of the gated scan's decode step takes
 // the host 17 us, here 5; a segment's forward and backward 130 us, here 55.)
-std::optional<std::tuple<at::Tensor, at::Tensor>> state_scan(const at::Tensor &alpha, const at::Tensor &beta,
-                                                             const std::optional<at::Tensor> &h_before, bool gated) {
+std::optional<std::tuple<at::Tensor, at::Tensor>> state_scan(py::handle first, py::handle second, py::handle before,
+                                                             bool gated) {
+  // (this path returns plain tensors; of a subclass's the Functions return the subclass's)
+  if (!THPVariable_CheckExact(first.ptr()) || !THPVariable_CheckExact(second.ptr()) ||
+      !(before.is_none() || THPVariable_CheckExact(before.ptr())))
+    return std::nullopt;
+  const at::Tensor &alpha = THPVariable_Unpack(first.ptr()), &beta = THPVariable_Unpack(second.ptr());
+  std::optional<at::Tensor> h_before;
+  if (!before.is_none()) h_before = THPVariable_Unpack(before.ptr());
   if (!g_state_fwd || !alpha.defined() || is_traced()) return std::nullopt;
   const at::ScalarType t = alpha.scalar_type();
   const int64_t code = code_of(t);

@@ -83,7 +83,6 @@ class SequentialScanSingle(Function):
 _UNRESOLVED = object()
 _fast: Any = _UNRESOLVED
 _fast_gated: Any = _UNRESOLVED
-_fast_state: Any = _UNRESOLVED
 _fast_cm: Any = _UNRESOLVED
 
 
@@ -158,21 +157,14 @@ class SequentialScanState(Function):
         return grad_alpha, grad_beta, grad_h_before
 
 
-# (the dispatch returns plain tensors; of a subclass's tensors the Functions return the subclass's)
-_PLAIN_TYPES = (torch.Tensor, torch.nn.Parameter)
-
-
-def _fast_state_scan(
-    first: torch.Tensor, second: torch.Tensor, h_before: Optional[torch.Tensor], gated: bool
-) -> Optional[Tuple[torch.Tensor, torch.Tensor]]:
+def _resolve_fast_state(*call: Any) -> Optional[Tuple[torch.Tensor, torch.Tensor]]:
     global _fast_state
-    if _fast_state is _UNRESOLVED:
-        binding = _ext.fast_dispatch()
-        _fast_state = binding.state_scan if binding is not None else None
-    if (_fast_state is None or type(first) not in _PLAIN_TYPES or type(second) not in _PLAIN_TYPES
-            or (h_before is not None and type(h_before) not in _PLAIN_TYPES)):
-        return None
-    return _fast_state(first, second, h_before, gated)
+    binding = _ext.fast_dispatch()
+    _fast_state = binding.state_scan if binding is not None else lambda *call: None
+    return _fast_state(*call)
+
+
+_fast_state: Any = _resolve_fast_state  # (itself until the first call)
 
 
 def scan_with_state(
@@ -181,7 +173,7 @@ def scan_with_state(
     """``h[t] = alpha[t]*h[t-1] + beta[t]`` from ``h[-1] = h_before`` (zeros when None; when given,
     ``alpha[:, 0]`` multiplies it).  Returns ``(h, h_last)`` with ``h_last`` the fp32 state after the
     last step, to be passed as ``h_before`` of the next segment."""
-    pair = _fast_state_scan(alpha, beta, h_before, False)
+    pair = _fast_state(alpha, beta, h_before, False)
     return pair if pair is not None else SequentialScanState.apply(alpha, beta, h_before)
 
 
@@ -249,7 +241,7 @@ def scan_gated_with_state(
     """:func:`scan_gated` from ``h[-1] = h_before`` (fp32 ``(bs, d_model)``, zeros when None).  Returns
     ``(h, h_last)`` with ``h_last`` the fp32 state after the last step, to be passed as ``h_before`` of
     the next segment (chunked prefill, decoding, a sequence sharded over devices)."""
-    pair = _fast_state_scan(gate, x, h_before, True)
+    pair = _fast_state(gate, x, h_before, True)
     return pair if pair is not None else SequentialScanGatedState.apply(gate, x, h_before)
 
 
