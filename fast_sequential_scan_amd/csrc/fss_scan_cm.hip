@@ -281,7 +281,7 @@ __global__ __launch_bounds__(1024) void cm_scan_kernel(const ScanArgs p) {
   c.trace_wave = 0;
 #endif
   c.chained = p.n_chunks > 1;
-  c.epoch = c.chained ? ld_u32(p.hdr + HDR_EPOCH) : 0u;
+  c.epoch = c.chained ? read_epoch(p) : 0u;
   c.tag = 0u;
   c.anchor = c.span = 0;
 

@@ -50,9 +50,9 @@
 //   start of the workgroups.  State handed between chunks travels as 64-bit
 //   words {tag, fp32} written and read with relaxed agent-scope atomics; value
 //   and validity arrive together, so no fence is needed.  The tag is a
-//   per-workspace launch counter ("epoch", never 0), so words never need
-//   clearing; workgroups count themselves out at the end (two-level counter) and
-//   the last one advances the epoch for the next launch.  The counter wraps
+//   per-workspace launch number ("epoch", never 0), so words never need
+//   clearing; every workgroup adds its share of one to it at the end (count_out) without
+//   waiting for the answer.  The number wraps
 //   after 2^32-1 launches; a host that can get there re-initialises the
 //   workspace first.  Every wait is bounded: a wave that exhausts its budget
 //   records an error in the workspace header (and in the host-visible word attached
@@ -513,8 +513,8 @@ __global__ __launch_bounds__(MAXW * 64) void scan_kernel(const ScanArgs p, const
   }
 #endif
   c.chained = p.n_chunks > 1;
-  // every workgroup of a launch reads the same value: it only changes when all are done
-  c.epoch = c.chained ? ld_u32(p.hdr + HDR_EPOCH) : 0u;
+  // every workgroup of a launch reads the same value (count_out)
+  c.epoch = c.chained ? read_epoch(p) : 0u;
   c.tag = 0u;
   c.anchor = c.span = 0;
 
