@@ -773,10 +773,11 @@ __device__ __forceinline__ void await_chunk(const ScanArgs &p, const TileCtx &c,
 __device__ __forceinline__ void announce_map(uint32_t *ready, int wave, uint32_t seq) {
   __hip_atomic_store(ready + wave, seq, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_WORKGROUP);
 }
-__device__ __forceinline__ void await_map(const uint32_t *ready, int wave, uint32_t seq) {
-  // (wave-uniform address: one LDS word, broadcast)
-  while (__hip_atomic_load(ready + wave, __ATOMIC_ACQUIRE, __HIP_MEMORY_SCOPE_WORKGROUP) < seq)
-    __builtin_amdgcn_s_sleep(1);
+// How many of the waves w, w+1, ... have left their maps, without a gap (lane l looks at wave l's word).
+__device__ __forceinline__ int arrived_maps(const uint32_t *ready, int lane, int w, int n_waves, uint32_t seq) {
+  const uint32_t r = lane < n_waves ? __hip_atomic_load(ready + lane, __ATOMIC_ACQUIRE, __HIP_MEMORY_SCOPE_WORKGROUP) : 0u;
+  const uint64_t missing = __builtin_amdgcn_ballot_w64(r < seq) >> w;  // (tile numbers start at 1: the bit of wave n_waves is set)
+  return __builtin_ctzll(missing);
 }
 // every wave of the column tile has left its map (lane l looks at wave l's word)
 __device__ __forceinline__ void await_all_maps(const uint32_t *ready, int lane, int n_waves, uint32_t seq) {
@@ -794,6 +795,38 @@ __device__ __forceinline__ void await_all_maps(const uint32_t *ready, int lane, 
 // composition of maps 0 .. w-1, in place of map w, which nobody else reads), and (A, B) the
 // chunk's map.  Every other wave then finds its prefix with one LDS read behind the next barrier.
 // The order of the composition is the waves' order, whatever the order of their arrival.
+// One look at all the waves' words says how many maps may be read, and those are read kFoldBatch at a
+// time: with a look and a read per map, each a round trip to the LDS that the next one waits for, the
+// chunk's map went out 0.1 us later for every wave of the workgroup.  bf16 gated forward (1, 7243, 64) 9.7 -> 8.8 us,
+// (2, 1024, 768) 7.6 -> 7.0; forward (8, 1819, 64) 8.5 -> 8.1, (1, 65521, 256) 23.3 -> 22.8; fp32 forward (2, 777,
+// 328) 9.4 -> 8.7; large launches up to 1 %.  Two at a time with two channels and more per lane: four cost the
+// gated kernel with 16 steps the 81st register and a third of its resident workgroups ((16, 2048, 512) in
+// that configuration 20.9 -> 23.4 us).
+template <int VEC>
+constexpr int kFoldBatch = VEC == 1 ? 4 : 2;
+template <int N>
+struct Count {
+  static constexpr int value = N;
+};
+template <int VEC>
+__device__ __forceinline__ void fold_maps(float2 *slot, int n, int lane, float *A, float *B) {
+  float2 m[kFoldBatch<VEC>][VEC];
+#pragma unroll
+  for (int i = 0; i < kFoldBatch<VEC>; ++i)
+#pragma unroll
+    for (int v = 0; v < VEC; ++v)
+      if (i < n) m[i][v] = slot[(i * VEC + v) * 64 + lane];
+#pragma unroll
+  for (int i = 0; i < kFoldBatch<VEC>; ++i)
+    if (i < n) {
+#pragma unroll
+      for (int v = 0; v < VEC; ++v) {
+        slot[(i * VEC + v) * 64 + lane] = make_float2(A[v], B[v]);
+        B[v] = fma0(m[i][v].x, B[v], m[i][v].y);
+        A[v] *= m[i][v].x;
+      }
+    }
+}
 template <int VEC>
 __device__ __forceinline__ void fold_arriving_maps(float2 *lds_map, const uint32_t *ready, uint32_t seq, int lane,
                                                    int count, float *A, float *B) {
@@ -802,17 +835,16 @@ __device__ __forceinline__ void fold_arriving_maps(float2 *lds_map, const uint32
     A[v] = 1.0f;
     B[v] = 0.0f;
   }
-  for (int w = 0; w < count; ++w) {
-    if (w > 0) await_map(ready, w, seq);  // (slot 0 is this wave's own)
-    float2 m[VEC];
-#pragma unroll
-    for (int v = 0; v < VEC; ++v) m[v] = lds_map[(w * VEC + v) * 64 + lane];
-#pragma unroll
-    for (int v = 0; v < VEC; ++v) {
-      lds_map[(w * VEC + v) * 64 + lane] = make_float2(A[v], B[v]);
-      B[v] = fma0(m[v].x, B[v], m[v].y);
-      A[v] *= m[v].x;
+  int w = 0;
+  while (w < count) {
+    const int here = arrived_maps(ready, lane, w, count, seq);
+    if (here == 0) {
+      __builtin_amdgcn_s_sleep(1);
+      continue;
     }
+    const int stop = w + here;
+    for (; w + kFoldBatch<VEC> <= stop; w += kFoldBatch<VEC>) fold_maps<VEC>(lds_map + w * VEC * 64, kFoldBatch<VEC>, lane, A, B);
+    for (; w < stop; ++w) fold_maps<VEC>(lds_map + w * VEC * 64, 1, lane, A, B);
   }
 }
 
@@ -834,7 +866,9 @@ __device__ __forceinline__ void fold_arriving_maps(float2 *lds_map, const uint32
 // `mid` (only with HAS_MID) is called once by every wave, by the look-back waves right after their
 // first fetch has been issued: loads it issues travel while the chain is resolved and
 // return after the fetch (loads return in issue order).
-template <int VEC, bool HAS_MID, typename Mid>
+//
+// `LOOKS`: how many of the look-back's results a wave reads from LDS at a time (fold_maps).
+template <int VEC, bool HAS_MID, int LOOKS, typename Mid>
 __device__ __forceinline__ void chain_chunks(const ScanArgs &p, const TileCtx &c, const float *mA,
                                              const float *mB, const float *seq_in, float *state, Mid &&mid) {
   constexpr int kLaneSlots = 64 * VEC;
@@ -850,6 +884,7 @@ __device__ __forceinline__ void chain_chunks(const ScanArgs &p, const TileCtx &c
   if (wave == 0) {
     // the chunk's own map, needed by later chunks: out as early as possible - and on the way
     // every wave's prefix, left where its map was (the waves read it behind the next barrier)
+    __builtin_amdgcn_s_setprio(3);  // (the other waves of the SIMD may have arithmetic left; every later chunk waits for this)
     fold_arriving_maps<VEC>(c.lds_map, c.s_ready, c.tile_no, lane, c.n_waves, cA, cB);
     if (c.chained && !c.last) {
       mine = p.words + (static_cast<size_t>(c.chunk) * p.n_ctiles + c.ctile) * 3 * kLaneSlots + lane;
@@ -866,6 +901,7 @@ __device__ __forceinline__ void chain_chunks(const ScanArgs &p, const TileCtx &c
           st_word(mine + (2 * VEC + v) * 64, c.tag, seq_in ? fma0(cA[v], seq_in[v], cB[v]) : cB[v]);
       }
     }
+    __builtin_amdgcn_s_setprio(0);
   }
   FSS_STAMP(c, p, 3);
 
@@ -953,14 +989,26 @@ __device__ __forceinline__ void chain_chunks(const ScanArgs &p, const TileCtx &c
   __syncthreads();
   // every wave folds what the look-back waves found (the same few LDS reads in each wave
   // cost less than a second barrier and a broadcast by wave 0)
-  for (int w = 0; w < c.look && c.chunk - 1 - w * c.span >= anchor; ++w) {
+  const auto looked = [&](int w) { return w < c.look && c.chunk - 1 - w * c.span >= anchor; };
+  const auto fold_looks = [&](const float2 *slot, auto batch) {
+    constexpr int n = decltype(batch)::value;
+    float2 m[n][VEC];
 #pragma unroll
-    for (int v = 0; v < VEC; ++v) {
-      const float2 m = c.lds_pred[(w * VEC + v) * 64 + lane];
-      accB[v] = fma0(accA[v], m.y, accB[v]);
-      accA[v] *= m.x;
-    }
-  }
+    for (int i = 0; i < n; ++i)
+#pragma unroll
+      for (int v = 0; v < VEC; ++v) m[i][v] = slot[(i * VEC + v) * 64 + lane];
+#pragma unroll
+    for (int i = 0; i < n; ++i)
+#pragma unroll
+      for (int v = 0; v < VEC; ++v) {
+        accB[v] = fma0(accA[v], m[i][v].y, accB[v]);
+        accA[v] *= m[i][v].x;
+      }
+  };
+  int w = 0;
+  if constexpr (LOOKS > 1)
+    for (; looked(w + LOOKS - 1); w += LOOKS) fold_looks(c.lds_pred + w * VEC * 64, Count<LOOKS>());
+  for (; looked(w); ++w) fold_looks(c.lds_pred + w * VEC * 64, Count<1>());
   // (the last group folded ended with the anchor's state, the map x -> 0*x + s: accB is the state)
 #pragma unroll
   for (int v = 0; v < VEC; ++v) hin[v] = accB[v];
