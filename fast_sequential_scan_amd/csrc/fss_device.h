@@ -773,6 +773,21 @@ __device__ __forceinline__ void await_chunk(const ScanArgs &p, const TileCtx &c,
 __device__ __forceinline__ void announce_map(uint32_t *ready, int wave, uint32_t seq) {
   __hip_atomic_store(ready + wave, seq, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_WORKGROUP);
 }
+// N consecutive waves have left their maps (wave-uniform addresses: N LDS words, broadcast)
+template <int N>
+__device__ __forceinline__ void await_maps(const uint32_t *ready, uint32_t seq) {
+  for (;;) {
+    uint32_t r[N];
+    bool all = true;
+#pragma unroll
+    for (int i = 0; i < N; ++i) r[i] = __hip_atomic_load(ready + i, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+#pragma unroll
+    for (int i = 0; i < N; ++i) all = all && r[i] >= seq;
+    if (all) break;
+    __builtin_amdgcn_s_sleep(1);
+  }
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+}
 // How many of the waves w, w+1, ... have left their maps, without a gap (lane l looks at wave l's word).
 __device__ __forceinline__ int arrived_maps(const uint32_t *ready, int lane, int w, int n_waves, uint32_t seq) {
   const uint32_t r = lane < n_waves ? __hip_atomic_load(ready + lane, __ATOMIC_ACQUIRE, __HIP_MEMORY_SCOPE_WORKGROUP) : 0u;
@@ -802,22 +817,37 @@ __device__ __forceinline__ void await_all_maps(const uint32_t *ready, int lane, 
 // 328) 9.4 -> 8.7; large launches up to 1 %.  Two at a time with two channels and more per lane: four cost the
 // gated kernel with 16 steps the 81st register and a third of its resident workgroups ((16, 2048, 512) in
 // that configuration 20.9 -> 23.4 us).
+// Looking at a wave's word and then reading its map, for one wave after the other, are two round trips to
+// the LDS that the next map waits for: 0.1 us later for every wave of the workgroup.  With one
+// channel per lane one look covers all the waves and the maps that have arrived are read four at a time;
+// with more, whose tiles wait longer for their rows (and whose arithmetic, in the gated kernels, fills
+// the SIMD that the looking wave shares), the maps are awaited and read in pairs.  bf16 gated forward (1, 7243,
+// 64) 9.7 -> 8.8 us, (2, 1024, 768) 7.6 -> 7.0; forward (8, 1819, 64) 8.5 -> 8.1; fp32 forward (2, 777, 328) 9.4 ->
+// 8.7; with two channels (8, 4096, 1024) 44.2 -> 43.6, (1, 65521, 256) 23.4 -> 22.9.  The other way round:
+// awaited in fours with one channel 9.2, 7.2, 8.2 and 9.1 us; one look with two channels (16, 2048, 512) gated, 16
+// steps and 8 waves, 20.9 -> 21.7; four maps at a time there 23.4 (the 81st register, a third of the
+// resident workgroups).
 template <int VEC>
 constexpr int kFoldBatch = VEC == 1 ? 4 : 2;
 template <int N>
 struct Count {
   static constexpr int value = N;
 };
-template <int VEC>
+// Folds the maps of the `n` waves whose slots begin at `slot` (n <= N, uniform).
+template <int VEC, int N>
 __device__ __forceinline__ void fold_maps(float2 *slot, int n, int lane, float *A, float *B) {
-  float2 m[kFoldBatch<VEC>][VEC];
+  float2 m[N][VEC];
 #pragma unroll
-  for (int i = 0; i < kFoldBatch<VEC>; ++i)
+  for (int i = 0; i < N; ++i)
 #pragma unroll
     for (int v = 0; v < VEC; ++v)
-      if (i < n) m[i][v] = slot[(i * VEC + v) * 64 + lane];
+      if (VEC == 1) {
+        if (i < n) m[i][v] = slot[(i * VEC + v) * 64 + lane];
+      } else {
+        m[i][v] = slot[((i < n ? i : 0) * VEC + v) * 64 + lane];
+      }
 #pragma unroll
-  for (int i = 0; i < kFoldBatch<VEC>; ++i)
+  for (int i = 0; i < N; ++i)
     if (i < n) {
 #pragma unroll
       for (int v = 0; v < VEC; ++v) {
@@ -830,12 +860,20 @@ __device__ __forceinline__ void fold_maps(float2 *slot, int n, int lane, float *
 template <int VEC>
 __device__ __forceinline__ void fold_arriving_maps(float2 *lds_map, const uint32_t *ready, uint32_t seq, int lane,
                                                    int count, float *A, float *B) {
+  constexpr int N = kFoldBatch<VEC>;
 #pragma unroll
   for (int v = 0; v < VEC; ++v) {
     A[v] = 1.0f;
     B[v] = 0.0f;
   }
   int w = 0;
+  if constexpr (VEC > 1) {
+    for (; w < count; w += N) {
+      await_maps<N>(ready + w, seq);  // (the words of waves that do not exist are set from the start)
+      fold_maps<VEC, N>(lds_map + w * VEC * 64, count - w, lane, A, B);
+    }
+    return;
+  }
   while (w < count) {
     const int here = arrived_maps(ready, lane, w, count, seq);
     if (here == 0) {
@@ -843,8 +881,8 @@ __device__ __forceinline__ void fold_arriving_maps(float2 *lds_map, const uint32
       continue;
     }
     const int stop = w + here;
-    for (; w + kFoldBatch<VEC> <= stop; w += kFoldBatch<VEC>) fold_maps<VEC>(lds_map + w * VEC * 64, kFoldBatch<VEC>, lane, A, B);
-    for (; w < stop; ++w) fold_maps<VEC>(lds_map + w * VEC * 64, 1, lane, A, B);
+    for (; w + N <= stop; w += N) fold_maps<VEC, N>(lds_map + w * VEC * 64, N, lane, A, B);
+    for (; w < stop; ++w) fold_maps<VEC, N>(lds_map + w * VEC * 64, 1, lane, A, B);
   }
 }
 

@@ -271,7 +271,7 @@ __global__ __launch_bounds__(1024) void cm_scan_kernel(const ScanArgs p) {
   c.lds_pred = lds_maps + 2 * c.n_waves * 64;
   c.seq = p.seq;
   c.s_ready = s_ready;
-  if (threadIdx.x < 16) s_ready[threadIdx.x] = 0u;
+  if (threadIdx.x < 16) s_ready[threadIdx.x] = threadIdx.x < static_cast<uint32_t>(c.n_waves) ? 0u : ~0u;
   __syncthreads();
   c.row_bytes = 0;
   c.lane_off = 0;

@@ -500,7 +500,7 @@ __global__ __launch_bounds__(MAXW * 64) void scan_kernel(const ScanArgs p, const
   c.seq = p.seq;
   c.row_bytes = p.d * E::kBytes;
   c.s_ready = s_ready + c.wcol * 16;
-  if (threadIdx.x < 2 * 16) s_ready[threadIdx.x] = 0u;
+  if (threadIdx.x < 2 * 16) s_ready[threadIdx.x] = (threadIdx.x & 15) < static_cast<uint32_t>(c.n_waves) ? 0u : ~0u;
   __syncthreads();
 #ifdef FSS_TRACE
   c.trace_wave = FSS_TRACE_WAVE < 0 ? c.n_waves - 1 : FSS_TRACE_WAVE;
