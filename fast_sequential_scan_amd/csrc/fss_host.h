@@ -129,6 +129,48 @@ inline int choose_cols(const fss_config &c, int64_t bs, int64_t seq, int64_t d, 
   return tiles > kCus && tiles <= 2 * kCus ? 2 : 1;
 }
 
+// What a launch of a forward kernel takes, in ns, as a function of its tiling: a launch and a tile's
+// serial work (more of it the more steps a wave takes one after the other, in the gated kernels their
+// arithmetic), the chain (a round trip to memory, and more maps to find the more chunks of a
+// sequence are in flight at once), every round of the resident workgroups after the first, and the
+// bytes: what the busiest compute unit moves, and all of them together, padding included.  Fitted to 4600
+// pairs of a shape of 2^17 to 2^25 elements (bs 1..64, seq 16..65536, d 64..4096, a quarter of the
+// widths odd or ragged) and a configuration, each weighted by how near it came to the shape's fastest.
+struct ForwardCost {
+  double launch, step, channel_step, chain, depth, round, unit_bytes, all_bytes;
+};
+constexpr ForwardCost kForwardCost[2][2] = {  // [16 bits, 32 bits][plain, gated]
+    {{3315, 55, -15, 772, 564, 2166, 11.47e-3, 17.98e-3}, {3230, 170, -54, 935, 545, 2786, 20.11e-3, 16.54e-3}},
+    {{2870, 11, 2, 847, 621, 3097, 8.80e-3, 18.24e-3}, {3203, 15, 15, 511, 493, 2282, 8.51e-3, 23.92e-3}}};
+inline double forward_ns(const ForwardCost &m, int64_t bs, int64_t seq, int64_t d, int esize, int vec, int steps, int waves) {
+  const int64_t columns = bs * ceil_div(d, 64 * static_cast<int64_t>(vec));
+  const int64_t chunks = ceil_div(seq, static_cast<int64_t>(steps) * waves), tiles = columns * chunks;
+  // (registers: six waves of up to 16 steps on a SIMD, four of 32)
+  const int64_t resident = kCus * ((steps <= 16 ? 6 : 4) / ((waves + 3) / 4));
+  const int64_t in_flight = ceil_div(resident, columns) < chunks ? ceil_div(resident, columns) : chunks;
+  const double tile_bytes = 3.0 * 64 * vec * steps * waves * esize;
+  return m.launch + m.step * steps + m.channel_step * vec * steps + (chunks > 1 ? m.chain : 0) +
+         m.depth * __builtin_sqrt(static_cast<double>(in_flight - 1)) + m.round * static_cast<double>(ceil_div(tiles, resident) - 1) +
+         tile_bytes * (m.unit_bytes * static_cast<double>(ceil_div(tiles, kCus)) + m.all_bytes / kCus * static_cast<double>(tiles));
+}
+
+// Forwards of fewer elements than this take the tiling that forward_ns finds fastest, if it is clearly faster
+// than the ladder's (complete_config): the ladder was drawn from launches that fill the device, and
+// below them "the largest tile that leaves one per compute unit" is the wrong question.  Against the
+// fastest of 15 to 25 configurations, bf16 forwards below 2^21 elements lost 16 % with the ladder and lose 3 %,
+// gated ones 18 and 3 %; from 2^21 to 2^24 (gated 2^23) 9 and 3 %, 16 and 4 %; fp32 below 2^21 12 and 3 %, gated below
+// 2^22 12 and 5 %.  The margin keeps out what the estimate cannot tell apart: without it one launch in ten
+// from 2^21 elements on became slower, with it one in fifty.  Ladder -> estimate, shapes
+// that the fit had not seen: bf16 gated forward (1, 1021, 1610) 12.7 -> 8.8 us, (10, 1098, 384) 14.7 -> 10.8, (2, 29970, 64)
+// 16.8 -> 12.4; fp32 (26, 82, 64) 5.3 -> 3.9; 175 of them 10 % in the mean, one in fifty slower (by 2 to 5 %).
+// Larger launches stay with the ladder, which is within 2-4 % of the fastest there.
+constexpr int64_t forward_model_elems(bool narrow, bool gated) {
+  return narrow ? (gated ? int64_t{1} << 23 : int64_t{15} << 20) : int64_t{1} << (gated ? 22 : 21);
+}
+// Chaining words a tiling chosen that way may need (smaller tiles need more than the ladder's): far below what
+// any caller's scratch is limited to.
+constexpr int64_t kModelWordBytes = int64_t{4} << 20;
+
 // Fills the zero fields of `c`.  `align` is the common alignment in bytes of all
 // tensors of the call.
 //
@@ -233,6 +275,26 @@ inline void complete_config(fss_config &c, int64_t bs, int64_t seq, int64_t d, i
     const int64_t rounds = ceil_div(tiles, kCus);
     if (rounds >= 2 && tiles * 10 < rounds * kCus * 9) pick.waves = 8;
   }
+  if (fwd && !c.vec && !c.steps && !c.waves && !c.cols && seq > 64 && elems < forward_model_elems(narrow, gated)) {
+    const ForwardCost &model = kForwardCost[narrow ? 0 : 1][gated ? 1 : 0];
+    double best = forward_ns(model, bs, seq, d, esize, pick.vec, pick.steps, pick.waves) /
+                  (elems < (int64_t{1} << 21) ? 1.04 : 1.08);
+    constexpr Rung shapes[] = {{0, 32, 16, 0}, {0, 32, 8, 0}, {0, 16, 16, 0}, {0, 16, 12, 0}, {0, 16, 8, 0}, {0, 8, 16, 0}, {0, 8, 8, 0}};
+    for (int v = can2 ? 2 : 1; v >= 1; --v)
+      for (const Rung &r : shapes) {
+        int s = r.steps, w = r.waves;
+        if (v * s > max_vec_steps(dtype) || (gated && !narrow && v > 1)) continue;
+        while (w > 1 && static_cast<int64_t>(s) * (w / 2) >= seq) w /= 2;
+        while (s > 8 && s / 2 >= seq) s /= 2;
+        const int64_t columns = bs * ceil_div(d, 64 * static_cast<int64_t>(v)), chunks = ceil_div(seq, static_cast<int64_t>(s) * w);
+        if (columns * chunks * v * (3 * 64 * static_cast<int64_t>(sizeof(uint64_t))) > kModelWordBytes) continue;
+        const double ns = forward_ns(model, bs, seq, d, esize, v, s, w);
+        if (ns < best) {
+          best = ns;
+          pick = fss_config{v, s, w, 0, 0};
+        }
+      }
+  }
   c.vec = pick.vec;
   c.steps = pick.steps;
   c.waves = pick.waves;
@@ -248,7 +310,7 @@ struct Plan {
   size_t ws_bytes;
 };
 
-inline int make_plan(Plan &pl, int64_t bs, int64_t seq, int64_t d, int dtype, int dir, size_t align,
+inline int compute_plan(Plan &pl, int64_t bs, int64_t seq, int64_t d, int dtype, int dir, size_t align,
               const fss_config *user) {
   if (bs < 0 || seq < 0 || d < 0) return FSS_ERR_BAD_SHAPE;
   if (dtype != FSS_BF16 && dtype != FSS_F32 && dtype != FSS_F16) return FSS_ERR_BAD_CONFIG;
@@ -281,6 +343,39 @@ inline int make_plan(Plan &pl, int64_t bs, int64_t seq, int64_t d, int dtype, in
   if (pl.n_chunks > 1)
     pl.ws_bytes += static_cast<size_t>(pl.n_ctiles * pl.n_chunks) * 3 * 64 * c.vec * sizeof(uint64_t);
   return FSS_OK;
+}
+
+// The same, with the plans of the shapes a thread launched last kept: what is planned is a function of these
+// arguments alone, and weighing a dozen tilings takes the host 0.5 us of a launch of a few.
+inline int make_plan(Plan &pl, int64_t bs, int64_t seq, int64_t d, int dtype, int dir, size_t align,
+                     const fss_config *user) {
+  if (user) return compute_plan(pl, bs, seq, d, dtype, dir, align, user);
+  struct Kept {
+    int64_t bs = -1, seq = 0, d = 0;
+    int dtype = 0, dir = 0;
+    size_t align = 0;
+    Plan plan;
+  };
+  constexpr uint32_t kKept = 16;
+  static thread_local Kept kept[kKept];
+  const uint64_t mix = (static_cast<uint64_t>(bs) * 0x9e3779b97f4a7c15ull ^ static_cast<uint64_t>(seq)) * 0xff51afd7ed558ccdull ^
+                       (static_cast<uint64_t>(d) * 8 + static_cast<uint64_t>(dtype * 4 + dir)) * 0xc4ceb9fe1a85ec53ull ^ align << 40;
+  Kept &k = kept[(mix >> 43) % kKept];
+  if (k.bs == bs && k.seq == seq && k.d == d && k.dtype == dtype && k.dir == dir && k.align == align && bs >= 0) {
+    pl = k.plan;
+    return FSS_OK;
+  }
+  const int rc = compute_plan(pl, bs, seq, d, dtype, dir, align, nullptr);
+  if (rc == FSS_OK) {
+    k.bs = bs;
+    k.seq = seq;
+    k.d = d;
+    k.dtype = dtype;
+    k.dir = dir;
+    k.align = align;
+    k.plan = pl;
+  }
+  return rc;
 }
 
 // Which cache hints a launch carries (ALT of scan_kernel).  The instantiations without hints exist for up to two

@@ -1,0 +1,61 @@
+"""Host-side checks of how small forwards are tiled (the cost estimate in csrc/fss_host.h)."""
+import ctypes
+import threading
+
+import numpy as np
+
+from fast_sequential_scan_amd import _native
+
+LIMIT = 4 << 20  # bytes of chaining words an estimate may ask for beyond the ladder's
+
+
+def choose(lib, shape, dtype, direction, align=16):
+    cfg = _native.FssConfig()
+    assert lib.fss_choose_config(*shape, dtype, direction, align, ctypes.byref(cfg)) == 0
+    return cfg.vec, cfg.steps, cfg.waves, cfg.cols
+
+
+def test_chaining_words_stay_far_below_the_scratch_limits():
+    """A tiling chosen by the estimate needs at most 4 MiB of words, or no more than the ladder's last rung
+    (32 or 16 steps, 8 waves): what fitted a caller's scratch still does."""
+    lib = _native.lib()
+    rng = np.random.default_rng(5)
+    for _ in range(3000):
+        d = int(rng.choice([1, 2, 3, 7, 63, 64, 65, 127, 200, 512, 1024]))
+        bs = int(rng.choice([1, 2, 5, 64, 300]))
+        seq = int(np.exp(rng.uniform(np.log(65), np.log(2e7 / (bs * d) + 66))))
+        dtype, direction = int(rng.integers(0, 3)), int(rng.choice([_native.FSS_FWD, _native.FSS_GATED_FWD]))
+        steps = 32 if direction == _native.FSS_FWD else 16
+        last_rung = _native.FssConfig(1, steps if seq > steps // 2 else 16, 8, 0)
+        need = lib.fss_workspace_bytes(bs, seq, d, dtype, direction, None)
+        ladder = lib.fss_workspace_bytes(bs, seq, d, dtype, direction, ctypes.byref(last_rung))
+        # (rows of an odd number of 64-channel tiles are padded to two channels per lane: up to 4/3 of the words and more)
+        assert need <= max(LIMIT + 4096, 2 * ladder), (bs, seq, d, dtype, direction)
+
+
+def test_plans_do_not_depend_on_what_was_planned_before():
+    """The plans a thread keeps are those it would compute: the same answers in another order and from another thread."""
+    lib = _native.lib()
+    rng = np.random.default_rng(6)
+    asked = [((int(rng.integers(1, 40)), int(rng.integers(1, 3000)), int(rng.integers(1, 700))), int(rng.integers(0, 3)),
+              int(rng.integers(0, 4)), int(rng.choice([4, 8, 16]))) for _ in range(300)]
+    first = [choose(lib, *a) for a in asked]
+    order = rng.permutation(len(asked))
+    again = {int(i): choose(lib, *asked[i]) for i in list(order) + list(order[::-1])}
+    assert [again[i] for i in range(len(asked))] == first
+    other = []
+    t = threading.Thread(target=lambda: other.extend(choose(lib, *a) for a in asked))
+    t.start()
+    t.join()
+    assert other == first
+
+
+def test_small_and_large_forwards():
+    lib = _native.lib()
+    # a launch that leaves most of the device idle takes short tiles, the device's ladder begins where launches fill it
+    assert choose(lib, (1, 697, 448), _native.FSS_BF16, _native.FSS_FWD)[1] == 8
+    assert choose(lib, (10, 1871, 256), _native.FSS_BF16, _native.FSS_GATED_FWD) == (2, 16, 12, 1)
+    assert choose(lib, (8, 2048, 1024), _native.FSS_BF16, _native.FSS_FWD) == (2, 32, 16, 1)
+    # never two channels per lane where rows or tensors do not allow them
+    assert choose(lib, (3, 614, 1007), _native.FSS_BF16, _native.FSS_FWD)[0] == 1
+    assert choose(lib, (10, 1871, 256), _native.FSS_BF16, _native.FSS_GATED_FWD, 2)[0] == 1
