@@ -205,6 +205,12 @@ inline void complete_config(fss_config &c, int64_t bs, int64_t seq, int64_t d, i
   const bool fwd = dir == FSS_FWD;
   if (!gated && fwd) {
     if (narrow) rung(2, 32, 16);
+    // (one channel per lane, where two do not go, and sequences of a few 32-step tiles: (24, 384, 1735) 23.2 -> 19.2 us,
+    // (29, 574, 1319) 44.4 -> 33.6, (28, 748, 445) 15.8 -> 13.7); their words, twice to four times as many, well within
+    // the scratch of the entry point that allocates nothing
+    const int64_t short_tiles = bs * ceil_div(d, 64) * ceil_div(seq, 128);
+    if (narrow && !can2 && seq <= 1024 && short_tiles * 3 * 64 * static_cast<int64_t>(sizeof(uint64_t)) <= FSS_NOALLOC_SCRATCH_BYTES / 2)
+      rung(1, 16, 8);
     if (wide32_fwd) rung(2, 16, 16);
     else if (big32 && seq <= 4096) rung(1, 16, 16);
     rung(1, 32, 16);
@@ -213,6 +219,9 @@ inline void complete_config(fss_config &c, int64_t bs, int64_t seq, int64_t d, i
   } else if (!gated) {
     // 32-step slices would cost the backward a dozen spilled registers per lane
     if (narrow) {
+      // (one channel per lane, where two do not go, in very large launches: (7, 4958, 3767) 8 waves 370 us, 16 waves
+      // 300; (4, 8354, 1531) 142 and 122; of 2^24 elements, (31, 607, 1041), 45 and 53)
+      if (!can2 && elems >= (static_cast<int64_t>(1) << 25)) rung(1, 16, 16);
       rung(2, 16, 16);
       if (seq >= 16384) rung(1, 16, 16); else rung(2, 16, 8);
       if (seq > 256) rung(1, 16, 8); else rung(2, 8, 8);
@@ -225,8 +234,28 @@ inline void complete_config(fss_config &c, int64_t bs, int64_t seq, int64_t d, i
   } else if (fwd) {
     // The gated kernels spend as much time on arithmetic as on memory and like more, smaller
     // waves; a sequence that 8 waves cover wants two workgroups per CU before it takes them.
-    if (narrow) {
-      // (from 8192 steps two 8-wave workgroups per CU are 3-5 % faster than one of 16 waves: 8 shapes of 9)
+    const bool filled = elems >= forward_model_elems(narrow, gated);  // (below: where the estimate starts from)
+    if (narrow && filled && !can2) {
+      // one channel per lane (odd widths, or rows that two would pad too far): three workgroups of 16 steps and 8 waves
+      // on a compute unit, whatever the length.  Before, with the 32 steps or 16 waves that larger tiles would be: (18,
+      // 7063, 287) 110 -> 84 us, (2, 5429, 2063) 59 -> 45, (23, 1901, 985) 111 -> 93, (2, 45563, 655) 140 -> 135; 30 shapes of
+      // 2^23 to 2^26 elements 15 % in the mean, two slower ((11, 7957, 369) 94 -> 104)
+      rung(1, 16, 8, 0);
+    } else if (narrow && filled) {
+      // the largest tile where there is just one for every compute unit: (4, 2048, 2048) one launch behind the other
+      // 23.0 us, 16 steps and 8 waves 27.2 (from 8192 steps two 8-wave workgroups are 3-5 % faster than one of 16: 8 shapes of 9)
+      const int64_t big = bs * ceil_div(d, 128) * ceil_div(seq, 512);
+      if (seq > 256 && seq < 8192 && big <= kCus && big * 50 >= kCus * 49) rung(2, 32, 16, 0);
+      // the same as with one channel per lane, for sequences of few chunks ((9, 1695, 1792) 42.6 -> 37.5 us against 32 steps and
+      // 16 waves, (34, 1201, 776) 64.9 -> 55.6, (26, 859, 1548) 61 -> 51); half as long where that pads the sequence by a
+      // tenth less ((29, 299, 1680) 34.4 -> 20.7)
+      if (seq <= 2048) rung(2, 16, ceil_div(seq, 64) * 64 * 10 <= ceil_div(seq, 128) * 128 * 9 ? 4 : 8);
+      // (longer chains want longer chunks, (8, 3000, 1024) 16 steps 35.2 us, 32 steps 29.9, where three quarters of the device's
+      // 8-wave workgroups have a tile; one channel per lane never: (1, 8379, 1740) 47.7 us, two channels 23.7)
+      if (seq > 2048 && seq < 8192) rung(2, 32, 16);
+      if (seq > 2048) rung(2, 32, 8, kCus * 3 / 2);
+      rung(2, 16, 8, 0);
+    } else if (narrow) {
       if (seq >= 8192) rung(2, 32, 8, 2 * kCus);
       if (seq > 256) rung(2, 32, 16); else rung(2, 32, 8, 2 * kCus);
       if (seq >= 4096) rung(1, 32, 16); else rung(2, 16, 16);
@@ -234,6 +263,10 @@ inline void complete_config(fss_config &c, int64_t bs, int64_t seq, int64_t d, i
       rung(1, 16, 16);
       if (seq >= 1024) rung(1, 16, 8, 0); else rung(1, 16, 16, 0);
     } else {
+      // fp32: the largest tile where its rounds are whole ((8, 4096, 1024) 32 steps and 16 waves 83 us, 16 steps 86),
+      // elsewhere 16 steps and 12 waves ((10, 24028, 128) 87 -> 78, (11, 1623, 1152) 62 -> 51, (9, 7795, 67) 33 -> 24)
+      const int64_t big = bs * ceil_div(d, 64) * ceil_div(seq, 512), of_round = ceil_div(big, kCus) * kCus;
+      if (filled && (big * 50 < of_round * 49 || seq * 50 < ceil_div(seq, 512) * 512 * 49)) rung(1, 16, 12, 0);
       if (seq > 256) rung(1, 32, 16); else rung(1, 32, 8, 2 * kCus);
       rung(1, 16, 16, 0);
     }

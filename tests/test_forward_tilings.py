@@ -16,8 +16,8 @@ def choose(lib, shape, dtype, direction, align=16):
 
 
 def test_chaining_words_stay_far_below_the_scratch_limits():
-    """A tiling chosen by the estimate needs at most 4 MiB of words, or no more than the ladder's last rung
-    (32 or 16 steps, 8 waves): what fitted a caller's scratch still does."""
+    """A tiling chosen by the estimate needs at most 4 MiB of words, or no more than the finest that launches that
+    fill the device take (16 steps; 4 waves up to 2048 steps, 8 beyond): what fitted a caller's scratch still does."""
     lib = _native.lib()
     rng = np.random.default_rng(5)
     for _ in range(3000):
@@ -25,12 +25,24 @@ def test_chaining_words_stay_far_below_the_scratch_limits():
         bs = int(rng.choice([1, 2, 5, 64, 300]))
         seq = int(np.exp(rng.uniform(np.log(65), np.log(2e7 / (bs * d) + 66))))
         dtype, direction = int(rng.integers(0, 3)), int(rng.choice([_native.FSS_FWD, _native.FSS_GATED_FWD]))
-        steps = 32 if direction == _native.FSS_FWD else 16
-        last_rung = _native.FssConfig(1, steps if seq > steps // 2 else 16, 8, 0)
+        finest = _native.FssConfig(1, 16, 4 if seq <= 2048 else 8, 0)
         need = lib.fss_workspace_bytes(bs, seq, d, dtype, direction, None)
-        ladder = lib.fss_workspace_bytes(bs, seq, d, dtype, direction, ctypes.byref(last_rung))
-        # (rows of an odd number of 64-channel tiles are padded to two channels per lane: up to 4/3 of the words and more)
-        assert need <= max(LIMIT + 4096, 2 * ladder), (bs, seq, d, dtype, direction)
+        bound = lib.fss_workspace_bytes(bs, seq, d, dtype, direction, ctypes.byref(finest))
+        # (rows of an odd number of 64-channel tiles are padded to two channels per lane)
+        assert need <= max(LIMIT + 4096, 2 * bound), (bs, seq, d, dtype, direction)
+
+
+def test_no_plain_forward_outgrows_the_static_scratch():
+    """Short odd-width forwards take tiles that need more words than the ladder's other rungs only while those stay within
+    half of the static array: around the array's size the words are those of 32 steps."""
+    lib = _native.lib()
+    for seq in (512, 700, 1000, 1024):
+        for d in (1, 63, 65, 999):
+            for bs in (1, 100, 1000, 1365, 1366, 5000, 6000, 20000):
+                need = lib.fss_workspace_bytes(bs, seq, d, _native.FSS_BF16, _native.FSS_FWD, None) - 4096
+                widest = max(lib.fss_workspace_bytes(bs, seq, d, _native.FSS_BF16, _native.FSS_FWD,
+                                                     ctypes.byref(_native.FssConfig(1, 32, w, 0))) - 4096 for w in (8, 16))
+                assert need <= max(8 << 20, widest), (bs, seq, d)
 
 
 def test_plans_do_not_depend_on_what_was_planned_before():

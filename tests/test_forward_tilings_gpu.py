@@ -47,15 +47,21 @@ def test_forward_is_the_model_bit_for_bit(oracle, dtype, shape):
     assert torch.equal(h, got) and torch.equal(last.to(dtype), got[:, -1])
 
 
-@pytest.mark.parametrize("shape", [(2, 65, 130), (3, 614, 1006), (10, 1871, 256), (10, 1727, 256), (10, 1920, 252), (7, 300, 513)])
-def test_gated_forward_matches_oracle(oracle, shape):
+# the last six: the tilings of launches that fill the device, short and odd and long
+@pytest.mark.parametrize("shape,dtype", [
+    ((2, 65, 130), torch.bfloat16), ((3, 614, 1006), torch.bfloat16), ((10, 1871, 256), torch.bfloat16), ((10, 1727, 256), torch.bfloat16),
+    ((10, 1920, 252), torch.bfloat16), ((7, 300, 513), torch.bfloat16),
+    ((29, 299, 1000), torch.bfloat16), ((33, 512, 512), torch.bfloat16), ((9, 1800, 519), torch.bfloat16), ((1, 16400, 520), torch.bfloat16),
+    ((2, 2500, 1700), torch.bfloat16), ((3, 1500, 1000), torch.float32)])
+def test_gated_forward_matches_oracle(oracle, shape, dtype):
     g = torch.Generator().manual_seed(sum(shape))
-    gate = (1.5 * torch.randn(shape, generator=g)).to(torch.bfloat16)
-    x = torch.randn(shape, generator=g).to(torch.bfloat16)
+    gate = (1.5 * torch.randn(shape, generator=g)).to(dtype)
+    x = torch.randn(shape, generator=g).to(dtype)
     got = ext.gated_scan_forward(gate.to(DEV), x.to(DEV)).float().cpu().numpy()
     ext.workspace_status()
+    rounding, rtol, atol = ("bf16", 1e-2, 1e-2) if dtype == torch.bfloat16 else ("f32", 1e-4, 1e-5)  # (the bars of tests/test_scan_gated_gpu.py)
     g32, x32 = gate.float().numpy(), x.float().numpy()
-    # (the bar of the bf16 scans, from either rounding of an alpha that lies on the edge of one)
-    ok = oracle.within_rounding_envelope(got, oracle.gated_scan_fwd(g32, x32, "bf16"), oracle.gated_scan_fwd(g32, x32, "bf16", True),
-                                         1e-2, 1e-2)
+    # (from either rounding of an alpha that lies on the edge of one)
+    ok = oracle.within_rounding_envelope(got, oracle.gated_scan_fwd(g32, x32, rounding), oracle.gated_scan_fwd(g32, x32, rounding, True),
+                                         rtol, atol)
     assert ok.all(), (~ok).sum()
