@@ -199,11 +199,17 @@ inline void complete_config(fss_config &c, int64_t bs, int64_t seq, int64_t d, i
   const bool big32 = !narrow && !gated && d >= 512 && elems >= (static_cast<int64_t>(1) << 26);
   const bool wide32_fwd = big32 && can2 && seq <= 512;
   const bool wide32_bwd = big32 && can2 && elems >= (static_cast<int64_t>(1) << 27);
+  // Rows of three 64-channel tiles, in large launches: with two channels per lane a quarter of the lanes idles.
+  // One launch behind the other, backward (6, 40000, 192) 106 -> 92 us, (30, 2000, 192) 29.3 -> 27.7; ten of eleven shapes 2 to
+  // 13 % faster, (8, 40000, 192) 120 -> 123.  Forward, 8 waves, (4, 57534, 192) 71 -> 61, (2, 60000, 192) 42 -> 35, (64, 4000, 192)
+  // 66 -> 63; six of seven faster, (8, 40000, 192) 81 -> 84; below 2^24 elements nothing.
+  const bool three_tiles = narrow && !gated && d == 3 * 64;
   Rung ladder[8];
   int n = 0;
   auto rung = [&](int v, int s, int w, int64_t need = kCus) { ladder[n++] = Rung{v, s, w, need}; };
   const bool fwd = dir == FSS_FWD;
   if (!gated && fwd) {
+    if (three_tiles && elems >= (int64_t{1} << 24) && elems <= (int64_t{1} << 27)) rung(1, 32, 8);
     if (narrow) rung(2, 32, 16);
     // (one channel per lane, where two do not go, and sequences of a few 32-step tiles: (24, 384, 1735) 23.2 -> 19.2 us,
     // (29, 574, 1319) 44.4 -> 33.6, (28, 748, 445) 15.8 -> 13.7); their words, twice to four times as many, well within
@@ -222,6 +228,12 @@ inline void complete_config(fss_config &c, int64_t bs, int64_t seq, int64_t d, i
       // (one channel per lane, where two do not go, in very large launches: (7, 4958, 3767) 8 waves 370 us, 16 waves
       // 300; (4, 8354, 1531) 142 and 122; of 2^24 elements, (31, 607, 1041), 45 and 53)
       if (!can2 && elems >= (static_cast<int64_t>(1) << 25)) rung(1, 16, 16);
+      if (three_tiles && elems >= (static_cast<int64_t>(1) << 23)) rung(1, 16, 16);
+      // (rows that share sectors, in very large launches: with 12 waves what is in flight leaves the L2 room to put the seams
+      // between column tiles together.  One launch behind the other, (27, 8422, 210) 140 -> 111 us, (9, 20000, 194) 108 -> 92,
+      // (26, 3001, 526) 110 -> 100, (64, 500, 1234) 93.6 -> 91.0; 32 shapes 4 % in the mean, the slowest (54, 608, 2168) 161 ->
+      // 167; (8, 16359, 232), of 30 million elements, 73.6 -> 77.3)
+      if (can2 && shares_sectors(d * esize) && elems >= (static_cast<int64_t>(1) << 25)) rung(2, 16, 12);
       rung(2, 16, 16);
       if (seq >= 16384) rung(1, 16, 16); else rung(2, 16, 8);
       if (seq > 256) rung(1, 16, 8); else rung(2, 8, 8);
