@@ -826,7 +826,8 @@ __device__ __forceinline__ void await_all_maps(const uint32_t *ready, int lane, 
 // 8.7; with two channels (8, 4096, 1024) 44.2 -> 43.6, (1, 65521, 256) 23.4 -> 22.9.  The other way round:
 // awaited in fours with one channel 9.2, 7.2, 8.2 and 9.1 us; one look with two channels (16, 2048, 512) gated, 16
 // steps and 8 waves, 20.9 -> 21.7; four maps at a time there 23.4 (the 81st register, a third of the
-// resident workgroups).
+// resident workgroups).  The channel-major kernels, a row's map to a lane, await theirs in fours: forward (8, 1024, 2047) 20.8 us,
+// with one look 21.9 (though chained ragged rows gain by the look: (13, 768, 4859) 71.3 -> 67.3).
 template <int VEC>
 constexpr int kFoldBatch = VEC == 1 ? 4 : 2;
 template <int N>
@@ -857,7 +858,7 @@ __device__ __forceinline__ void fold_maps(float2 *slot, int n, int lane, float *
       }
     }
 }
-template <int VEC>
+template <int VEC, bool AWAIT>
 __device__ __forceinline__ void fold_arriving_maps(float2 *lds_map, const uint32_t *ready, uint32_t seq, int lane,
                                                    int count, float *A, float *B) {
   constexpr int N = kFoldBatch<VEC>;
@@ -867,7 +868,7 @@ __device__ __forceinline__ void fold_arriving_maps(float2 *lds_map, const uint32
     B[v] = 0.0f;
   }
   int w = 0;
-  if constexpr (VEC > 1) {
+  if constexpr (AWAIT) {
     for (; w < count; w += N) {
       await_maps<N>(ready + w, seq);  // (the words of waves that do not exist are set from the start)
       fold_maps<VEC, N>(lds_map + w * VEC * 64, count - w, lane, A, B);
@@ -905,8 +906,9 @@ __device__ __forceinline__ void fold_arriving_maps(float2 *lds_map, const uint32
 // first fetch has been issued: loads it issues travel while the chain is resolved and
 // return after the fetch (loads return in issue order).
 //
-// `LOOKS`: how many of the look-back's results a wave reads from LDS at a time (fold_maps).
-template <int VEC, bool HAS_MID, int LOOKS, typename Mid>
+// `LOOKS`: how many of the look-back's results a wave reads from LDS at a time (fold_maps).  `AWAIT`: whether
+// the waves' maps are awaited in batches, not looked at all together (fold_arriving_maps).
+template <int VEC, bool HAS_MID, int LOOKS, bool AWAIT, typename Mid>
 __device__ __forceinline__ void chain_chunks(const ScanArgs &p, const TileCtx &c, const float *mA,
                                              const float *mB, const float *seq_in, float *state, Mid &&mid) {
   constexpr int kLaneSlots = 64 * VEC;
@@ -923,7 +925,7 @@ __device__ __forceinline__ void chain_chunks(const ScanArgs &p, const TileCtx &c
     // the chunk's own map, needed by later chunks: out as early as possible - and on the way
     // every wave's prefix, left where its map was (the waves read it behind the next barrier)
     __builtin_amdgcn_s_setprio(3);  // (the other waves of the SIMD may have arithmetic left; every later chunk waits for this)
-    fold_arriving_maps<VEC>(c.lds_map, c.s_ready, c.tile_no, lane, c.n_waves, cA, cB);
+    fold_arriving_maps<VEC, AWAIT>(c.lds_map, c.s_ready, c.tile_no, lane, c.n_waves, cA, cB);
     if (c.chained && !c.last) {
       mine = p.words + (static_cast<size_t>(c.chunk) * p.n_ctiles + c.ctile) * 3 * kLaneSlots + lane;
       if (look_back) {

@@ -205,7 +205,7 @@ __device__ __forceinline__ void cm_tile(const ScanArgs &p, TileCtx &c, int64_t r
   float slice_in = 0.0f;
   if (!SHORT && (c.chained || c.n_waves > 1)) {
     c.tag = launch_tag(c);
-    chain_chunks<1, BWD, kFoldBatch<1>>(p, c, &mA, &mB, nullptr, &slice_in, load_h);
+    chain_chunks<1, BWD, kFoldBatch<1>, true>(p, c, &mA, &mB, nullptr, &slice_in, load_h);
   } else {
     load_h();
   }

@@ -201,7 +201,7 @@ __device__ __forceinline__ void scan_tile(const ScanArgs &p, const StateArgs<STA
     }
     FSS_STAMP(c, p, 1);
     c.tag = launch_tag(c);
-    chain_chunks<VEC, BWD, kFoldBatch<VEC>>(p, c, mA, mB, STATE ? seq_in : nullptr, state, load_h_early);
+    chain_chunks<VEC, BWD, kFoldBatch<VEC>, (VEC > 1)>(p, c, mA, mB, STATE ? seq_in : nullptr, state, load_h_early);
   }
 
   // ---- phase 3: the recurrence from the true incoming state, in order ---------------
@@ -397,7 +397,7 @@ __device__ __forceinline__ void gated_tile(const ScanArgs &p, const StateArgs<ST
   } else {
     c.tag = launch_tag(c);
     // (with two channels per lane the look-back's results one at a time: two cost (16, 2048, 512) 22.1 -> 22.5 us)
-    chain_chunks<VEC, false, VEC == 1 ? kFoldBatch<VEC> : 1>(p, c, mA, mB, STATE ? seq_in : nullptr, state, [] {});
+    chain_chunks<VEC, false, VEC == 1 ? kFoldBatch<VEC> : 1, (VEC > 1)>(p, c, mA, mB, STATE ? seq_in : nullptr, state, [] {});
   }
 
   // ---- phase 3 -------------------------------------------------------------------------
