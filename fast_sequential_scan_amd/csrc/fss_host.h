@@ -201,15 +201,16 @@ inline void complete_config(fss_config &c, int64_t bs, int64_t seq, int64_t d, i
   const bool wide32_bwd = big32 && can2 && elems >= (static_cast<int64_t>(1) << 27);
   // Rows of three 64-channel tiles, in large launches: with two channels per lane a quarter of the lanes idles.
   // One launch behind the other, backward (6, 40000, 192) 106 -> 92 us, (30, 2000, 192) 29.3 -> 27.7; ten of eleven shapes 2 to
-  // 13 % faster, (8, 40000, 192) 120 -> 123.  Forward, 8 waves, (4, 57534, 192) 71 -> 61, (2, 60000, 192) 42 -> 35, (64, 4000, 192)
-  // 66 -> 63; six of seven faster, (8, 40000, 192) 81 -> 84; below 2^24 elements nothing.
+  // 13 % faster, (8, 40000, 192) 120 -> 123.  Forward, 8 waves, (4, 57534, 192) 71 -> 61, (2, 60000, 192) 42 -> 35, (7, 30000,
+  // 192) 61.8 -> 55.5, up to 45 Mi elements; from there (5, 50000, 192) 63.3 -> 65.2, (8, 40000, 192) 80.6 -> 84.1,
+  // (16, 16000, 192) 65.4 -> 63.9; below 2^24 elements nothing.
   const bool three_tiles = narrow && !gated && d == 3 * 64;
   Rung ladder[8];
   int n = 0;
   auto rung = [&](int v, int s, int w, int64_t need = kCus) { ladder[n++] = Rung{v, s, w, need}; };
   const bool fwd = dir == FSS_FWD;
   if (!gated && fwd) {
-    if (three_tiles && elems >= (int64_t{1} << 24) && elems <= (int64_t{1} << 27)) rung(1, 32, 8);
+    if (three_tiles && elems >= (int64_t{1} << 24) && elems < (int64_t{45} << 20)) rung(1, 32, 8);
     if (narrow) rung(2, 32, 16);
     // (one channel per lane, where two do not go, and sequences of a few 32-step tiles: (24, 384, 1735) 23.2 -> 19.2 us,
     // (29, 574, 1319) 44.4 -> 33.6, (28, 748, 445) 15.8 -> 13.7); their words, twice to four times as many, well within
@@ -248,11 +249,14 @@ inline void complete_config(fss_config &c, int64_t bs, int64_t seq, int64_t d, i
     // waves; a sequence that 8 waves cover wants two workgroups per CU before it takes them.
     const bool filled = elems >= forward_model_elems(narrow, gated);  // (below: where the estimate starts from)
     if (narrow && filled && !can2) {
-      // one channel per lane (odd widths, or rows that two would pad too far): three workgroups of 16 steps and 8 waves
-      // on a compute unit, whatever the length.  Before, with the 32 steps or 16 waves that larger tiles would be: (18,
-      // 7063, 287) 110 -> 84 us, (2, 5429, 2063) 59 -> 45, (23, 1901, 985) 111 -> 93, (2, 45563, 655) 140 -> 135; 30 shapes of
-      // 2^23 to 2^26 elements 15 % in the mean, two slower ((11, 7957, 369) 94 -> 104)
-      rung(1, 16, 8, 0);
+      // one channel per lane (odd widths, or rows that two would pad too far): 16 steps and 12 waves, two workgroups on a
+      // compute unit, whatever the length, or 8 waves and three, where 12 pad the sequence by a tenth more.  One launch behind
+      // the other, 32 steps and 16 waves / 16 steps and 8 / 16 steps and 12: (11, 7957, 369) 96.6, 106.6 and 77.1 us; (13, 6000,
+      // 749) 154.7, 197.8, 127.0; (5, 25000, 383) 143.1, 165.7, 112.5; (18, 7063, 287) 112, 86.6, 85.8; (23, 1901, 985) 121,
+      // 98.1, 92.4.  8 waves lose most where the column tiles are a multiple of three, as the launch's 768 workgroups are; of 34
+      // shapes 12 are 10 % faster than 8 in the mean, the slowest (83, 1166, 405) 97.5 -> 104.8.
+      const bool twelve = ceil_div(seq, 192) * 192 * 10 <= ceil_div(seq, 128) * 128 * 11;
+      rung(1, 16, twelve ? 12 : 8, 0);
     } else if (narrow && filled) {
       // the largest tile where there is just one for every compute unit: (4, 2048, 2048) one launch behind the other
       // 23.0 us, 16 steps and 8 waves 27.2 (from 8192 steps two 8-wave workgroups are 3-5 % faster than one of 16: 8 shapes of 9)
