@@ -190,6 +190,10 @@ inline void complete_config(fss_config &c, int64_t bs, int64_t seq, int64_t d, i
   // two channels per lane: even d, 2-element alignment, and never pad a row to twice its width
   const bool can2 = d % 2 == 0 && align % (2 * static_cast<size_t>(esize)) == 0 &&
                     ceil_div(d, 128) * 128 < 2 * ceil_div(d, 64) * 64;
+  // The rungs marked `open`, and the estimate at the end, choose a tiling as a whole: with numbers of waves or of tiles per
+  // row that a caller's two column tiles do not divide, or lanes that a caller's steps do not fit.  Where the caller
+  // names any part of the tiling, the ladder is the one without them.
+  const bool open = !c.vec && !c.steps && !c.waves && !c.cols;
   // fp32, very large tensors with wide rows (56 shapes of 2^24..2^27 elements, d 512..4096, seq
   // 512..8192, six configurations each).  Forward from 2^26 elements: 16 steps per lane are 2-6 %
   // faster than 32 up to seq 4096, and 8 bytes per lane another 3-8 % at seq 512 (4-9 % slower
@@ -204,7 +208,7 @@ inline void complete_config(fss_config &c, int64_t bs, int64_t seq, int64_t d, i
   // 13 % faster, (8, 40000, 192) 120 -> 123.  Forward, 8 waves, (4, 57534, 192) 71 -> 61, (2, 60000, 192) 42 -> 35, (7, 30000,
   // 192) 61.8 -> 55.5, up to 45 Mi elements; from there (5, 50000, 192) 63.3 -> 65.2, (8, 40000, 192) 80.6 -> 84.1,
   // (16, 16000, 192) 65.4 -> 63.9; below 2^24 elements nothing.
-  const bool three_tiles = narrow && !gated && d == 3 * 64;
+  const bool three_tiles = open && narrow && !gated && d == 3 * 64;
   Rung ladder[8];
   int n = 0;
   auto rung = [&](int v, int s, int w, int64_t need = kCus) { ladder[n++] = Rung{v, s, w, need}; };
@@ -216,7 +220,7 @@ inline void complete_config(fss_config &c, int64_t bs, int64_t seq, int64_t d, i
     // (29, 574, 1319) 44.4 -> 33.6, (28, 748, 445) 15.8 -> 13.7); their words, twice to four times as many, well within
     // the scratch of the entry point that allocates nothing
     const int64_t short_tiles = bs * ceil_div(d, 64) * ceil_div(seq, 128);
-    if (narrow && !can2 && seq <= 1024 && short_tiles * 3 * 64 * static_cast<int64_t>(sizeof(uint64_t)) <= FSS_NOALLOC_SCRATCH_BYTES / 2)
+    if (open && narrow && !can2 && seq <= 1024 && short_tiles * 3 * 64 * static_cast<int64_t>(sizeof(uint64_t)) <= FSS_NOALLOC_SCRATCH_BYTES / 2)
       rung(1, 16, 8);
     if (wide32_fwd) rung(2, 16, 16);
     else if (big32 && seq <= 4096) rung(1, 16, 16);
@@ -228,13 +232,13 @@ inline void complete_config(fss_config &c, int64_t bs, int64_t seq, int64_t d, i
     if (narrow) {
       // (one channel per lane, where two do not go, in very large launches: (7, 4958, 3767) 8 waves 370 us, 16 waves
       // 300; (4, 8354, 1531) 142 and 122; of 2^24 elements, (31, 607, 1041), 45 and 53)
-      if (!can2 && elems >= (static_cast<int64_t>(1) << 25)) rung(1, 16, 16);
+      if (open && !can2 && elems >= (static_cast<int64_t>(1) << 25)) rung(1, 16, 16);
       if (three_tiles && elems >= (static_cast<int64_t>(1) << 23)) rung(1, 16, 16);
       // (rows that share sectors, in very large launches: with 12 waves what is in flight leaves the L2 room to put the seams
       // between column tiles together.  One launch behind the other, (27, 8422, 210) 140 -> 111 us, (9, 20000, 194) 108 -> 92,
       // (26, 3001, 526) 110 -> 100, (64, 500, 1234) 93.6 -> 91.0; 32 shapes 4 % in the mean, the slowest (54, 608, 2168) 161 ->
       // 167; (8, 16359, 232), of 30 million elements, 73.6 -> 77.3)
-      if (can2 && shares_sectors(d * esize) && elems >= (static_cast<int64_t>(1) << 25)) rung(2, 16, 12);
+      if (open && can2 && shares_sectors(d * esize) && elems >= (static_cast<int64_t>(1) << 25)) rung(2, 16, 12);
       rung(2, 16, 16);
       if (seq >= 16384) rung(1, 16, 16); else rung(2, 16, 8);
       if (seq > 256) rung(1, 16, 8); else rung(2, 8, 8);
@@ -247,7 +251,7 @@ inline void complete_config(fss_config &c, int64_t bs, int64_t seq, int64_t d, i
   } else if (fwd) {
     // The gated kernels spend as much time on arithmetic as on memory and like more, smaller
     // waves; a sequence that 8 waves cover wants two workgroups per CU before it takes them.
-    const bool filled = elems >= forward_model_elems(narrow, gated);  // (below: where the estimate starts from)
+    const bool filled = open && elems >= forward_model_elems(narrow, gated);  // (below: where the estimate starts from)
     if (narrow && filled && !can2) {
       // one channel per lane (odd widths, or rows that two would pad too far): 16 steps and 12 waves, two workgroups on a
       // compute unit, whatever the length, or 8 waves and three, where 12 pad the sequence by a tenth more.  One launch behind
@@ -324,7 +328,7 @@ inline void complete_config(fss_config &c, int64_t bs, int64_t seq, int64_t d, i
     const int64_t rounds = ceil_div(tiles, kCus);
     if (rounds >= 2 && tiles * 10 < rounds * kCus * 9) pick.waves = 8;
   }
-  if (fwd && !c.vec && !c.steps && !c.waves && !c.cols && seq > 64 && elems < forward_model_elems(narrow, gated)) {
+  if (fwd && open && seq > 64 && elems < forward_model_elems(narrow, gated)) {
     const ForwardCost &model = kForwardCost[narrow ? 0 : 1][gated ? 1 : 0];
     double best = forward_ns(model, bs, seq, d, esize, pick.vec, pick.steps, pick.waves) /
                   (elems < (int64_t{1} << 21) ? 1.04 : 1.08);

@@ -71,3 +71,21 @@ def test_small_and_large_forwards():
     # never two channels per lane where rows or tensors do not allow them
     assert choose(lib, (3, 614, 1007), _native.FSS_BF16, _native.FSS_FWD)[0] == 1
     assert choose(lib, (10, 1871, 256), _native.FSS_BF16, _native.FSS_GATED_FWD, 2)[0] == 1
+
+
+def test_named_parts_of_a_tiling_keep_their_ladder():
+    """A caller who names two column tiles (or steps, or waves) and leaves the rest open gets a tiling that these divide,
+    at the shapes where the library's own choice has three tiles per row, twelve waves or wider lanes."""
+    lib = _native.lib()
+    bf16, fp16, fp32 = _native.FSS_BF16, _native.FSS_F16, _native.FSS_F32
+    fwd, bwd, gfwd = _native.FSS_FWD, _native.FSS_BWD, _native.FSS_GATED_FWD
+    for shape, dtype, direction, named, want in [
+            ((4, 20000, 192), bf16, bwd, (0, 0, 0, 2), (2, 16, 16, 2)), ((31, 3327, 192), bf16, fwd, (0, 0, 0, 2), (2, 32, 8, 2)),
+            ((34, 5677, 192), bf16, bwd, (0, 32, 0, 2), (2, 32, 8, 2)), ((64, 40, 13200), bf16, bwd, (0, 0, 0, 2), (2, 16, 4, 2)),
+            ((256, 38, 3500), fp16, bwd, (0, 0, 0, 2), (2, 16, 4, 2)), ((126, 107, 13200), bf16, bwd, (8, 8, 0, 2), (8, 8, 4, 2)),
+            ((3, 7752, 384), fp16, gfwd, (0, 0, 0, 2), (1, 32, 8, 2)), ((40, 751, 384), bf16, gfwd, (0, 32, 0, 2), (1, 32, 16, 2)),
+            ((4000, 40, 128), fp32, gfwd, (0, 0, 0, 2), (1, 32, 2, 2)), ((7, 4958, 3711), bf16, bwd, (0, 0, 0, 1), (1, 16, 8, 1))]:
+        cfg = _native.FssConfig(named[0], named[1], named[2], 0, named[3])
+        out = (ctypes.c_int32 * 8)()
+        assert lib.fss_debug_chain_plan(*shape, dtype, direction, 16, ctypes.byref(cfg), out) == 0, (shape, named)
+        assert (out[6], out[2], out[1] * out[7], out[7]) == want, (shape, named, list(out))
