@@ -37,6 +37,7 @@ EXPORTED_SYMBOLS = (
     "fss_debug_noalloc_reinit_after",
     "fss_debug_chain_plan",
     "fss_debug_chain_anchor",
+    "fss_debug_plans_computed",
     "fss_scan_fwd_noalloc",
     "fss_choose_config",
     "fss_scan_fwd_bf16",
@@ -113,6 +114,8 @@ def _declare(lib: ctypes.CDLL) -> None:
     lib.fss_debug_noalloc_reinit_after.argtypes = [ctypes.c_uint64]
     lib.fss_debug_chain_plan.restype = _int
     lib.fss_debug_chain_plan.argtypes = [_i64, _i64, _i64, _int, _int, _sz, _cfgp, ctypes.POINTER(ctypes.c_int32)]
+    lib.fss_debug_plans_computed.restype = ctypes.c_uint64
+    lib.fss_debug_plans_computed.argtypes = []
     lib.fss_debug_chain_anchor.restype = ctypes.c_int32
     lib.fss_debug_chain_anchor.argtypes = [ctypes.c_int32, ctypes.c_int32, ctypes.c_int32]
     lib.fss_scan_fwd_noalloc.restype = _int

@@ -6,6 +6,7 @@
 namespace fss {
 
 thread_local int tls_hip_error = 0;
+thread_local uint64_t tls_plans_computed = 0;
 #ifdef FSS_TRACE
 uint64_t *g_trace = nullptr;
 #endif
@@ -414,6 +415,8 @@ int fss_debug_chain_plan(int64_t bs, int64_t seq, int64_t d, int dtype, int dir,
   out[7] = pl.cfg.cols;
   return FSS_OK;
 }
+
+uint64_t fss_debug_plans_computed(void) { return fss::tls_plans_computed; }
 
 int32_t fss_debug_chain_anchor(int32_t chunk, int32_t period, int32_t stride) {
   if (chunk < 0 || period < 1 || stride < 1) return -1;

@@ -15,6 +15,7 @@
 namespace fss {
 
 extern thread_local int tls_hip_error;  // hipError_t of this thread's last failed HIP call
+extern thread_local uint64_t tls_plans_computed;  // fss_debug_plans_computed
 extern uint32_t g_spin_limit;           // polls before a look-back gives up (a test may lower it)
 #ifdef FSS_TRACE
 extern uint64_t *g_trace;
@@ -399,7 +400,8 @@ inline int compute_plan(Plan &pl, int64_t bs, int64_t seq, int64_t d, int dtype,
 }
 
 // The same, with the plans of the shapes a thread launched last kept: what is planned is a function of these
-// arguments alone, and weighing a dozen tilings takes the host 0.5 us of a launch of a few.
+// arguments alone, and weighing a dozen tilings takes the host 0.5 us of a launch of a few.  The alignment shifts the
+// slot, so that the plans for 2 to 16 bytes, which fss_workspace_bytes asks for in turn, never replace each other.
 inline int make_plan(Plan &pl, int64_t bs, int64_t seq, int64_t d, int dtype, int dir, size_t align,
                      const fss_config *user) {
   if (user) return compute_plan(pl, bs, seq, d, dtype, dir, align, user);
@@ -412,13 +414,14 @@ inline int make_plan(Plan &pl, int64_t bs, int64_t seq, int64_t d, int dtype, in
   constexpr uint32_t kKept = 16;
   static thread_local Kept kept[kKept];
   const uint64_t mix = (static_cast<uint64_t>(bs) * 0x9e3779b97f4a7c15ull ^ static_cast<uint64_t>(seq)) * 0xff51afd7ed558ccdull ^
-                       (static_cast<uint64_t>(d) * 8 + static_cast<uint64_t>(dtype * 4 + dir)) * 0xc4ceb9fe1a85ec53ull ^ align << 40;
-  Kept &k = kept[(mix >> 43) % kKept];
+                       (static_cast<uint64_t>(d) * 8 + static_cast<uint64_t>(dtype * 4 + dir)) * 0xc4ceb9fe1a85ec53ull;
+  Kept &k = kept[((mix >> 43) + kKept / 4 * static_cast<uint32_t>(__builtin_ctzll(align))) % kKept];
   if (k.bs == bs && k.seq == seq && k.d == d && k.dtype == dtype && k.dir == dir && k.align == align && bs >= 0) {
     pl = k.plan;
     return FSS_OK;
   }
   const int rc = compute_plan(pl, bs, seq, d, dtype, dir, align, nullptr);
+  ++tls_plans_computed;
   if (rc == FSS_OK) {
     k.bs = bs;
     k.seq = seq;

@@ -206,6 +206,11 @@ int fss_debug_tile_groups(int32_t n_groups, int32_t grid, int32_t n_tiles, int32
 int fss_debug_chain_plan(int64_t bs, int64_t seq, int64_t d, int dtype, int dir, size_t align_bytes,
                          const fss_config *cfg, int32_t *out);
 int32_t fss_debug_chain_anchor(int32_t chunk, int32_t period, int32_t stride);
+/*
+ * Test hook: how often this thread has planned a row-major scan that names no configuration and whose plan it
+ * had not kept.
+ */
+uint64_t fss_debug_plans_computed(void);
 
 /* The configuration the library would choose for this shape (for reporting). */
 int fss_choose_config(int64_t bs, int64_t seq, int64_t d, int dtype, int dir,

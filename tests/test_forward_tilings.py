@@ -62,6 +62,21 @@ def test_plans_do_not_depend_on_what_was_planned_before():
     assert other == first
 
 
+def test_the_plans_for_all_alignments_are_kept_together():
+    """fss_workspace_bytes plans a shape for 2, 4, 8 and 16 bytes: asked again, it plans nothing anew."""
+    lib = _native.lib()
+    rng = np.random.default_rng(7)
+    for _ in range(200):
+        shape = int(rng.integers(1, 64)), int(rng.integers(1, 5000)), int(rng.integers(1, 2000))
+        dtype, direction = int(rng.integers(0, 3)), int(rng.integers(0, 4))
+        need = lib.fss_workspace_bytes(*shape, dtype, direction, None)
+        before = lib.fss_debug_plans_computed()
+        assert lib.fss_workspace_bytes(*shape, dtype, direction, None) == need
+        # (fp32 tensors never start at 2 bytes: that plan is refused, and refusals are not kept)
+        refused = 1 if dtype == _native.FSS_F32 else 0
+        assert lib.fss_debug_plans_computed() - before == refused, (shape, dtype, direction)
+
+
 def test_small_and_large_forwards():
     lib = _native.lib()
     # a launch that leaves most of the device idle takes short tiles, the device's ladder begins where launches fill it
