@@ -236,10 +236,15 @@ inline void complete_config(fss_config &c, int64_t bs, int64_t seq, int64_t d, i
       if (open && !can2 && elems >= (static_cast<int64_t>(1) << 25)) rung(1, 16, 16);
       if (three_tiles && elems >= (static_cast<int64_t>(1) << 23)) rung(1, 16, 16);
       // (rows that share sectors, in very large launches: with 12 waves what is in flight leaves the L2 room to put the seams
-      // between column tiles together.  One launch behind the other, (27, 8422, 210) 140 -> 111 us, (9, 20000, 194) 108 -> 92,
-      // (26, 3001, 526) 110 -> 100, (64, 500, 1234) 93.6 -> 91.0; 32 shapes 4 % in the mean, the slowest (54, 608, 2168) 161 ->
-      // 167; (8, 16359, 232), of 30 million elements, 73.6 -> 77.3)
-      if (open && can2 && shares_sectors(d * esize) && elems >= (static_cast<int64_t>(1) << 25)) rung(2, 16, 12);
+      // between column tiles together.  So not for rows of one tile, which have no seam: (48, 17050, 82) 162 -> 175 us.  Nor
+      // where 192-step chunks pad the sequence further, (43, 235, 3380) 79 -> 92, where it has only a few chunks, (54, 608,
+      // 2168) 160 -> 167, or more of them to find than the look-back has at hand, (4, 25461, 382) 94 -> 101.  Elsewhere, one
+      // launch behind the other, (27, 8422, 210) 140 -> 111, (54, 5718, 146) 147 -> 114, (26, 3001, 526) 110 -> 100, (13,
+      // 2846, 1194) 115 -> 104; 121 shapes 5 % in the mean, the slowest (7, 11540, 494) 88.6 -> 92.8; (8, 16359, 232), of 30
+      // million elements, 73.6 -> 77.3)
+      if (open && can2 && shares_sectors(d * esize) && d > 128 && elems >= (static_cast<int64_t>(1) << 25) && seq >= 1024 &&
+          seq < 16384 && ceil_div(seq, 192) * 192 <= ceil_div(seq, 256) * 256)
+        rung(2, 16, 12);
       rung(2, 16, 16);
       if (seq >= 16384) rung(1, 16, 16); else rung(2, 16, 8);
       if (seq > 256) rung(1, 16, 8); else rung(2, 8, 8);

@@ -1,0 +1,29 @@
+"""Host-side checks of which tilings large launches take: on both sides of each line that a rule draws."""
+import ctypes
+
+import pytest
+
+from fast_sequential_scan_amd import _native
+
+BF16, F32, FP16 = _native.FSS_BF16, _native.FSS_F32, _native.FSS_F16
+FWD, BWD, GATED_FWD = _native.FSS_FWD, _native.FSS_BWD, _native.FSS_GATED_FWD
+
+
+def choose(shape, dtype, direction, align=16):
+    cfg = _native.FssConfig()
+    assert _native.lib().fss_choose_config(*shape, dtype, direction, align, ctypes.byref(cfg)) == 0
+    return cfg.vec, cfg.steps, cfg.waves, cfg.cols
+
+
+# backwards of rows that are no whole number of 64-byte sectors: 12 waves, and each reason for 16
+@pytest.mark.parametrize("shape,waves", [
+    ((27, 8422, 210), 12), ((26, 3001, 526), 12), ((1, 14448, 2346), 12),
+    ((26, 5000, 210), 16),                                          # below 2^25 elements
+    ((27, 8422, 224), 16), ((27, 8422, 256), 16),                   # whole sectors
+    ((48, 17050, 82), 16), ((64, 8422, 126), 16),                   # one column tile per row: no seam
+    ((43, 235, 3380), 16), ((60, 407, 1424), 16), ((49, 1268, 1994), 16),  # 192-step chunks pad further
+    ((54, 608, 2168), 16), ((24, 956, 2034), 16),                   # few chunks
+    ((4, 25461, 382), 16), ((1, 51198, 794), 16)])                  # a long chain
+def test_backward_of_sector_sharing_rows(shape, waves):
+    for dtype in (BF16, FP16):
+        assert choose(shape, dtype, BWD) == (2, 16, waves, 1), shape
