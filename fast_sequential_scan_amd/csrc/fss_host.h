@@ -232,8 +232,11 @@ inline void complete_config(fss_config &c, int64_t bs, int64_t seq, int64_t d, i
     // 32-step slices would cost the backward a dozen spilled registers per lane
     if (narrow) {
       // (one channel per lane, where two do not go, in very large launches: (7, 4958, 3767) 8 waves 370 us, 16 waves
-      // 300; (4, 8354, 1531) 142 and 122; of 2^24 elements, (31, 607, 1041), 45 and 53)
-      if (open && !can2 && elems >= (static_cast<int64_t>(1) << 25)) rung(1, 16, 16);
+      // 300; (4, 8354, 1531) 142 and 122; of 2^24 elements, (31, 607, 1041), 45 and 53.  Not where 256-step chunks pad the
+      // sequence an eighth further than 128-step ones: (28, 525, 2681) 108 and 117, (57, 261, 2529) 111 and 131; of the 82
+      // measured shapes that remain, 10 % faster in the mean, the slowest is (43, 11902, 75), 142.4 and 144.0)
+      if (open && !can2 && elems >= (static_cast<int64_t>(1) << 25) && ceil_div(seq, 256) * 256 * 8 <= ceil_div(seq, 128) * 128 * 9)
+        rung(1, 16, 16);
       if (three_tiles && elems >= (static_cast<int64_t>(1) << 23)) rung(1, 16, 16);
       // (rows that share sectors, in very large launches: with 12 waves what is in flight leaves the L2 room to put the seams
       // between column tiles together.  So not for rows of one tile, which have no seam: (48, 17050, 82) 162 -> 175 us.  Nor

@@ -27,3 +27,15 @@ def choose(shape, dtype, direction, align=16):
 def test_backward_of_sector_sharing_rows(shape, waves):
     for dtype in (BF16, FP16):
         assert choose(shape, dtype, BWD) == (2, 16, waves, 1), shape
+
+
+# backwards of odd width: 16 waves from 2^25 elements on, where their chunks do not pad the sequence much further
+@pytest.mark.parametrize("shape,waves", [
+    ((7, 4958, 3767), 16), ((4, 8354, 1531), 16), ((20, 1072, 1817), 16), ((48, 185, 3847), 16),
+    ((31, 607, 1041), 8),                                           # below 2^25 elements
+    ((57, 261, 2529), 8), ((28, 525, 2681), 8), ((16, 812, 2613), 8)])  # 512, 768 and 1024 for 384, 640 and 896
+def test_backward_of_odd_width(shape, waves):
+    for dtype in (BF16, FP16):
+        assert choose(shape, dtype, BWD) == (1, 16, waves, 1), shape
+    # (tensors of even width that start at an odd element are the same case)
+    assert choose((shape[0], shape[1], shape[2] + 1), BF16, BWD, 2) == (1, 16, waves, 1)
