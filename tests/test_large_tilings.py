@@ -39,3 +39,16 @@ def test_backward_of_odd_width(shape, waves):
         assert choose(shape, dtype, BWD) == (1, 16, waves, 1), shape
     # (tensors of even width that start at an odd element are the same case)
     assert choose((shape[0], shape[1], shape[2] + 1), BF16, BWD, 2) == (1, 16, waves, 1)
+
+
+# forwards of odd width and up to 1024 steps: 128-step chunks where they pad a fifth less than 512-step ones
+@pytest.mark.parametrize("shape,steps", [
+    ((29, 574, 1319), 16), ((23, 749, 1927), 16), ((24, 384, 1735), 16), ((33, 561, 2107), 16),
+    ((36, 393, 1921), 32), ((62, 1000, 343), 32), ((13, 872, 1465), 32),  # 512 for 512, 1024 for 1024 and 896
+    ((35, 169, 2995), 32), ((53, 188, 2485), 32), ((61, 254, 3011), 32),  # one chunk of 256 steps
+    ((24, 1300, 1735), 32),                                               # more than 1024 steps
+    ((85, 588, 1999), 32)])                                               # words beyond half the static array
+def test_forward_of_odd_width(shape, steps):
+    for dtype in (BF16, FP16):
+        assert choose(shape, dtype, FWD)[:2] == (1, steps), shape
+    assert choose((shape[0], shape[1], shape[2] + 1), BF16, FWD, 2)[:2] == (1, steps)
