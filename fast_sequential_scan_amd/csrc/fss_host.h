@@ -265,6 +265,7 @@ inline void complete_config(fss_config &c, int64_t bs, int64_t seq, int64_t d, i
     // The gated kernels spend as much time on arithmetic as on memory and like more, smaller
     // waves; a sequence that 8 waves cover wants two workgroups per CU before it takes them.
     const bool filled = open && elems >= forward_model_elems(narrow, gated);  // (below: where the estimate starts from)
+    const bool twelve = ceil_div(seq, 192) * 192 * 10 <= ceil_div(seq, 128) * 128 * 11;
     if (narrow && filled && !can2) {
       // one channel per lane (odd widths, or rows that two would pad too far): 16 steps and 12 waves, two workgroups on a
       // compute unit, whatever the length, or 8 waves and three, where 12 pad the sequence by a tenth more.  One launch behind
@@ -272,7 +273,6 @@ inline void complete_config(fss_config &c, int64_t bs, int64_t seq, int64_t d, i
       // 749) 154.7, 197.8, 127.0; (5, 25000, 383) 143.1, 165.7, 112.5; (18, 7063, 287) 112, 86.6, 85.8; (23, 1901, 985) 121,
       // 98.1, 92.4.  8 waves lose most where the column tiles are a multiple of three, as the launch's 768 workgroups are; of 34
       // shapes 12 are 10 % faster than 8 in the mean, the slowest (83, 1166, 405) 97.5 -> 104.8.
-      const bool twelve = ceil_div(seq, 192) * 192 * 10 <= ceil_div(seq, 128) * 128 * 11;
       rung(1, 16, twelve ? 12 : 8, 0);
     } else if (narrow && filled) {
       // the largest tile where there is just one for every compute unit: (4, 2048, 2048) one launch behind the other
@@ -297,9 +297,13 @@ inline void complete_config(fss_config &c, int64_t bs, int64_t seq, int64_t d, i
       if (seq >= 1024) rung(1, 16, 8, 0); else rung(1, 16, 16, 0);
     } else {
       // fp32: the largest tile where its rounds are whole ((8, 4096, 1024) 32 steps and 16 waves 83 us, 16 steps 86),
-      // elsewhere 16 steps and 12 waves ((10, 24028, 128) 87 -> 78, (11, 1623, 1152) 62 -> 51, (9, 7795, 67) 33 -> 24)
+      // elsewhere 16 steps and 12 waves ((10, 24028, 128) 87 -> 78, (11, 1623, 1152) 62 -> 51, (9, 7795, 67) 33 -> 24),
+      // or 8 waves where 12 pad the sequence by a tenth more, as many as with 16 bits: up to 256 steps 12 were 4 % slower in the
+      // mean than the largest tile's ladder and 8 are 10 % faster, (42, 196, 2368) 46.8, 62.7 and 48.9 us, (34, 214, 664)
+      // 17.2, 21.0 and 17.1; of 95 shapes 8 lose most against that ladder in (18, 72, 3328), 13.8 and 18.6.  Known to be
+      // slower with 12 waves: (7, 5420, 175) 29.3 -> 32.6, whose second round is nearly empty
       const int64_t big = bs * ceil_div(d, 64) * ceil_div(seq, 512), of_round = ceil_div(big, kCus) * kCus;
-      if (filled && (big * 50 < of_round * 49 || seq * 50 < ceil_div(seq, 512) * 512 * 49)) rung(1, 16, 12, 0);
+      if (filled && (big * 50 < of_round * 49 || seq * 50 < ceil_div(seq, 512) * 512 * 49)) rung(1, 16, twelve ? 12 : 8, 0);
       if (seq > 256) rung(1, 32, 16); else rung(1, 32, 8, 2 * kCus);
       rung(1, 16, 16, 0);
     }
