@@ -206,16 +206,22 @@ inline void complete_config(fss_config &c, int64_t bs, int64_t seq, int64_t d, i
   const bool wide32_bwd = big32 && can2 && elems >= (static_cast<int64_t>(1) << 27);
   // Rows of three 64-channel tiles, in large launches: with two channels per lane a quarter of the lanes idles.
   // One launch behind the other, backward (6, 40000, 192) 106 -> 92 us, (30, 2000, 192) 29.3 -> 27.7; ten of eleven shapes 2 to
-  // 13 % faster, (8, 40000, 192) 120 -> 123.  Forward, 8 waves, (4, 57534, 192) 71 -> 61, (2, 60000, 192) 42 -> 35, (7, 30000,
-  // 192) 61.8 -> 55.5, up to 45 Mi elements; from there (5, 50000, 192) 63.3 -> 65.2, (8, 40000, 192) 80.6 -> 84.1,
-  // (16, 16000, 192) 65.4 -> 63.9; below 2^24 elements nothing.
+  // 13 % faster, (8, 40000, 192) 120 -> 123.  Forward, 8 waves, from 2^24 elements (below them nothing): (4, 57534, 192) 71 ->
+  // 61, (7, 30000, 192) 61.8 -> 55.5, (30, 13002, 192) 97 -> 88, (11, 56047, 192) 151 -> 138; of 17 shapes from 45 Mi to 2^27
+  // elements, 7 % in the mean, the slowest is (8, 42392, 192), 88.4 -> 88.8; (8, 40000, 192) 80.6 -> 84.1.  Not where 16 waves cover the
+  // sequence in one chunk and 8 do not: (591, 268, 192) 44.6 and 55.5, (878, 284, 192) 71 and 79.  The forward's words,
+  // a third and more above those with two channels, have to stay within the scratch of the entry point that allocates
+  // nothing.  Other widths with idle lanes: 320 channels and 448 gain up to 5 % in the backward and lose as much as
+  // they gain in the forward; rows below 192 that share sectors are a case of their own (160: 114 -> 121 us backward).
   const bool three_tiles = open && narrow && !gated && d == 3 * 64;
   Rung ladder[8];
   int n = 0;
   auto rung = [&](int v, int s, int w, int64_t need = kCus) { ladder[n++] = Rung{v, s, w, need}; };
   const bool fwd = dir == FSS_FWD;
   if (!gated && fwd) {
-    if (three_tiles && elems >= (int64_t{1} << 24) && elems < (int64_t{45} << 20)) rung(1, 32, 8);
+    if (three_tiles && elems >= (int64_t{1} << 24) && (seq <= 256 || seq > 512) &&
+        bs * 3 * ceil_div(seq, 256) * 3 * 64 * static_cast<int64_t>(sizeof(uint64_t)) + static_cast<int64_t>(kHeaderBytes) <= FSS_NOALLOC_SCRATCH_BYTES)
+      rung(1, 32, 8);
     if (narrow) rung(2, 32, 16);
     // (one channel per lane, where two do not go, and sequences that 512-step chunks pad a quarter further than 128-step ones:
     // (24, 384, 1735) 23.2 -> 19.2 us, (29, 574, 1319) 44.4 -> 33.6, (28, 748, 445) 15.8 -> 13.7; 15 shapes above 15 Mi

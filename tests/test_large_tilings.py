@@ -62,3 +62,23 @@ def test_forward_of_odd_width(shape, steps):
     ((8, 4096, 1024), (1, 32, 16, 1))])                             # whole rounds of the largest tile
 def test_gated_forward_in_single_precision(shape, want):
     assert choose(shape, F32, GATED_FWD) == want
+
+
+# rows of three 64-channel tiles: one channel per lane in large launches
+def test_rows_of_three_column_tiles():
+    for dtype in (BF16, FP16):
+        for shape in [(4, 57534, 192), (7, 30000, 192), (30, 13002, 192), (11, 56047, 192), (12, 14564, 192)]:
+            assert choose(shape, dtype, FWD) == (1, 32, 8, 1), shape
+        for shape in [(591, 268, 192), (878, 284, 192), (350, 512, 192)]:  # one chunk of 16 waves
+            assert choose(shape, dtype, FWD)[:2] == (2, 32), shape
+        # (words beyond the static array of the forward that allocates nothing, which takes these shapes otherwise)
+        for shape in [(2, 480000, 192), (1000, 1000, 192)]:
+            assert choose(shape, dtype, FWD)[0] == 2
+            assert _native.lib().fss_workspace_bytes(*shape, dtype, FWD, None) <= 16 << 20, shape
+        for shape in [(4, 20000, 192), (30, 2000, 192), (8, 40000, 192)]:
+            assert choose(shape, dtype, BWD) == (1, 16, 16, 1), shape
+        assert choose((20, 2000, 192), dtype, BWD)[0] == 2  # below 2^23 elements
+        for d in (128, 256, 320):
+            assert choose((8, 20000, d), dtype, FWD)[0] == 2 and choose((8, 20000, d), dtype, BWD)[0] == 2
+    # fp32 has one channel per lane at these widths anyhow
+    assert choose((4, 57534, 192), F32, FWD)[0] == 1
