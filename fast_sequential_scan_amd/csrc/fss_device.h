@@ -810,13 +810,6 @@ __device__ __forceinline__ void await_all_maps(const uint32_t *ready, int lane, 
 // composition of maps 0 .. w-1, in place of map w, which nobody else reads), and (A, B) the
 // chunk's map.  Every other wave then finds its prefix with one LDS read behind the next barrier.
 // The order of the composition is the waves' order, whatever the order of their arrival.
-// One look at all the waves' words says how many maps may be read, and those are read kFoldBatch at a
-// time: with a look and a read per map, each a round trip to the LDS that the next one waits for, the
-// chunk's map went out 0.1 us later for every wave of the workgroup.  bf16 gated forward (1, 7243, 64) 9.7 -> 8.8 us,
-// (2, 1024, 768) 7.6 -> 7.0; forward (8, 1819, 64) 8.5 -> 8.1, (1, 65521, 256) 23.3 -> 22.8; fp32 forward (2, 777,
-// 328) 9.4 -> 8.7; large launches up to 1 %.  Two at a time with two channels and more per lane: four cost the
-// gated kernel with 16 steps the 81st register and a third of its resident workgroups ((16, 2048, 512) in
-// that configuration 20.9 -> 23.4 us).
 // Looking at a wave's word and then reading its map, for one wave after the other, are two round trips to
 // the LDS that the next map waits for: 0.1 us later for every wave of the workgroup.  With one
 // channel per lane one look covers all the waves and the maps that have arrived are read four at a time;
@@ -826,8 +819,8 @@ __device__ __forceinline__ void await_all_maps(const uint32_t *ready, int lane, 
 // 8.7; with two channels (8, 4096, 1024) 44.2 -> 43.6, (1, 65521, 256) 23.4 -> 22.9.  The other way round:
 // awaited in fours with one channel 9.2, 7.2, 8.2 and 9.1 us; one look with two channels (16, 2048, 512) gated, 16
 // steps and 8 waves, 20.9 -> 21.7; four maps at a time there 23.4 (the 81st register, a third of the
-// resident workgroups).  The channel-major kernels, a row's map to a lane, await theirs in fours: forward (8, 1024, 2047) 20.8 us,
-// with one look 21.9 (though chained ragged rows gain by the look: (13, 768, 4859) 71.3 -> 67.3).
+// resident workgroups).  The channel-major kernels, a row's map to a lane, take one look where the launch is chained and
+// await fours where it is not (cm_scan_kernel).
 template <int VEC>
 constexpr int kFoldBatch = VEC == 1 ? 4 : 2;
 template <int N>

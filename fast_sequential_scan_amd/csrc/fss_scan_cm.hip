@@ -50,7 +50,7 @@ struct Flag {
 // again.  bf16, one row to a wave -> shared: (64, 4096, 64) forward 62 -> 16.7 us, backward 84 -> 28.8 (5.8
 // TB/s); (64, 1024, 250) 29.4 -> 17.6 and 40.2 -> 30.7 us; (2, 1024, 256) 6.4 -> 4.4 and 5.7 -> 5.0; (64, 4096,
 // 23), before with one step per lane, 52 -> 11.6 and 63 -> 19.1.
-template <typename E, int VEC, int ROWS, bool BWD, bool RAGGED, bool SHORT>
+template <typename E, int VEC, int ROWS, bool BWD, bool RAGGED, bool SHORT, bool CHAINED>
 __device__ __forceinline__ void cm_tile(const ScanArgs &p, TileCtx &c, int64_t row0, int64_t n_rows) {
   using RowT = Row<E, VEC>;
   using OneT = Row<E, 1>;
@@ -203,9 +203,9 @@ __device__ __forceinline__ void cm_tile(const ScanArgs &p, TileCtx &c, int64_t r
   }
 
   float slice_in = 0.0f;
-  if (!SHORT && (c.chained || c.n_waves > 1)) {
+  if (!SHORT && (CHAINED || c.n_waves > 1)) {
     c.tag = launch_tag(c);
-    chain_chunks<1, BWD, kFoldBatch<1>, true>(p, c, &mA, &mB, nullptr, &slice_in, load_h);
+    chain_chunks<1, BWD, kFoldBatch<1>, !CHAINED>(p, c, &mA, &mB, nullptr, &slice_in, load_h);
   } else {
     load_h();
   }
@@ -256,7 +256,18 @@ __device__ __forceinline__ void cm_tile(const ScanArgs &p, TileCtx &c, int64_t r
 
 // ScanArgs here: seq = the contiguous length, d = number of rows (bs * channels),
 // n_ctiles = ceil(rows / ROWS) row groups, n_chunks = ceil(seq / (waves*64*VEC)).
-template <typename E, int VEC, int ROWS, bool BWD, bool RAGGED, bool SHORT>
+//
+// CHAINED: more than one chunk.  Later chunks wait for a chunk's map, so wave 0 folds what has arrived after one look at
+// all the waves' words; in a launch of one chunk only the workgroup's own waves wait, and wave 0 awaits
+// their maps in fours.  Kernels of their own because a branch inside one kernel pays for both: the part that
+// chains costs a backward 25 vector registers and 33 spilled scalar ones, a forward 11 and 29.  bf16, one launch behind the
+// other, fours everywhere / one look everywhere / as it is: chained forwards (13, 768, 4859) 69.6, 66.0 and 65.7 us, (6, 192,
+// 32814) 53.7, 50.8 and 51.1; unchained (8, 1024, 2047) 22.0, 22.8 and 21.4, (8, 1024, 1023) 14.8, 14.3 and 13.5, (8, 1024,
+// 4095) 45.4, 44.1 and 43.0, backward (8, 1024, 4096) 59.0, 59.1 and 56.0.  22 shapes in both directions and in bf16 and
+// fp32: 1.5 % faster in the mean than fours everywhere, 0.8 % than one look; the slowest, forwards (8, 1024, 4096)
+// 40.1 -> 40.7 and (4, 300, 9001) 19.8 -> 20.1.  One look without a chain: 0.4 % slower in the mean, forward (8,
+// 1024, 1023) 13.8.
+template <typename E, int VEC, int ROWS, bool BWD, bool RAGGED, bool SHORT, bool CHAINED>
 __global__ __launch_bounds__(1024) void cm_scan_kernel(const ScanArgs p) {
   extern __shared__ float lds[];
   __shared__ uint32_t s_ready[16];  // per wave: see announce_map
@@ -280,8 +291,8 @@ __global__ __launch_bounds__(1024) void cm_scan_kernel(const ScanArgs p) {
 #ifdef FSS_TRACE
   c.trace_wave = 0;
 #endif
-  c.chained = p.n_chunks > 1;
-  c.epoch = c.chained ? read_epoch(p) : 0u;
+  c.chained = CHAINED;
+  c.epoch = CHAINED ? read_epoch(p) : 0u;
   c.tag = 0u;
   c.anchor = c.span = 0;
 
@@ -297,24 +308,24 @@ __global__ __launch_bounds__(1024) void cm_scan_kernel(const ScanArgs p) {
     c.ctile = static_cast<int>(ctile);
     c.last = c.chunk == p.n_chunks - 1;
     place_in_chain(plan, c);
-    cm_tile<E, VEC, ROWS, BWD, RAGGED, SHORT>(p, c, static_cast<int64_t>(ctile) * (SHORT ? ROWS * (64 >> p.row_lanes_log2) : ROWS), p.d);
+    cm_tile<E, VEC, ROWS, BWD, RAGGED, SHORT, CHAINED>(p, c, static_cast<int64_t>(ctile) * (SHORT ? ROWS * (64 >> p.row_lanes_log2) : ROWS), p.d);
   }
   count_out(p, c);
 }
 
 // ---- launching ---------------------------------------------------------------------
 
-template <typename E, int VEC, bool BWD, bool RAGGED = false, bool SHORT = false>
-int launch_cm_one(const ScanArgs &args, const CmPlan &pl, int max_groups, hipStream_t stream) {
+template <typename E, int VEC, bool BWD, bool RAGGED, bool SHORT, bool CHAINED>
+int launch_cm_kernel(const ScanArgs &args, const CmPlan &pl, int max_groups, hipStream_t stream) {
   constexpr int kRows = BWD || SHORT ? kCmRowsBwd : kCmRowsFwd;  // (eight vectors a lane would cost SHORT 23 spilled registers)
   static int resident[17] = {0};
   const int waves = pl.waves;
   const size_t lds = lds_bytes(waves, 1);
-  const int fit = resident_workgroups(cm_scan_kernel<E, VEC, kRows, BWD, RAGGED, SHORT>, waves, lds, resident);
+  const int fit = resident_workgroups(cm_scan_kernel<E, VEC, kRows, BWD, RAGGED, SHORT, CHAINED>, waves, lds, resident);
   if (fit <= 0) return FSS_ERR_LAUNCH;
   int64_t n_groups = pl.n_tiles < fit ? pl.n_tiles : fit;
   if (max_groups > 0 && max_groups < n_groups) n_groups = max_groups;
-  hipLaunchKernelGGL((cm_scan_kernel<E, VEC, kRows, BWD, RAGGED, SHORT>), dim3(static_cast<uint32_t>(n_groups)),
+  hipLaunchKernelGGL((cm_scan_kernel<E, VEC, kRows, BWD, RAGGED, SHORT, CHAINED>), dim3(static_cast<uint32_t>(n_groups)),
                      dim3(static_cast<uint32_t>(waves) * 64), lds, stream, args);
   const hipError_t e = hipGetLastError();
   if (e != hipSuccess) {
@@ -322,6 +333,13 @@ int launch_cm_one(const ScanArgs &args, const CmPlan &pl, int max_groups, hipStr
     return FSS_ERR_LAUNCH;
   }
   return FSS_OK;
+}
+
+template <typename E, int VEC, bool BWD, bool RAGGED = false, bool SHORT = false>
+int launch_cm_one(const ScanArgs &args, const CmPlan &pl, int max_groups, hipStream_t stream) {
+  if constexpr (!SHORT)  // (whose rows are one lane group's, in one chunk)
+    if (pl.n_chunks > 1) return launch_cm_kernel<E, VEC, BWD, RAGGED, SHORT, true>(args, pl, max_groups, stream);
+  return launch_cm_kernel<E, VEC, BWD, RAGGED, SHORT, false>(args, pl, max_groups, stream);
 }
 
 template <typename E, bool BWD>

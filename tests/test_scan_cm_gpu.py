@@ -112,6 +112,19 @@ def test_cm_result_does_not_depend_on_config_f32(oracle, config):
     _run(oracle, 2, 6, 600, torch.float32, config=config, seed=2, recipe="normal")
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32], ids=["bf16", "f32"])
+@pytest.mark.parametrize("waves", [1, 2, 3, 5, 7, 8, 13, 16])
+def test_cm_one_chunk_and_two_of_any_number_of_waves(oracle, waves, dtype):
+    """Launches of one chunk and chained ones are different kernels: the longest row of the one, the shortest of the
+    other, whole and ragged last vectors, numbers of waves that are no multiple of four."""
+    vec = 8 if dtype == torch.bfloat16 else 4
+    reach = waves * 64 * vec
+    for seq in (reach, reach + vec):
+        _run(oracle, 2, 9, seq, dtype, config=(vec, 0, waves), seed=waves)
+    for seq in (reach - 1, reach + 1):  # (a ragged row's number of waves is the library's)
+        _run(oracle, 2, 9, seq, dtype, seed=waves)
+
+
 def test_cm_headline_size_and_row_major_agreement(oracle):
     """bs8 d1024 seq4096 bf16 against the oracle, and against the row-major kernels on the
     permuted tensors (two different decompositions of the same recurrence)."""
