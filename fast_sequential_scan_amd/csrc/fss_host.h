@@ -244,8 +244,8 @@ inline void complete_config(fss_config &c, int64_t bs, int64_t seq, int64_t d, i
       // (one channel per lane, where two do not go, in very large launches: (7, 4958, 3767) 8 waves 370 us, 16 waves
       // 300; (4, 8354, 1531) 142 and 122; of 2^24 elements, (31, 607, 1041), 45 and 53.  Not where 256-step chunks pad the
       // sequence an eighth further than 128-step ones: (28, 525, 2681) 108 and 117, (57, 261, 2529) 111 and 131.  Nor in
-      // narrow rows: 65 to 87 channels 2 % slower in the mean of 21 shapes, (212, 2488, 67) 130 and 148, (75, 11521, 71) 229
-      // and 240, and up to 64 the same; from 91 to 191, 6 % faster in the mean of 31, the slowest (252, 4063, 97) 279 and 284;
+      // narrow rows: 65 to 87 channels 3 % slower in the mean of 16 shapes, (212, 2488, 67) 130 and 148, (75, 11521, 71) 229
+      // and 240, and up to 64 no faster; from 93 to 191, 7 % faster in the mean of 28, the slowest (252, 4063, 97) 279 and 284;
       // 82 wider ones 10 %)
       if (open && !can2 && d >= 88 && elems >= (static_cast<int64_t>(1) << 25) &&
           ceil_div(seq, 256) * 256 * 8 <= ceil_div(seq, 128) * 128 * 9)

@@ -31,7 +31,7 @@ def test_backward_of_sector_sharing_rows(shape, waves):
 
 # backwards of odd width: 16 waves from 2^25 elements on, where their chunks do not pad the sequence much further and rows are not narrow
 @pytest.mark.parametrize("shape,waves", [
-    ((75, 11521, 71), 8), ((171, 8554, 85), 8), ((171, 8554, 89), 16), ((29, 43921, 47), 8),
+    ((75, 11521, 71), 8), ((171, 8554, 85), 8), ((171, 8554, 89), 16), ((179, 8888, 47), 8),
     ((7, 4958, 3767), 16), ((4, 8354, 1531), 16), ((20, 1072, 1817), 16), ((48, 185, 3847), 16),
     ((31, 607, 1041), 8),                                           # below 2^25 elements
     ((57, 261, 2529), 8), ((28, 525, 2681), 8), ((16, 812, 2613), 8)])  # 512, 768 and 1024 for 384, 640 and 896
