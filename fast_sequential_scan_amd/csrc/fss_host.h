@@ -307,12 +307,16 @@ inline void complete_config(fss_config &c, int64_t bs, int64_t seq, int64_t d, i
     } else {
       // fp32: the largest tile where its rounds are whole ((8, 4096, 1024) 32 steps and 16 waves 83 us, 16 steps 86),
       // elsewhere 16 steps and 12 waves ((10, 24028, 128) 87 -> 78, (11, 1623, 1152) 62 -> 51, (9, 7795, 67) 33 -> 24),
-      // or 8 waves where 12 pad the sequence by a tenth more, as many as with 16 bits: up to 256 steps 12 were 4 % slower in the
-      // mean than the largest tile's ladder and 8 are 10 % faster, (42, 196, 2368) 46.8, 62.7 and 48.9 us, (34, 214, 664)
-      // 17.2, 21.0 and 17.1; of 95 shapes 8 lose most against that ladder in (18, 72, 3328), 13.8 and 18.6.  Known to be
-      // slower with 12 waves: (7, 5420, 175) 29.3 -> 32.6, whose second round is nearly empty
+      // or 8 waves where 12 pad the sequence by a tenth more ((34, 214, 664) 17.2 -> 17.1, with 12 21.0).  What a sequence of up to
+      // 512 steps gains by those 8 hangs on the steps of the last wave of the larger tile, which all the others wait for: 16 to
+      // 31 of 32, 30 % in the mean of 88 shapes, (237, 59, 704) 43.3 -> 29.5, the slowest (186, 80, 3063) 168 -> 192.  Fewer or
+      // all 32, nothing in the mean of 81; above 64 steps, in rows of whole sectors, a loss of 3 % in the mean of 48, (60, 78, 1024)
+      // 16.1 -> 23.3, (142, 386, 1088) 134 -> 155: there the ladder keeps its tile, at a loss of at most 9 % ((149, 206, 896) 77.5
+      // -> 84.9).  Known to be slower with 12 waves: (7, 5420, 175) 29.3 -> 32.6, whose second round is nearly empty, (12, 12130, 782)
+      // 323 -> 341, (40, 942, 1345) 151 -> 165; 80 shapes from 4 Mi to 128 Mi elements are 13 % faster in the mean.
       const int64_t big = bs * ceil_div(d, 64) * ceil_div(seq, 512), of_round = ceil_div(big, kCus) * kCus;
-      if (filled && (big * 50 < of_round * 49 || seq * 50 < ceil_div(seq, 512) * 512 * 49)) rung(1, 16, twelve ? 12 : 8, 0);
+      const bool ladder = !twelve && seq > 64 && seq <= 512 && seq % 32 < 16 && !shares_sectors(d * esize);
+      if (filled && !ladder && (big * 50 < of_round * 49 || seq * 50 < ceil_div(seq, 512) * 512 * 49)) rung(1, 16, twelve ? 12 : 8, 0);
       if (seq > 256) rung(1, 32, 16); else rung(1, 32, 8, 2 * kCus);
       rung(1, 16, 16, 0);
     }

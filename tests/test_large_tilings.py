@@ -55,10 +55,14 @@ def test_forward_of_odd_width(shape, steps):
     assert choose((shape[0], shape[1], shape[2] + 1), BF16, FWD, 2)[:2] == (1, steps)
 
 
-# gated forwards of fp32 from 4 Mi elements on: 12 waves, or 8 where 12 pad the sequence by more than a tenth
+# gated forwards of fp32 from 4 Mi elements on: 12 waves, or 8 where 12 pad the sequence by more than a tenth; the ladder's where one
+# of its tiles covers the sequence and the last wave has fewer than 16 of 32 steps, in rows of whole sectors
 @pytest.mark.parametrize("shape,want", [
     ((10, 24028, 128), (1, 16, 12, 1)), ((11, 1623, 1152), (1, 16, 12, 1)), ((9, 7795, 67), (1, 16, 12, 1)),
-    ((34, 214, 664), (1, 16, 8, 1)), ((42, 196, 2368), (1, 16, 8, 1)), ((40, 459, 1280), (1, 16, 8, 1)),
+    ((34, 214, 664), (1, 16, 8, 1)), ((229, 444, 256), (1, 16, 8, 1)), ((60, 80, 1024), (1, 16, 8, 1)), ((41, 430, 3648), (1, 32, 16, 1)),
+    ((42, 196, 2368), (1, 32, 8, 1)), ((60, 78, 1024), (1, 32, 4, 1)), ((142, 386, 1088), (1, 32, 16, 1)), ((92, 96, 3328), (1, 32, 4, 1)),
+    ((41, 417, 3646), (1, 16, 8, 1)), ((45, 590, 3264), (1, 16, 8, 1)),  # rows that share sectors; more than 512 steps
+    ((30, 322, 3264), (1, 16, 12, 1)),                              # 384 steps either way
     ((59, 47, 3904), (1, 16, 4, 1)), ((24, 55, 3756), (1, 16, 4, 1)), ((43, 32, 3345), (1, 16, 2, 1)),
     ((8, 4096, 1024), (1, 32, 16, 1))])                             # whole rounds of the largest tile
 def test_gated_forward_in_single_precision(shape, want):
