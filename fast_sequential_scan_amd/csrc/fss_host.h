@@ -130,13 +130,17 @@ inline int choose_cols(const fss_config &c, int64_t bs, int64_t seq, int64_t d, 
   return tiles > kCus && tiles <= 2 * kCus ? 2 : 1;
 }
 
-// What a launch of a forward kernel takes, in ns, as a function of its tiling: a launch and a tile's
-// serial work (more of it the more steps a wave takes one after the other, in the gated kernels their
-// arithmetic), the chain (a round trip to memory, and more maps to find the more chunks of a
-// sequence are in flight at once), every round of the resident workgroups after the first, and the
-// bytes: what the busiest compute unit moves, and all of them together, padding included.  Fitted to 4600
-// pairs of a shape of 2^17 to 2^25 elements (bs 1..64, seq 16..65536, d 64..4096, a quarter of the
-// widths odd or ragged) and a configuration, each weighted by how near it came to the shape's fastest.
+// An estimate, in ns, of what a launch of a forward kernel takes with a tiling, for comparing tilings of one shape.  A
+// regression on eight terms: a launch, the steps that a wave takes one after the other, the same times channels per lane, the
+// chain (a round trip to memory, and more maps to find the more chunks of a sequence are in flight at
+// once), every round of the resident workgroups after the first, and the bytes, padding included: what the busiest
+// compute unit moves, and all of them together.  Fitted to 4600 pairs of a shape of 2^17 to 2^25 elements (bs 1..64, seq
+// 16..65536, d 64..4096, a quarter of the widths odd or ragged) and a configuration, each weighted by how near it came to
+// the shape's fastest.  The terms grow together in such pairs (steps with bytes, channels with both), so no coefficient is
+// a cost by itself: the negative `channel_step` of 16 bits does not say that a step of two channels takes less time than
+// one of one.  What the estimate is good for is measured on 480 other shapes (profiles/forward_tilings_pairs.csv, 5166 pairs,
+// checked by tests/test_forward_tilings.py): its values scatter by 11 to 12 % around the plain kernels' times and 20 % around
+// the gated.
 struct ForwardCost {
   double launch, step, channel_step, chain, depth, round, unit_bytes, all_bytes;
 };
@@ -157,14 +161,18 @@ inline double forward_ns(const ForwardCost &m, int64_t bs, int64_t seq, int64_t 
 
 // Forwards of fewer elements than this take the tiling that forward_ns finds fastest, if it is clearly faster
 // than the ladder's (complete_config): the ladder was drawn from launches that fill the device, and
-// below them "the largest tile that leaves one per compute unit" is the wrong question.  Against the
-// fastest of 15 to 25 configurations, bf16 forwards below 2^21 elements lost 16 % with the ladder and lose 3 %,
-// gated ones 18 and 3 %; from 2^21 to 2^24 (gated 2^23) 9 and 3 %, 16 and 4 %; fp32 below 2^21 12 and 3 %, gated below
-// 2^22 12 and 5 %.  The margin keeps out what the estimate cannot tell apart: without it one launch in ten
-// from 2^21 elements on became slower, with it one in fifty.  Ladder -> estimate, shapes
-// that the fit had not seen: bf16 gated forward (1, 1021, 1610) 12.7 -> 8.8 us, (10, 1098, 384) 14.7 -> 10.8, (2, 29970, 64)
-// 16.8 -> 12.4; fp32 (26, 82, 64) 5.3 -> 3.9; 175 of them 10 % in the mean, one in fifty slower (by 2 to 5 %).
-// Larger launches stay with the ladder, which is within 2-4 % of the fastest there.
+// below them "the largest tile that leaves one per compute unit" is the wrong question.  What a choice loses against the fastest of
+// about eleven tilings on those 480 shapes, in the mean, ladder and estimate, below a sixteenth of the limit, a quarter, half
+// and the limit, and from there to twice it (where the ladder is taken):
+//   bf16   25.6 and 3.6 %, 12.6 and 3.1, 9.2 and 2.1, 6.1 and 3.2;   5.6 and 2.4
+//   gated  27.7 and 1.9 %, 34.4 and 5.6, 33.9 and 9.9, 20.8 and 7.3;  3.4 and 5.6
+//   fp32   below a quarter 19.1 and 3.8 %, 14.9 and 4.6, 8.2 and 3.3;  4.5 and 3.8
+//   gated  19.1 and 2.5 %, 22.7 and 8.5, 10.7 and 4.3, 4.2 and 4.3;  7.5 and 9.8
+// So the gated limits lie where the ladder becomes the better one; the plain ones lie lower than they could, at the sizes
+// (for 16 bits just below 2^24 elements) that the ladder's own sweeps cover.  The margin keeps out what the
+// estimate cannot tell apart: of the 349 shapes below the limits 8 are slower by it than with the ladder, gated ones
+// all, (3, 9524, 128) 11.3 -> 13.1 us the furthest.  Furthest from the fastest: gated (30, 610, 144) 16.7 us, two channels and
+// 12 waves 10.8.
 constexpr int64_t forward_model_elems(bool narrow, bool gated) {
   return narrow ? (gated ? int64_t{1} << 23 : int64_t{15} << 20) : int64_t{1} << (gated ? 22 : 21);
 }
@@ -176,14 +184,15 @@ constexpr int64_t kModelWordBytes = int64_t{4} << 20;
 // tensors of the call.
 //
 // From sweeps over bs 1..64, seq 256..16384, d 256..4096 per storage type and kernel
-// family (every shape against 8-11 configurations), which all show the same thing: the
-// largest tile that still leaves one tile per CU wins.  Large tiles mean few chunks per
+// family (every shape against 8-11 configurations): for lengths and widths that tiles divide,
+// the largest tile that still leaves one tile per CU wins.  Large tiles mean few chunks per
 // sequence (a short chain) and long uninterrupted streams per wave; 16 waves of 32
 // (backward 16) timesteps with 4 bytes per lane is the largest that fits the register
 // file.  So the choice walks down a ladder of tile sizes, each half the one before, and
 // takes the first with at least one tile per CU; which of time, channels per lane and waves
-// is halved at each rung is what the sweeps decided.  Below the last rung the problem
-// is latency-bound and the smallest tile is as good as any.
+// is halved at each rung is what the sweeps decided.  Odd and line-sharing widths, ragged lengths and the gated
+// kernels differ from that; each such rung says by how much.  Forwards that leave the device idle are
+// weighed by forward_ns, whatever the ladder says.
 inline void complete_config(fss_config &c, int64_t bs, int64_t seq, int64_t d, int dtype, int dir,
                      size_t align, bool gated = false) {
   const bool narrow = dtype != FSS_F32;  // 16-bit storage

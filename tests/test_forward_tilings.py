@@ -1,11 +1,15 @@
 """Host-side checks of how small forwards are tiled (the cost estimate in csrc/fss_host.h)."""
+import csv
 import ctypes
+import os
 import threading
 
 import numpy as np
+import pytest
 
 from fast_sequential_scan_amd import _native
 
+PAIRS = os.path.join(os.path.dirname(os.path.dirname(os.path.abspath(__file__))), "profiles", "forward_tilings_pairs.csv")
 LIMIT = 4 << 20  # bytes of chaining words an estimate may ask for beyond the ladder's
 
 
@@ -104,3 +108,25 @@ def test_named_parts_of_a_tiling_keep_their_ladder():
         out = (ctypes.c_int32 * 8)()
         assert lib.fss_debug_chain_plan(*shape, dtype, direction, 16, ctypes.byref(cfg), out) == 0, (shape, named)
         assert (out[6], out[2], out[1] * out[7], out[7]) == want, (shape, named, list(out))
+
+
+# kernel, type, elements below which the estimate chooses, and what its choice may lose in the mean against the fastest
+# measured tiling (what it loses, rounded up; the ladder alone loses 14, 29, 14 and 14 %)
+@pytest.mark.parametrize("kernel,dtype,limit,loss", [
+    ("plain", "bf16", 15 << 20, 0.035), ("gated", "bf16", 1 << 23, 0.07),
+    ("plain", "fp32", 1 << 21, 0.045), ("gated", "fp32", 1 << 22, 0.06)])
+def test_the_choice_is_near_the_fastest_measured_tiling(kernel, dtype, limit, loss):
+    """The estimate against times of shapes that it was not fitted to (us, one launch of many)."""
+    lib = _native.lib()
+    code = {"bf16": _native.FSS_BF16, "fp32": _native.FSS_F32}[dtype]
+    times = {}
+    with open(PAIRS) as f:
+        for row in csv.DictReader(f):
+            if (row["kernel"], row["dtype"]) == (kernel, dtype):
+                shape = tuple(int(row[k]) for k in ("bs", "seq", "d"))
+                times.setdefault(shape, {})[tuple(int(row[k]) for k in ("vec", "steps", "waves", "cols"))] = float(row["us"])
+    shapes = [s for s in times if s[0] * s[1] * s[2] < limit]
+    assert len(shapes) >= 70
+    ratios = [times[s][choose(lib, s, code, _native.FSS_FWD if kernel == "plain" else _native.FSS_GATED_FWD)] / min(times[s].values())
+              for s in shapes]
+    assert np.exp(np.mean(np.log(ratios))) - 1 <= loss
