@@ -66,6 +66,34 @@ def test_plans_do_not_depend_on_what_was_planned_before():
     assert other == first
 
 
+@pytest.mark.parametrize("which", range(6), ids=["bs", "seq", "d", "dtype", "dir", "align"])
+def test_kept_plans_are_told_apart_by_every_argument(which):
+    """Requests that differ in one argument only, asked in turn so that they meet in the table's slots, get what a plan
+    that is never kept (of a configuration of zeros) says: a lookup that left the argument out would not.  (One shape's types
+    and directions never share a slot, so those two are told apart already there.)"""
+    lib = _native.lib()
+    rng = np.random.default_rng(8)
+
+    def plan(request, cfg):
+        out = (ctypes.c_int32 * 8)()
+        rc = lib.fss_debug_chain_plan(*request, cfg, out)
+        return (rc, *out) if rc == 0 else (rc,)
+
+    zeros = ctypes.byref(_native.FssConfig())
+    told_apart = 0
+    for _ in range(150):
+        draw = [lambda: int(rng.integers(1, 200)), lambda: int(rng.integers(65, 20000)), lambda: int(rng.integers(32, 2000)),
+                lambda: int(rng.integers(0, 3)), lambda: int(rng.integers(0, 4)), lambda: int(rng.choice([2, 4, 8, 16, 32]))]
+        start = [f() for f in draw]
+        values = [range(3), range(4), (2, 4, 8, 16, 32)][which - 3] if which >= 3 else [draw[which]() for _ in range(12)]
+        requests = [tuple(start[:which] + [int(v)] + start[which + 1:]) for v in values]
+        want = [plan(r, zeros) for r in requests]
+        told_apart += len(set(want)) > 1
+        for i in rng.integers(0, len(requests), 4 * len(requests)):
+            assert plan(requests[i], None) == want[i], requests[i]
+    assert told_apart >= 50
+
+
 def test_the_plans_for_all_alignments_are_kept_together():
     """fss_workspace_bytes plans a shape for 2, 4, 8 and 16 bytes: asked again, it plans nothing anew."""
     lib = _native.lib()
