@@ -21,7 +21,9 @@ def choose(lib, shape, dtype, direction, align=16):
 
 def test_chaining_words_stay_far_below_the_scratch_limits():
     """A tiling chosen by the estimate needs at most 4 MiB of words, or no more than the finest that launches that
-    fill the device take (16 steps; 4 waves up to 2048 steps, 8 beyond): what fitted a caller's scratch still does."""
+    fill the device take (16 steps; 4 waves up to 2048 steps, 8 beyond).  In no case more than chunks of 64 steps would:
+    24 bytes per chunk and channel, 6 % of what the forward moves in 16 bits.  (Not a promise that a workspace of one
+    length serves every shorter one: see below.)"""
     lib = _native.lib()
     rng = np.random.default_rng(5)
     for _ in range(3000):
@@ -34,6 +36,17 @@ def test_chaining_words_stay_far_below_the_scratch_limits():
         bound = lib.fss_workspace_bytes(bs, seq, d, dtype, direction, ctypes.byref(finest))
         # (rows of an odd number of 64-channel tiles are padded to two channels per lane)
         assert need <= max(LIMIT + 4096, 2 * bound), (bs, seq, d, dtype, direction)
+        assert need - 4096 <= max(LIMIT, 24 * bs * -(-d // 128) * 128 * -(-seq // 64)), (bs, seq, d, dtype, direction)
+
+
+def test_a_shorter_sequence_may_need_the_larger_workspace():
+    """What include/fss_scan.h tells a caller that keeps one workspace for many lengths."""
+    lib = _native.lib()
+    bf16, gated = _native.FSS_BF16, _native.FSS_GATED_FWD
+    assert lib.fss_workspace_bytes(64, 500, 1680, bf16, gated, None) < lib.fss_workspace_bytes(64, 300, 1680, bf16, gated, None)
+    assert lib.fss_workspace_bytes(8, 1000, 1007, bf16, _native.FSS_FWD, None) < lib.fss_workspace_bytes(8, 700, 1007, bf16, _native.FSS_FWD, None)
+    # (one workgroup would cover these: four that share the sequence are faster, and chain)
+    assert lib.fss_workspace_bytes(64, 512, 4096, bf16, gated, None) == 4096 + 24 * 64 * 4096 * 4
 
 
 def test_no_plain_forward_outgrows_the_static_scratch():
