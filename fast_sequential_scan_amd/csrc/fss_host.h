@@ -282,7 +282,14 @@ inline void complete_config(fss_config &c, int64_t bs, int64_t seq, int64_t d, i
   } else if (fwd) {
     // The gated kernels spend as much time on arithmetic as on memory and like more, smaller
     // waves; a sequence that 8 waves cover wants two workgroups per CU before it takes them.
-    const bool filled = open && elems >= forward_model_elems(narrow, gated);  // (below: where the estimate starts from)
+    // (below: where the estimate starts from)  Not a launch of the limit's size itself that the ladder's tile covers in one
+    // round, as powers of two do: 16-bit, two channels, (16, 2048, 256) 13.9 us and 14.5 with 8 waves, (32, 256, 1024) 12.3
+    // and 13.5; one channel from 4096 steps, (8, 4096, 256) 14.6 and 16.3, (1, 32768, 256) 16.4 and 23.9; fp32 (8, 2048, 256)
+    // 11.5 and 14.6 with 12.  42 shapes in 16 bits 8 % faster in the mean, 27 in fp32 of more than 512 steps 15 %; the slowest is
+    // (1, 2048, 4096) in 16 bits, 14.7 -> 15.8
+    const int64_t ones = bs * ceil_div(d, 64), twos = bs * ceil_div(d, 128);
+    const int64_t round = !narrow ? ones * ceil_div(seq, 256) : seq >= 4096 ? ones * ceil_div(seq, 512) : can2 ? twos * ceil_div(seq, 256) : 0;
+    const bool filled = open && elems >= forward_model_elems(narrow, gated) && round != kCus;
     const bool twelve = ceil_div(seq, 192) * 192 * 10 <= ceil_div(seq, 128) * 128 * 11;
     if (narrow && filled && !can2) {
       // one channel per lane (odd widths, or rows that two would pad too far): 16 steps and 12 waves, two workgroups on a

@@ -87,3 +87,15 @@ def test_rows_of_three_column_tiles():
             assert choose((8, 20000, d), dtype, FWD)[0] == 2 and choose((8, 20000, d), dtype, BWD)[0] == 2
     # fp32 has one channel per lane at these widths anyhow
     assert choose((4, 57534, 192), F32, FWD)[0] == 1
+
+
+# gated forwards of just the size from which launches count as filling the device: the ladder's tile where it has one round
+@pytest.mark.parametrize("shape,dtype,want", [
+    ((16, 2048, 256), BF16, (2, 16, 16, 1)), ((32, 256, 1024), BF16, (2, 16, 16, 1)), ((8, 1024, 1024), FP16, (2, 16, 16, 1)),
+    ((8, 4096, 256), BF16, (1, 32, 16, 1)), ((1, 32768, 256), BF16, (1, 32, 16, 1)), ((16, 8192, 64), BF16, (1, 32, 16, 1)),
+    ((64, 128, 1024), BF16, (2, 16, 8, 1)), ((64, 2048, 64), BF16, (1, 16, 12, 1)),  # no one round of a 16-wave tile
+    ((9, 1695, 1792), BF16, (2, 16, 8, 1)),                                         # above that size
+    ((8, 2048, 256), F32, (1, 16, 16, 1)), ((1, 16384, 256), F32, (1, 16, 16, 1)), ((256, 64, 256), F32, (1, 16, 4, 1)),
+    ((8, 2049, 256), F32, (1, 16, 12, 1))])
+def test_gated_forward_of_one_round(shape, dtype, want):
+    assert choose(shape, dtype, GATED_FWD) == want
