@@ -287,7 +287,7 @@ inline void complete_config(fss_config &c, int64_t bs, int64_t seq, int64_t d, i
     // and 13.5; one channel from 4096 steps, (8, 4096, 256) 14.6 and 16.3, (1, 32768, 256) 16.4 and 23.9; fp32 (8, 2048, 256)
     // 11.5 and 14.6 with 12.  42 shapes in 16 bits 8 % faster in the mean, 27 in fp32 of more than 512 steps 15 %; the slowest is
     // (1, 2048, 4096) in 16 bits, 14.7 -> 15.8
-    const int64_t ones = bs * ceil_div(d, 64), twos = bs * ceil_div(d, 128);
+    const int64_t ones = bs * ceil_div(d, 64), twos = bs * ceil_div(d, 128), big = (narrow ? twos : ones) * ceil_div(seq, 512);
     const int64_t round = !narrow ? ones * ceil_div(seq, 256) : seq >= 4096 ? ones * ceil_div(seq, 512) : can2 ? twos * ceil_div(seq, 256) : 0;
     const bool filled = open && elems >= forward_model_elems(narrow, gated) && round != kCus;
     const bool twelve = ceil_div(seq, 192) * 192 * 10 <= ceil_div(seq, 128) * 128 * 11;
@@ -301,9 +301,15 @@ inline void complete_config(fss_config &c, int64_t bs, int64_t seq, int64_t d, i
       rung(1, 16, twelve ? 12 : 8, 0);
     } else if (narrow && filled) {
       // the largest tile where there is just one for every compute unit: (4, 2048, 2048) one launch behind the other
-      // 23.0 us, 16 steps and 8 waves 27.2 (from 8192 steps two 8-wave workgroups are 3-5 % faster than one of 16: 8 shapes of 9)
-      const int64_t big = bs * ceil_div(d, 128) * ceil_div(seq, 512);
+      // 23.0 us, 16 steps and 8 waves 27.2 (from 8192 steps two 8-wave workgroups are 3-5 % faster than one of 16: 8 shapes of 9).
+      // 16 shapes of 252 to 256 such tiles are 2 % faster with them in the mean, the slowest (16, 721, 968) 18.9 -> 22.0; 23 of
+      // 225 to 251 1 % slower; 5 of 260, (1, 5120, 3328) among them, 28.7 and 38.9
       if (seq > 256 && seq < 8192 && big <= kCus && big * 50 >= kCus * 49) rung(2, 32, 16, 0);
+      // and in many rounds of rows that share sectors, where one covers the sequence and pads it by less than a third: (129, 410,
+      // 3944) 345 -> 311 us, (256, 400, 1182) 211 -> 195; 14 shapes 7 % faster in the mean, the slowest (89, 478, 3226) 209 -> 210.
+      // Of 7 to 8.5 rounds, or padding it further, (230, 404, 1134) 173 and 176, (116, 455, 1948) 163 and 162, (123, 265, 3048)
+      // 162 and 180; of fewer, (47, 436, 1536) 45 and 56.
+      if (shares_sectors(d * esize) && seq > 384 && seq <= 512 && big * 2 >= 17 * kCus) rung(2, 32, 16, 0);
       // the same as with one channel per lane, for sequences of few chunks ((9, 1695, 1792) 42.6 -> 37.5 us against 32 steps and
       // 16 waves, (34, 1201, 776) 64.9 -> 55.6, (26, 859, 1548) 61 -> 51); half as long where that pads the sequence by a
       // tenth less ((29, 299, 1680) 34.4 -> 20.7)
@@ -330,7 +336,7 @@ inline void complete_config(fss_config &c, int64_t bs, int64_t seq, int64_t d, i
       // 16.1 -> 23.3, (142, 386, 1088) 134 -> 155: there the ladder keeps its tile, at a loss of at most 9 % ((149, 206, 896) 77.5
       // -> 84.9).  Known to be slower with 12 waves: (7, 5420, 175) 29.3 -> 32.6, whose second round is nearly empty, (12, 12130, 782)
       // 323 -> 341, (40, 942, 1345) 151 -> 165; 80 shapes from 4 Mi to 128 Mi elements are 13 % faster in the mean.
-      const int64_t big = bs * ceil_div(d, 64) * ceil_div(seq, 512), of_round = ceil_div(big, kCus) * kCus;
+      const int64_t of_round = ceil_div(big, kCus) * kCus;
       const bool ladder = !twelve && seq > 64 && seq <= 512 && seq % 32 < 16 && !shares_sectors(d * esize);
       if (filled && !ladder && (big * 50 < of_round * 49 || seq * 50 < ceil_div(seq, 512) * 512 * 49)) rung(1, 16, twelve ? 12 : 8, 0);
       if (seq > 256) rung(1, 32, 16); else rung(1, 32, 8, 2 * kCus);

@@ -99,3 +99,14 @@ def test_rows_of_three_column_tiles():
     ((8, 2049, 256), F32, (1, 16, 12, 1))])
 def test_gated_forward_of_one_round(shape, dtype, want):
     assert choose(shape, dtype, GATED_FWD) == want
+
+
+# gated forwards in 16 bits of rows that share sectors and one chunk: the largest tile in many rounds
+@pytest.mark.parametrize("shape,want", [
+    ((129, 410, 3944), (2, 32, 16, 1)), ((83, 512, 3450), (2, 32, 16, 1)), ((256, 385, 1182), (2, 32, 16, 1)),
+    ((129, 410, 3936), (2, 16, 4, 1)),                                      # whole sectors
+    ((116, 455, 1948), (2, 16, 8, 1)),                                      # 7.25 rounds
+    ((142, 384, 3450), (2, 16, 8, 1)), ((142, 513, 3450), (2, 16, 4, 1))])  # padded by a third; two chunks
+def test_gated_forward_of_one_chunk_that_shares_sectors(shape, want):
+    for dtype in (BF16, FP16):
+        assert choose(shape, dtype, GATED_FWD) == want
