@@ -334,11 +334,15 @@ inline void complete_config(fss_config &c, int64_t bs, int64_t seq, int64_t d, i
       // 31 of 32, 30 % in the mean of 88 shapes, (237, 59, 704) 43.3 -> 29.5, the slowest (186, 80, 3063) 168 -> 192.  Fewer or
       // all 32, nothing in the mean of 81; above 64 steps, in rows of whole sectors, a loss of 3 % in the mean of 48, (60, 78, 1024)
       // 16.1 -> 23.3, (142, 386, 1088) 134 -> 155: there the ladder keeps its tile, at a loss of at most 9 % ((149, 206, 896) 77.5
-      // -> 84.9).  Known to be slower with 12 waves: (7, 5420, 175) 29.3 -> 32.6, whose second round is nearly empty, (12, 12130, 782)
-      // 323 -> 341, (40, 942, 1345) 151 -> 165; 80 shapes from 4 Mi to 128 Mi elements are 13 % faster in the mean.
+      // -> 84.9).
+      // Not 12 waves where just a few of their tiles go into a second round, in a launch that the largest tile does not fill: (7, 5420,
+      // 175) 28.4 and 31.9 us, (2, 1306, 2560) 20.8 and 22.9; 38 shapes with up to a fifth of a second round are 3 % faster
+      // without in the mean, the slowest (1, 17281, 347) 25.8 -> 28.2; 16 with more of it 1 %, 12 with none 6 % slower.
+      // Known to be slower with 12 waves: (12, 12130, 782) 323 -> 341, (40, 942, 1345) 151 -> 165; 80 shapes from 4 Mi to 128 Mi elements are 13 % faster in the mean.
       const int64_t of_round = ceil_div(big, kCus) * kCus;
       const bool ladder = !twelve && seq > 64 && seq <= 512 && seq % 32 < 16 && !shares_sectors(d * esize);
-      if (filled && !ladder && (big * 50 < of_round * 49 || seq * 50 < ceil_div(seq, 512) * 512 * 49)) rung(1, 16, twelve ? 12 : 8, 0);
+      const bool spills = twelve && seq > 512 && big <= kCus && ones * ceil_div(seq, 192) > 2 * kCus && ones * ceil_div(seq, 192) * 5 <= 2 * kCus * 6;
+      if (filled && !ladder && !spills && (big * 50 < of_round * 49 || seq * 50 < ceil_div(seq, 512) * 512 * 49)) rung(1, 16, twelve ? 12 : 8, 0);
       if (seq > 256) rung(1, 32, 16); else rung(1, 32, 8, 2 * kCus);
       rung(1, 16, 16, 0);
     }

@@ -110,3 +110,13 @@ def test_gated_forward_of_one_round(shape, dtype, want):
 def test_gated_forward_of_one_chunk_that_shares_sectors(shape, want):
     for dtype in (BF16, FP16):
         assert choose(shape, dtype, GATED_FWD) == want
+
+
+# gated forwards in fp32 that the largest tile does not fill the device with: not 12 waves where they begin a second round
+@pytest.mark.parametrize("shape,want", [
+    ((7, 5420, 175), (1, 16, 16, 1)), ((2, 1306, 2560), (1, 16, 16, 1)), ((1, 1654, 3712), (1, 16, 8, 1)), ((1, 17185, 384), (1, 16, 8, 1)),
+    ((1, 14009, 448), (1, 16, 12, 1)),                              # 511 tiles of 12 waves, 512 have a place
+    ((1, 9031, 896), (1, 16, 12, 1)),                               # a second round that is no longer short
+    ((29, 1522, 142), (1, 16, 12, 1)), ((65, 366, 1217), (1, 16, 12, 1))])  # the largest tile fills the device
+def test_gated_forward_in_single_precision_without_a_short_second_round(shape, want):
+    assert choose(shape, F32, GATED_FWD) == want
