@@ -338,11 +338,17 @@ inline void complete_config(fss_config &c, int64_t bs, int64_t seq, int64_t d, i
       // Not 12 waves where just a few of their tiles go into a second round, in a launch that the largest tile does not fill: (7, 5420,
       // 175) 28.4 and 31.9 us, (2, 1306, 2560) 20.8 and 22.9; 38 shapes with up to a fifth of a second round are 3 % faster
       // without in the mean, the slowest (1, 17281, 347) 25.8 -> 28.2; 16 with more of it 1 %, 12 with none 6 % slower.
-      // Known to be slower with 12 waves: (12, 12130, 782) 323 -> 341, (40, 942, 1345) 151 -> 165; 80 shapes from 4 Mi to 128 Mi elements are 13 % faster in the mean.
+      // Nor in large launches of wide rows that share sectors, (6, 12955, 2369) 493 and 580, (44, 1451, 1809) 327 and 385: 24 shapes from 80 Mi
+      // elements and 1280 channels on, padded by up to a quarter, are 8 % faster with the largest tile in the mean, the slowest
+      // (2, 15075, 3558) 307 -> 314.  Of 48 to 80 Mi elements they are 3 % slower (11 shapes), narrower 4 % (11), padded further 5 % (11); one
+      // chunk of that tile, 410 to 512 steps, is 13 % faster to 17 % slower and the same in the mean of 14.
+      // Known to be slower with 12 waves: (12, 12130, 782) 323 -> 341, (40, 942, 1345) 151 -> 165; 80 shapes from
+      // 4 Mi to 128 Mi elements are 13 % faster in the mean.
       const int64_t of_round = ceil_div(big, kCus) * kCus;
       const bool ladder = !twelve && seq > 64 && seq <= 512 && seq % 32 < 16 && !shares_sectors(d * esize);
       const bool spills = twelve && seq > 512 && big <= kCus && ones * ceil_div(seq, 192) > 2 * kCus && ones * ceil_div(seq, 192) * 5 <= 2 * kCus * 6;
-      if (filled && !ladder && !spills && (big * 50 < of_round * 49 || seq * 50 < ceil_div(seq, 512) * 512 * 49)) rung(1, 16, twelve ? 12 : 8, 0);
+      const bool wide = shares_sectors(d * esize) && d >= 1280 && seq > 512 && elems >= (int64_t{80} << 20) && ceil_div(seq, 512) * 512 * 4 <= seq * 5;
+      if (filled && !ladder && !spills && !wide && (big * 50 < of_round * 49 || seq * 50 < ceil_div(seq, 512) * 512 * 49)) rung(1, 16, twelve ? 12 : 8, 0);
       if (seq > 256) rung(1, 32, 16); else rung(1, 32, 8, 2 * kCus);
       rung(1, 16, 16, 0);
     }

@@ -120,3 +120,14 @@ def test_gated_forward_of_one_chunk_that_shares_sectors(shape, want):
     ((29, 1522, 142), (1, 16, 12, 1)), ((65, 366, 1217), (1, 16, 12, 1))])  # the largest tile fills the device
 def test_gated_forward_in_single_precision_without_a_short_second_round(shape, want):
     assert choose(shape, F32, GATED_FWD) == want
+
+
+# gated forwards in fp32 of wide rows that share sectors: the largest tile in large launches that it does not pad much
+@pytest.mark.parametrize("shape,want", [
+    ((44, 1451, 1809), (1, 32, 16, 1)), ((6, 12955, 2369), (1, 32, 16, 1)), ((98, 1664, 1286), (1, 32, 16, 1)),
+    ((35, 1451, 1630), (1, 16, 12, 1)),                             # below 80 Mi elements
+    ((60, 1451, 1270), (1, 16, 12, 1)),                             # narrower
+    ((44, 1451, 1808), (1, 16, 12, 1)),                             # whole sectors
+    ((44, 1200, 1809), (1, 16, 12, 1)), ((77, 449, 3374), (1, 16, 8, 1))])  # padded by more than a quarter; one chunk
+def test_gated_forward_in_single_precision_of_wide_rows_that_share_sectors(shape, want):
+    assert choose(shape, F32, GATED_FWD) == want

@@ -78,6 +78,8 @@ def test_large_backwards_with_states(oracle, shape, tiling):
 @pytest.mark.parametrize("shape,dtype,tiling", [
     ((34, 214, 664), torch.float32, (1, 16, 8)), ((24, 55, 3756), torch.float32, (1, 16, 4)),
     ((43, 32, 3345), torch.float32, (1, 16, 2)), ((9, 7795, 67), torch.float32, (1, 16, 12)),
+    ((7, 5420, 175), torch.float32, (1, 16, 16)), ((2, 2048, 1024), torch.float32, (1, 16, 16)),
+    ((4, 2048, 1024), torch.bfloat16, (2, 16, 16)), ((2, 4096, 1024), torch.bfloat16, (1, 32, 16)),
     ((11, 2100, 369), torch.bfloat16, (1, 16, 12)), ((64, 299, 440), torch.bfloat16, (2, 32, 16)), ((64, 299, 640), torch.bfloat16, (2, 16, 4))])
 def test_large_gated_forwards(oracle, shape, dtype, tiling):
     plan(shape, dtype, GATED_FWD, tiling)
