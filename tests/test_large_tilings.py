@@ -21,9 +21,12 @@ def choose(shape, dtype, direction, align=16):
     ((26, 5000, 210), 16),                                          # below 2^25 elements
     ((27, 8422, 224), 16), ((27, 8422, 256), 16),                   # whole sectors
     ((48, 17050, 82), 16), ((64, 8422, 126), 16),                   # one column tile per row: no seam
-    ((43, 235, 3380), 16), ((60, 407, 1424), 16), ((49, 1268, 1994), 16),  # 192-step chunks pad further
-    ((54, 608, 2168), 16), ((24, 956, 2034), 16),                   # few chunks
-    ((4, 25461, 382), 16), ((1, 51198, 794), 16)])                  # a long chain
+    ((43, 235, 3380), 16), ((60, 407, 1424), 16),                   # 192-step chunks pad an eighth further
+    ((10, 1190, 3804), 12), ((130, 1745, 342), 12),                 # a twentieth and a fourteenth
+    ((54, 608, 2168), 16), ((20, 640, 3828), 16), ((40, 641, 4008), 12),  # four chunks for three, the last nearly empty
+    ((90, 265, 1458), 12), ((190, 256, 1458), 16), ((24, 956, 2034), 12),  # few chunks
+    ((4, 25461, 382), 16), ((1, 51198, 794), 16), ((9, 20000, 194), 12), ((8, 20000, 250), 16),  # a long chain: 18 columns or fewer
+    ((14, 54771, 174), 12), ((14, 51817, 144), 16), ((14, 51817, 146), 12)])
 def test_backward_of_sector_sharing_rows(shape, waves):
     for dtype in (BF16, FP16):
         assert choose(shape, dtype, BWD) == (2, 16, waves, 1), shape
