@@ -327,9 +327,6 @@ __device__ __forceinline__ uint32_t ld_u32(const uint32_t *p) {
 __device__ __forceinline__ void st_u32(uint32_t *p, uint32_t v) {
   __hip_atomic_store((FSS_GLOBAL uint32_t *)p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
-__device__ __forceinline__ uint32_t add_u32(uint32_t *p, uint32_t v) {
-  return __hip_atomic_fetch_add((FSS_GLOBAL uint32_t *)p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-}
 __device__ __forceinline__ void add_u64(uint64_t *p, uint64_t v) {
   (void)__hip_atomic_fetch_add((FSS_GLOBAL uint64_t *)p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
@@ -408,7 +405,7 @@ struct ScanArgs {
   int32_t n_groups;       // column groups per chunk: n_ctiles / column tiles per workgroup
   int32_t look_waves;     // waves per column tile that look back in parallel (1..kMaxLookWaves)
   int32_t row_lanes_log2; // channel-major only: lanes that cover a row of at most half a wave's (6: the row has waves to itself)
-  int32_t period;         // chunks of one sequence that a full grid works on at once (chain_anchor), >= 1
+  int32_t period;         // chunks of one sequence that a nominal full grid works on at once (chain_anchor), >= 1
   uint32_t spin_limit;    // polls before a look-back gives up (kSpinLimit unless a test lowered it)
   uint32_t *hdr;          // workspace header
   uint64_t *words;        // tagged words
@@ -658,7 +655,8 @@ struct TileCtx {
 // grid of the planned size finished a round ago (in round 0: of chunk 0, which needs no
 // look-back).  The period is planned from the nominal device, not from the grid actually
 // launched: a smaller grid or device meets the same anchors (and merely finds the maps
-// already there), so the results do not depend on it either.
+// already there), a larger one (chain_period) waits for some of them as it does for maps, so the results do not
+// depend on it either.
 //
 // Where a round holds more chunks than one round of the look-back reaches (`stride` = look-back
 // waves x kMaxSpan chunks; a single long sequence whose chunks are all in flight at once), every

@@ -76,8 +76,9 @@ inline bool config_valid(const fss_config &c, int dtype, bool gated = false, int
 constexpr int64_t kCus = 256;
 
 // Chunks of one sequence that a full grid works on at once: the spacing of the chain's anchors
-// (chain_anchor in fss_device.h).  Planned from the nominal device - kCus compute units holding
-// 16 waves of a scan each - and from nothing that can differ between two launches of one
+// (chain_anchor in fss_device.h).  Planned from a nominal device - kCus compute units holding
+// 16 waves of a scan each, though kernels of up to 16 steps have registers for 24: with 8 or 12 waves a grid of those
+// works on one and a half or two periods at once, and a chunk's anchor may still be in flight - and from nothing that can differ between two launches of one
 // configuration (not the grid actually launched, not the device's own CU count), so that the
 // order in which carries are composed, and with it every bit of the result, is fixed by the
 // shape and the configuration.

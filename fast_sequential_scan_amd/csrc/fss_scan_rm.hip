@@ -509,7 +509,7 @@ __global__ __launch_bounds__(MAXW * 64) void scan_kernel(const ScanArgs p, const
 #ifdef FSS_RESIDENCY_PROBE
   // debug build only: header words 8/9 = workgroups resident now / the most ever seen
   if (threadIdx.x == 0 && p.hdr) {
-    const uint32_t now = add_u32(p.hdr + 8, 1u) + 1u;
+    const uint32_t now = __hip_atomic_fetch_add(p.hdr + 8, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) + 1u;
     __hip_atomic_fetch_max(p.hdr + 9, now, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   }
 #endif
