@@ -68,7 +68,7 @@
  *   stream).  A workspace sized for one shape serves any shape whose
  *   fss_workspace_bytes is not larger - which a shorter sequence's, a smaller
  *   batch's or a narrower row's may be: the tiling follows the shape, and the
- *   need is 24 bytes per chunk and channel, 0.1 to 50 % of one tensor's
+ *   need is 24 bytes per chunk and channel, 0.1 to 64 % of one tensor's
  *   bytes (bf16 forward, bs 8, d 1007: 0.4 MB at seq 1000, 1.2 MB at 700; gated,
  *   bs 64, d 4096, seq 512: 25 MB).  Keep one workspace for several shapes by
  *   taking the largest need among them, and for a captured graph before the

@@ -1,6 +1,9 @@
 """Host-side checks of which tilings large launches take: on both sides of each line that a rule draws."""
+import csv
 import ctypes
+from pathlib import Path
 
+import numpy as np
 import pytest
 
 from fast_sequential_scan_amd import _native
@@ -134,3 +137,22 @@ def test_gated_forward_in_single_precision_without_a_short_second_round(shape, w
     ((44, 1200, 1809), (1, 16, 12, 1)), ((77, 449, 3374), (1, 16, 8, 1))])  # padded by more than a quarter; one chunk
 def test_gated_forward_in_single_precision_of_wide_rows_that_share_sectors(shape, want):
     assert choose(shape, F32, GATED_FWD) == want
+
+
+PAIRS = Path(__file__).resolve().parent.parent / "profiles" / "large_tilings_pairs.csv"
+
+
+# what the choice may lose in the mean against the fastest measured tiling (what it loses, rounded up; the ladder alone 4, 8 and 8 %)
+@pytest.mark.parametrize("kernel,dtype,loss", [("backward", "bf16", 0.01), ("gated", "bf16", 0.025), ("gated", "fp32", 0.045)])
+def test_the_choice_is_near_the_fastest_measured_tiling(kernel, dtype, loss):
+    times = {}
+    with open(PAIRS) as f:
+        for row in csv.DictReader(f):
+            if (row["kernel"], row["dtype"]) == (kernel, dtype):
+                shape = tuple(int(row[k]) for k in ("bs", "seq", "d"))
+                times.setdefault(shape, {})[tuple(int(row[k]) for k in ("vec", "steps", "waves", "cols"))] = float(row["us"])
+    direction = BWD if kernel == "backward" else GATED_FWD
+    chosen = {s: choose(s, BF16 if dtype == "bf16" else F32, direction) for s in times}
+    ratios = [times[s][c] / min(times[s].values()) for s, c in chosen.items() if c in times[s]]
+    assert len(ratios) >= 300  # (some short sequences take a tiling that was not among the named ones)
+    assert np.exp(np.mean(np.log(ratios))) - 1 <= loss
