@@ -253,12 +253,15 @@ inline void complete_config(fss_config &c, int64_t bs, int64_t seq, int64_t d, i
     if (narrow) {
       // (one channel per lane, where two do not go, in very large launches: (7, 4958, 3767) 8 waves 370 us, 16 waves
       // 300; (4, 8354, 1531) 142 and 122; of 2^24 elements, (31, 607, 1041), 45 and 53.  Not where 256-step chunks pad the
-      // sequence an eighth further than 128-step ones: (28, 525, 2681) 108 and 117, (57, 261, 2529) 111 and 131.  Nor in
-      // narrow rows: 65 to 87 channels 3 % slower in the mean of 16 shapes, (212, 2488, 67) 130 and 148, (75, 11521, 71) 229
-      // and 240, and up to 64 no faster; from 93 to 191, 7 % faster in the mean of 28, the slowest (252, 4063, 97) 279 and 284;
-      // 82 wider ones 10 %)
-      if (open && !can2 && d >= 88 && elems >= (static_cast<int64_t>(1) << 25) &&
-          ceil_div(seq, 256) * 256 * 8 <= ceil_div(seq, 128) * 128 * 9)
+      // sequence a fifth further than 128-step ones: (28, 525, 2681) 108 and 117, (57, 261, 2529) 111 and 131; 16 shapes of 513 to
+      // 640 steps the same in the mean, but 30 of 769 to 896, a seventh further, 3 % faster, (40, 870, 3567) 338 and 292, the slowest
+      // (133, 769, 385) 111 and 117.  Nor in narrow rows: 65 to 87 channels 3 % slower in the mean of 16 shapes, (212, 2488, 67) 130 and 148,
+      // (75, 11521, 71) 229 and 240, and below 64 no faster (64, whose lanes are all busy, 3 % in the mean
+      // of 13, (2721, 214, 64) 83 and 71, the slowest (433, 1391, 64) by 7 %); from 93 to 191, 7 % faster in the mean of 28, the slowest (252, 4063,
+      // 97) 279 and 284; 82 wider ones 10 %.  8 of them cover 65 to 128 steps: 8 steps and 8 waves take 15 % longer there in the
+      // mean of 28 shapes, (512, 66, 3475) 431 and 285, the slowest (190, 128, 2633) 160 and 160; for fewer steps they are 5 % faster)
+      const int64_t of128 = ceil_div(seq, 128) * 128, of192 = ceil_div(seq, 192) * 192, of256 = ceil_div(seq, 256) * 256;
+      if (open && !can2 && (d >= 88 || d == 64) && elems >= (static_cast<int64_t>(1) << 25) && seq > 64 && (seq <= 128 || of256 * 7 <= of128 * 8))
         rung(1, 16, 16);
       if (three_tiles && elems >= (static_cast<int64_t>(1) << 23)) rung(1, 16, 16);
       // (rows that share sectors, in very large launches: with 12 waves what is in flight leaves the L2 room to put the seams
@@ -271,7 +274,6 @@ inline void complete_config(fss_config &c, int64_t bs, int64_t seq, int64_t d, i
       // with a last one that is nearly empty, (54, 608, 2168) 160 -> 167; from 16384 steps on, rows of up to 144 channels, (14,
       // 51817, 144) 252 -> 264, and few columns, of which more chunks are in flight than the look-back has at hand, (4, 25461, 382)
       // 94 -> 101.  Below 2^25 elements, (8, 16359, 232), 73.6 -> 77.3)
-      const int64_t of192 = ceil_div(seq, 192) * 192, of256 = ceil_div(seq, 256) * 256;
       if (open && can2 && shares_sectors(d * esize) && d > 128 && elems >= (static_cast<int64_t>(1) << 25) && seq > 256 &&
           of192 * 10 <= of256 * 11 && (of192 < of256 || seq > 640) && (seq < 16384 || (d > 144 && bs * ceil_div(d, 128) >= 18)))
         rung(2, 16, 12);

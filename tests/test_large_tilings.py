@@ -40,12 +40,23 @@ def test_backward_of_sector_sharing_rows(shape, waves):
     ((75, 11521, 71), 8), ((171, 8554, 85), 8), ((171, 8554, 89), 16), ((179, 8888, 47), 8),
     ((7, 4958, 3767), 16), ((4, 8354, 1531), 16), ((20, 1072, 1817), 16), ((48, 185, 3847), 16),
     ((31, 607, 1041), 8),                                           # below 2^25 elements
-    ((57, 261, 2529), 8), ((28, 525, 2681), 8), ((16, 812, 2613), 8)])  # 512, 768 and 1024 for 384, 640 and 896
+    ((57, 261, 2529), 8), ((28, 525, 2681), 8), ((40, 870, 3567), 16),  # 512, 768 and 1024 for 384, 640 and 896
+    ((512, 66, 3475), 8), ((190, 128, 2633), 8), ((113, 137, 3563), 16), ((48, 12642, 61), 8)])  # 8 waves cover it; narrow
 def test_backward_of_odd_width(shape, waves):
     for dtype in (BF16, FP16):
         assert choose(shape, dtype, BWD) == (1, 16, waves, 1), shape
     # (tensors of even width that start at an odd element are the same case)
     assert choose((shape[0], shape[1], shape[2] + 1), BF16, BWD, 2) == (1, 16, waves, 1)
+
+
+def test_backward_of_rows_of_one_whole_tile():
+    for shape, waves in [((48, 12642, 64), 16), ((2721, 214, 64), 16), ((1825, 426, 64), 16), ((3121, 266, 64), 8)]:  # 512 for 384
+        assert choose(shape, BF16, BWD) == (1, 16, waves, 1), shape
+
+
+def test_backward_of_odd_width_and_few_steps():
+    for shape in [(577, 60, 3709), (880, 51, 1161), (600, 64, 1161)]:
+        assert choose(shape, BF16, BWD) == (1, 8, 8, 1), shape
 
 
 # forwards of odd width and up to 1024 steps: 128-step chunks where they pad a fifth less than 512-step ones
