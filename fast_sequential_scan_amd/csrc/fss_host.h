@@ -265,17 +265,22 @@ inline void complete_config(fss_config &c, int64_t bs, int64_t seq, int64_t d, i
         rung(1, 16, 16);
       if (three_tiles && elems >= (static_cast<int64_t>(1) << 23)) rung(1, 16, 16);
       // (rows that share sectors, in very large launches: with 12 waves what is in flight leaves the L2 room to put the seams
-      // between column tiles together.  So not for rows of one tile, which have no seam: (48, 17050, 82) 162 -> 175 us.  One launch
-      // behind the other, (27, 8422, 210) 140 -> 111, (54, 5718, 146) 147 -> 114, (26, 3001, 526) 110 -> 100, (13, 2846, 1194) 115
-      // -> 104; 249 shapes of 2^25 to 2^27 elements that the lines below leave in, 5 % faster in the mean: 84 of 257 to 1023
-      // steps 6 %, the slowest (24, 956, 2034) 105 -> 107; 99 of up to 16383 4 %, the slowest (106, 1942, 246) 112 -> 121; 66
-      // longer ones 5 %, (14, 54771, 174) 448 -> 319, the slowest (14, 27263, 242) 201 -> 216.  Left out, 76 shapes, 0 % in the
-      // mean: where 192-step chunks pad the sequence a tenth further, (43, 235, 3380) 79 -> 92, (232, 406, 364) 79 -> 90, or as far
-      // with a last one that is nearly empty, (54, 608, 2168) 160 -> 167; from 16384 steps on, rows of up to 144 channels, (14,
-      // 51817, 144) 252 -> 264, and few columns, of which more chunks are in flight than the look-back has at hand, (4, 25461, 382)
-      // 94 -> 101.  Below 2^25 elements, (8, 16359, 232), 73.6 -> 77.3)
-      if (open && can2 && shares_sectors(d * esize) && d > 128 && elems >= (static_cast<int64_t>(1) << 25) && seq > 256 &&
-          of192 * 10 <= of256 * 11 && (of192 < of256 || seq > 640) && (seq < 16384 || (d > 144 && bs * ceil_div(d, 128) >= 18)))
+      // between column tiles together.  So not for rows of one tile, which have no seam: (48, 17050, 82) 162 -> 175 us, 23 shapes 2 %
+      // slower in the mean, but where 192-step chunks pad the sequence a quarter less, (3249, 269, 112) 259 -> 217.  One launch
+      // behind the other, (27, 8422, 210) 140 -> 111, (54, 5718, 146) 147 -> 114, (26, 3001, 526) 110
+      // -> 100, (13, 2846, 1194) 115 -> 104; some 290 shapes of 2^25 to 2^27 elements that the lines below leave in are 5 % faster in
+      // the mean: 84 of 257 to 1023 steps 6 %, the slowest (24, 956, 2034) 105 -> 107; 99 of up to 16383 4 %, the slowest (106,
+      // 1942, 246) 112 -> 121; 93 longer ones 4 %, (14, 54771, 174) 448 -> 319, the slowest (4, 25461, 382) 94 -> 101.  Fewer than 97
+      // steps are covered by fewer waves, 6 for 12: 49 to 64 by 6 8 % faster than by 4, (420, 51, 3588) 172 -> 158; 97 to 128 by 12
+      // 11 % faster than by 8, (1362, 124, 692) 324 -> 226, the slowest (953, 98, 624) 119 -> 121; 65 to 96 by 6 3 % slower than
+      // by 8, and fewer than 49 the same.  Left out as well: where 192-step chunks pad the sequence a tenth further, (43, 235,
+      // 3380) 79 -> 92, (232, 406, 364) 79 -> 90 - but 449 to 512 steps, whose third chunk is a third full and more, 3 % faster in the
+      // mean of 13, (340, 457, 222) 98 -> 87, the slowest (127, 456, 1948) by 3 % - or as far with a last one
+      // that is nearly empty, (54, 608, 2168) 160 -> 167; and from
+      // 16384 steps on rows of up to 144 channels, 10 shapes 4 % slower, (14, 51817, 144) 252 -> 264.  Below 2^25 elements, (8,
+      // 16359, 232), 73.6 -> 77.3)
+      if (open && can2 && shares_sectors(d * esize) && (d > 128 || of192 * 4 <= of256 * 3) && elems >= (static_cast<int64_t>(1) << 25) &&
+          (seq > 96 || (seq > 48 && seq <= 64)) && ((seq > 448 && seq <= 512) || (of192 * 10 <= of256 * 11 && (of192 < of256 || seq > 640))) && (seq < 16384 || d > 144))
         rung(2, 16, 12);
       rung(2, 16, 16);
       if (seq >= 16384) rung(1, 16, 16); else rung(2, 16, 8);

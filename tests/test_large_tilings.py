@@ -28,8 +28,12 @@ def choose(shape, dtype, direction, align=16):
     ((10, 1190, 3804), 12), ((130, 1745, 342), 12),                 # a twentieth and a fourteenth
     ((54, 608, 2168), 16), ((20, 640, 3828), 16), ((40, 641, 4008), 12),  # four chunks for three, the last nearly empty
     ((90, 265, 1458), 12), ((190, 256, 1458), 16), ((24, 956, 2034), 12),  # few chunks
-    ((4, 25461, 382), 16), ((1, 51198, 794), 16), ((9, 20000, 194), 12), ((8, 20000, 250), 16),  # a long chain: 18 columns or fewer
-    ((14, 54771, 174), 12), ((14, 51817, 144), 16), ((14, 51817, 146), 12)])
+    ((1362, 124, 692), 12), ((445, 97, 1938), 12), ((582, 84, 2186), 8), ((256, 96, 3158), 8), ((420, 51, 3588), 6),  # one, of as many
+    ((330, 64, 3588), 6), ((700, 48, 1676), 4),                            # waves as the steps need
+    ((340, 457, 222), 12), ((340, 448, 222), 16), ((114, 512, 700), 12), ((114, 513, 700), 12),  # the third chunk a third full
+    ((3249, 269, 112), 12), ((470, 800, 112), 16),                         # one column tile: three chunks for four
+    ((4, 25461, 382), 12), ((1, 51198, 794), 12), ((14, 54771, 174), 12),  # a long chain
+    ((14, 51817, 144), 16), ((14, 51817, 146), 12)])
 def test_backward_of_sector_sharing_rows(shape, waves):
     for dtype in (BF16, FP16):
         assert choose(shape, dtype, BWD) == (2, 16, waves, 1), shape
