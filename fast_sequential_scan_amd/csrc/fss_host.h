@@ -237,10 +237,11 @@ inline void complete_config(fss_config &c, int64_t bs, int64_t seq, int64_t d, i
     // (24, 384, 1735) 23.2 -> 19.2 us, (29, 574, 1319) 44.4 -> 33.6, (28, 748, 445) 15.8 -> 13.7; 15 shapes above 15 Mi
     // elements 8 % faster in the mean, the slowest (21, 277, 3669) 36.9 -> 37.9.  Where less padding goes, and where one chunk
     // of 256 steps covers the sequence, the smaller tiles lose 2 % in the mean: (36, 393, 1921) 43.5 -> 48.6, (35, 169, 2995)
-    // 25.9 -> 30.6); their words, twice to four times as many, well within the scratch of the entry point that
+    // 25.9 -> 30.6.  Up to 64 steps, at any size, half the steps and twice the waves are 9 % faster in the mean of 19 shapes,
+    // (208, 59, 97) 6.9 -> 5.0, (122, 44, 1043) 10.3 -> 9.5, the slowest (2675, 20, 113) 11.5 -> 12.8); their words, twice to four times as many, well within the scratch of the entry point that
     // allocates nothing
     const int64_t reach = ceil_div(seq, 128), short_tiles = bs * ceil_div(d, 64) * reach;
-    if (open && narrow && !can2 && seq > 256 && seq <= 1024 && reach * 128 * 5 <= ceil_div(seq, 512) * 512 * 4 &&
+    if (open && narrow && !can2 && (seq <= 64 || (seq > 256 && seq <= 1024 && reach * 128 * 5 <= ceil_div(seq, 512) * 512 * 4)) &&
         short_tiles * 3 * 64 * static_cast<int64_t>(sizeof(uint64_t)) <= FSS_NOALLOC_SCRATCH_BYTES / 2)
       rung(1, 16, 8);
     if (wide32_fwd) rung(2, 16, 16);

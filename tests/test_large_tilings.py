@@ -68,6 +68,7 @@ def test_backward_of_odd_width_and_few_steps():
     ((29, 574, 1319), 16), ((23, 749, 1927), 16), ((24, 384, 1735), 16), ((33, 561, 2107), 16),
     ((36, 393, 1921), 32), ((62, 1000, 343), 32), ((13, 872, 1465), 32),  # 512 for 512, 1024 for 1024 and 896
     ((35, 169, 2995), 32), ((53, 188, 2485), 32), ((61, 254, 3011), 32),  # one chunk of 256 steps
+    ((208, 59, 97), 16), ((35, 38, 2715), 16), ((2675, 20, 113), 16), ((150, 64, 1735), 16), ((180, 65, 1735), 32),  # up to 64 steps
     ((24, 1300, 1735), 32),                                               # more than 1024 steps
     ((85, 588, 1999), 32)])                                               # words beyond half the static array
 def test_forward_of_odd_width(shape, steps):
