@@ -321,8 +321,8 @@ inline void complete_config(fss_config &c, int64_t bs, int64_t seq, int64_t d, i
       // and in many rounds of rows that share sectors, where one covers the sequence and pads it by less than a third: (129, 410,
       // 3944) 345 -> 311 us, (256, 400, 1182) 211 -> 195; 14 shapes 7 % faster in the mean, the slowest (89, 478, 3226) 209 -> 210.
       // Of 7 to 8.5 rounds, or padding it further, (230, 404, 1134) 173 and 176, (116, 455, 1948) 163 and 162, (123, 265, 3048)
-      // 162 and 180; of fewer, (47, 436, 1536) 45 and 56.
-      if (shares_sectors(d * esize) && seq > 384 && seq <= 512 && big * 2 >= 17 * kCus) rung(2, 32, 16, 0);
+      // 162 and 180; of fewer, (47, 436, 1536) 45 and 56; of narrow rows, (2429, 416, 86) 152 and 181.
+      if (shares_sectors(d * esize) && d >= 1024 && seq > 384 && seq <= 512 && big * 2 >= 17 * kCus) rung(2, 32, 16, 0);
       // the same as with one channel per lane, for sequences of few chunks ((9, 1695, 1792) 42.6 -> 37.5 us against 32 steps and
       // 16 waves, (34, 1201, 776) 64.9 -> 55.6, (26, 859, 1548) 61 -> 51); half as long where that pads the sequence by a
       // tenth less ((29, 299, 1680) 34.4 -> 20.7)

@@ -126,7 +126,7 @@ def test_gated_forward_of_one_round(shape, dtype, want):
 # gated forwards in 16 bits of rows that share sectors and one chunk: the largest tile in many rounds
 @pytest.mark.parametrize("shape,want", [
     ((129, 410, 3944), (2, 32, 16, 1)), ((83, 512, 3450), (2, 32, 16, 1)), ((256, 385, 1182), (2, 32, 16, 1)),
-    ((129, 410, 3936), (2, 16, 4, 1)),                                      # whole sectors
+    ((129, 410, 3936), (2, 16, 4, 1)), ((2429, 416, 86), (2, 16, 4, 1)),    # whole sectors; narrow rows
     ((116, 455, 1948), (2, 16, 8, 1)),                                      # 7.25 rounds
     ((142, 384, 3450), (2, 16, 8, 1)), ((142, 513, 3450), (2, 16, 4, 1))])  # padded by a third; two chunks
 def test_gated_forward_of_one_chunk_that_shares_sectors(shape, want):
