@@ -158,8 +158,8 @@ def test_gated_forward_in_single_precision_of_wide_rows_that_share_sectors(shape
 PAIRS = Path(__file__).resolve().parent.parent / "profiles" / "large_tilings_pairs.csv"
 
 
-# what the choice may lose in the mean against the fastest measured tiling (what it loses, rounded up; the ladder alone 4, 8 and 8 %)
-@pytest.mark.parametrize("kernel,dtype,loss", [("backward", "bf16", 0.01), ("gated", "bf16", 0.025), ("gated", "fp32", 0.045)])
+# what the choice may lose in the mean against the fastest measured tiling (what it loses, rounded up; the ladder alone 5, 8 and 9 %)
+@pytest.mark.parametrize("kernel,dtype,loss", [("backward", "bf16", 0.01), ("gated", "bf16", 0.025), ("gated", "fp32", 0.035)])
 def test_the_choice_is_near_the_fastest_measured_tiling(kernel, dtype, loss):
     times = {}
     with open(PAIRS) as f:
