@@ -259,8 +259,8 @@ inline void complete_config(fss_config &c, int64_t bs, int64_t seq, int64_t d, i
       // (133, 769, 385) 111 and 117.  Nor in narrow rows: 65 to 87 channels 3 % slower in the mean of 16 shapes, (212, 2488, 67) 130 and 148,
       // (75, 11521, 71) 229 and 240, and below 64 no faster (64, whose lanes are all busy, 3 % in the mean
       // of 13, (2721, 214, 64) 83 and 71, the slowest (433, 1391, 64) by 7 %); from 93 to 191, 7 % faster in the mean of 28, the slowest (252, 4063,
-      // 97) 279 and 284; 82 wider ones 10 %.  8 of them cover 65 to 128 steps: 8 steps and 8 waves take 15 % longer there in the
-      // mean of 28 shapes, (512, 66, 3475) 431 and 285, the slowest (190, 128, 2633) 160 and 160; for fewer steps they are 5 % faster)
+      // 97) 279 and 284; 82 wider ones 10 %.  8 of them cover 65 to 128 steps: 8 steps and 8 waves take 17 % longer there in the
+      // mean of 29 shapes, (512, 66, 3475) 431 and 285, the least (190, 128, 2633) 160 and 160; for fewer steps they are 3 % faster)
       const int64_t of128 = ceil_div(seq, 128) * 128, of192 = ceil_div(seq, 192) * 192, of256 = ceil_div(seq, 256) * 256;
       if (open && !can2 && (d >= 88 || d == 64) && elems >= (static_cast<int64_t>(1) << 25) && seq > 64 && (seq <= 128 || of256 * 7 <= of128 * 8))
         rung(1, 16, 16);
@@ -276,12 +276,12 @@ inline void complete_config(fss_config &c, int64_t bs, int64_t seq, int64_t d, i
       // 11 % faster than by 8, (1362, 124, 692) 324 -> 226, the slowest (953, 98, 624) 119 -> 121; 65 to 96 by 6 3 % slower than
       // by 8, and fewer than 49 the same.  Left out as well: where 192-step chunks pad the sequence a tenth further, (43, 235,
       // 3380) 79 -> 92, (232, 406, 364) 79 -> 90 - but 449 to 512 steps, whose third chunk is a third full and more, 3 % faster in the
-      // mean of 13, (340, 457, 222) 98 -> 87, the slowest (127, 456, 1948) by 3 % - or as far with a last one
-      // that is nearly empty, (54, 608, 2168) 160 -> 167; and from
-      // 16384 steps on rows of up to 144 channels, 10 shapes 4 % slower, (14, 51817, 144) 252 -> 264.  Below 2^25 elements, (8,
+      // mean of 13, (340, 457, 222) 98 -> 87, the slowest (127, 456, 1948) by 3 % - or as far with a last one that is nearly
+      // empty, (54, 608, 2168) 160 -> 167; and from 16384 steps on rows of up to 144 channels, 10 shapes 4 % slower, (14, 51817, 144) 252 -> 264.  Below 2^25 elements, (8,
       // 16359, 232), 73.6 -> 77.3)
       if (open && can2 && shares_sectors(d * esize) && (d > 128 || of192 * 4 <= of256 * 3) && elems >= (static_cast<int64_t>(1) << 25) &&
-          (seq > 96 || (seq > 48 && seq <= 64)) && ((seq > 448 && seq <= 512) || (of192 * 10 <= of256 * 11 && (of192 < of256 || seq > 640))) && (seq < 16384 || d > 144))
+          (seq > 96 || (seq > 48 && seq <= 64)) && (seq < 16384 || d > 144) &&
+          ((seq > 448 && seq <= 512) || (of192 * 10 <= of256 * 11 && (of192 < of256 || seq > 640))))
         rung(2, 16, 12);
       rung(2, 16, 16);
       if (seq >= 16384) rung(1, 16, 16); else rung(2, 16, 8);
@@ -355,7 +355,7 @@ inline void complete_config(fss_config &c, int64_t bs, int64_t seq, int64_t d, i
       // elements and 1280 channels on, padded by up to a quarter, are 8 % faster with the largest tile in the mean, the slowest
       // (2, 15075, 3558) 307 -> 314.  Of 48 to 80 Mi elements they are 3 % slower (11 shapes), narrower 4 % (11), padded further 5 % (11); one
       // chunk of that tile, 410 to 512 steps, is 13 % faster to 17 % slower and the same in the mean of 14.
-      // Known to be slower with 12 waves: (12, 12130, 782) 323 -> 341, (40, 942, 1345) 151 -> 165; 80 shapes from
+      // Known to be slower: with 8 waves (226, 635, 371) 203 -> 238 us, with 12 (12, 12130, 782) 323 -> 341, (40, 942, 1345) 151 -> 165; 80 shapes from
       // 4 Mi to 128 Mi elements are 13 % faster in the mean.
       const int64_t of_round = ceil_div(big, kCus) * kCus;
       const bool ladder = !twelve && seq > 64 && seq <= 512 && seq % 32 < 16 && !shares_sectors(d * esize);
